@@ -949,19 +949,14 @@ static hipError_t launch_fwd_dt(const Geo &g, FwdParams p, int bm, int row0, int
                                 hipStream_t s) {
     p.mt_base = row0 / bm;
     p.mtiles = rows / bm;
-    if constexpr (sizeof(T) == 2) {
-        if (g.Mp <= kBiasRows) {
-            if (bm == 256 && ws_two_waves_per_simd<T, 2>()) return launch_fwd_ws<T, 2>(g, p, s);
-            if (bm == 128 && ws_two_waves_per_simd<T, 1>()) return launch_fwd_ws<T, 1>(g, p, s);
-        }
-        // more than kBiasRows output rows (or a register count that would let
-        // three waves share a SIMD): the non-specialised kernel
-        if (bm == 256) return launch_fwd_t<T, 8, 1, 1, 4>(g, p, s);
-        return launch_fwd_t<T, 2, 4, 2, 1>(g, p, s);
-    } else {
-        if (bm == 256) return launch_fwd_t<T, 8, 1, 1, 4>(g, p, s);
-        return launch_fwd_t<T, 2, 4, 2, 1>(g, p, s);
+    if (g.Mp <= kBiasRows) {
+        if (bm == 256 && ws_two_waves_per_simd<T, 2>()) return launch_fwd_ws<T, 2>(g, p, s);
+        if (bm == 128 && ws_two_waves_per_simd<T, 1>()) return launch_fwd_ws<T, 1>(g, p, s);
     }
+    // more than kBiasRows output rows (or a register count that would let
+    // three waves share a SIMD): the non-specialised kernel
+    if (bm == 256) return launch_fwd_t<T, 8, 1, 1, 4>(g, p, s);
+    return launch_fwd_t<T, 2, 4, 2, 1>(g, p, s);
 }
 
 // Ungrouped (or not splittable): one launch over every row and chunk.  With
@@ -992,6 +987,8 @@ hipError_t launch_forward(const Geo &g, const void *xt, const void *wp, const vo
                           const void *offset, const void *mask, const void *bias, void *out,
                           hipStream_t s) {
     if (g.B == 0) return hipSuccess;
+    if (g.dtype == DCN2_F32)
+        return launch_forward_f32(g, xt, wp, tab, offset, mask, bias, out, s);
     FwdParams p;
     p.xt = xt;
     p.wp = wp;
@@ -1021,11 +1018,7 @@ hipError_t launch_forward(const Geo &g, const void *xt, const void *wp, const vo
     p.Wo = g.Wo;
     p.Kp = g.Kp;
     p.Mp = g.Mp;
-    switch (g.dtype) {
-    case DCN2_F16: return launch_fwd_groups<f16>(g, p, s);
-    case DCN2_BF16: return launch_fwd_groups<bf16>(g, p, s);
-    default: return launch_fwd_groups<float>(g, p, s);
-    }
+    return g.dtype == DCN2_F16 ? launch_fwd_groups<f16>(g, p, s) : launch_fwd_groups<bf16>(g, p, s);
 }
 
 }  // namespace dcn2

@@ -256,8 +256,10 @@ static hipError_t pack_t(const Geo &g, const void *input, void *xt, const void *
     p.Cw = g.Cw;
     p.mpg = g.Cout / g.WG;
     p.kc = g.KC;
-    p.kstep = g.dtype == DCN2_F32 ? 2 : 16;
-    p.kpl = g.dtype == DCN2_F32 ? 1 : 8;
+    // fp32: the forward's lanes read 4 consecutive channels, one per MFMA
+    const bool f4 = g.dtype == DCN2_F32 && !transpose;
+    p.kstep = g.dtype == DCN2_F32 ? (f4 ? 8 : 2) : 16;
+    p.kpl = g.dtype == DCN2_F32 ? (f4 ? 4 : 1) : 8;
     p.Mp = g.Mp;
     p.Kp = g.Kp;
     p.transpose = transpose ? 1 : 0;
