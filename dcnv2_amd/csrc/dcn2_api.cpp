@@ -198,8 +198,8 @@ BwdWorkspace bwd_workspace(const Geo &g0) {
     o += align256((size_t)gg.rows * g.Cgp * gg.row_esz);
     w.rsc = o;
     if (gg.row_scaled) o += align256((size_t)gg.rows * (g.Cgp / 32));
-    w.csum = o;  // fp32 corner sums [B][G*KK][N][4] of the fused kernel
-    if (fused_bwd_shape(g) && g.Cgp > g.KC) o += align256((size_t)g.B * g.G * g.KK * g.N * 16);
+    w.csum = o;  // fp32 corner sums [B][G*KK][N][4] of groups that workgroups share
+    if (csum_shape(g)) o += align256((size_t)g.B * g.G * g.KK * g.N * 16);
     w.rec = o;
     o += align256((size_t)gg.rows * 12);  // 12-byte sample records
     w.bcnt = o;

@@ -33,63 +33,11 @@
 #include "dcn2_common.h"
 #include "dcn2_sampler.h"
 #include "dcn2_kernels.h"
+#include "dcn2_backward.h"
 #include "dcn2_profile.h"
 #include "../../include/dcnv2_amd.h"
 
 namespace dcn2 {
-
-// Record of a placed sample: its floor corner (y0 in the low, x0 in the high
-// 16 bits, both >= -2) and the bilinear fractions (12 bytes: the consumers
-// find the sample's hand-off row from the record's own position).
-struct BucketRec {
-    int yx;
-    float ly, lx;
-};
-
-struct BwdParams {
-    const void *xt, *wt, *tab, *offset, *mask, *gout;
-    void *goff, *gmask;
-    float *gi_acc, *gw_acc, *gb_acc;
-    int B, H, W, Cout, kh, kw, sh, sw, ph, pw, dh, dw, G, Cg, Cgp, Ho, Wo, Kp, Mp;
-    int tiles_per_img, splits;
-    int go_nhwc;  // grad_output is channels-last [B][Ho][Wo][Cout]
-    // grad_output can be read with 16-byte loads: 8 consecutive pixels of a row
-    // (NCHW, N % 8 == 0) or channels of a pixel (channels-last, Cout % 8 == 0),
-    // from a 16-byte aligned base
-    int go_vec;
-    // grad_input gather: cell-tile buckets (see dcn2_gi_gather_kernel).  The
-    // rows of all buckets are packed back to back, bucket k owning rows
-    // [bstart[k], bstart[k+1]); there are at most B*G*KK*N of them (one per
-    // sample), so the storage is sized exactly and no bucket can overflow.
-    void *cgm;          // [rows][Cgp] masked column gradient rows (RowOf)
-    unsigned char *rsc; // [rows][Cgp/32] scale codes of bf16 rows (row_block_scale)
-    float *csum;        // [B][G*KK][N][4] corner sums of groups of several chunks (fused kernel)
-    struct BucketRec *rec;  // [rows] sample records, in bucket order
-    int *bcnt;          // [nbuckets] samples per bucket (count pass)
-    int *bstart;        // [nbuckets + 1] first row of each bucket (exclusive scan of bcnt)
-    int *bcur;          // [nbuckets] next free row of each bucket (place pass)
-    int *sidx;          // [B][G*KK][N] bucket row of each sample; -1 no corner inside
-    int ntx, nty;       // cell tiles per row / column
-    float *ring;        // [nbuckets][kRing][Cgp] grad_input sums of each window's border ring
-    // grad_input written directly by the per-cell kernel and ring_final_kernel
-    // (no fp32 accumulator): the caller's buffer, whether it is channels-last
-    // [B][H][W][C] (else [B][C][H][W]), and whether 8-element runs take vector
-    // stores there (NCHW: W % 8 == 0; channels-last: C and C/G multiples of
-    // 8; both with a 16-byte aligned base)
-    void *gi_out;
-    int gi_nhwc, gi_vec;
-    // offset / mask (and grad_offset / grad_mask) elements between images, and
-    // whether the mask buffer holds logits (see mask_value; grad_mask is then
-    // the gradient of the logits)
-    long long off_bs, msk_bs;
-    int msk_logit;
-    // grad_weight work items: gw_nch chunks per M chunk.  Ungrouped (gw_cog
-    // 0): every chunk.  Weight groups whose chunks never mix: an M chunk of
-    // group w = m0 / gw_cog walks only that group's chunks tap*gw_cpt +
-    // w*gw_cpw + i, i < gw_cpw (the other blocks of the block-diagonal packed
-    // weight are zero and their grad_weight is not kept).
-    int gw_nch, gw_cpt, gw_cpw, gw_cog;
-};
 
 // Eight consecutive elements as 16-byte stores (dst 16-byte aligned).
 template <typename T> __device__ __forceinline__ void store8(T *dst, const T (&v)[8]) {
@@ -3034,6 +2982,10 @@ bool fused_bwd_shape(const Geo &g) {
            (long long)g.H * g.W * g.cs * g.esz <= kGoOutOfRange;
 }
 
+bool csum_shape(const Geo &g) {
+    return g.dtype == DCN2_F32 ? g.Cgp > f32_chan_tile(g) : fused_bwd_shape(g) && g.Cgp > g.KC;
+}
+
 template <typename T>
 static hipError_t backward_t(const Geo &g, const BwdParams &p0, void *grad_input,
                              void *grad_weight, void *grad_bias, bool last, hipStream_t s) {
@@ -3113,18 +3065,15 @@ static hipError_t backward_t(const Geo &g, const BwdParams &p0, void *grad_input
                     else DCN2_FUSED(128);
 #undef DCN2_FUSED
                     if ((e = hipGetLastError()) != hipSuccess) return e;
-                    // groups of several chunks: grad_offset / grad_mask from
-                    // the corner sums the chunks added up in csum, finished by
-                    // ring_final_kernel
-                    corner_blocks = cpg > 1 ? ((long)g.B * g.G * g.KK * g.N + 255) / 256 : 0;
                 }
             }
         }
-        if (!fused) {
+        if constexpr (sizeof(T) == 4) {
+            if ((e = launch_colgrad_f32(g, p, s)) != hipSuccess) return e;
+        } else if (!fused) {
             dim3 grid(p.tiles_per_img, g.B);
             // W'^T staged in LDS when a chunk of it fits (Mp <= 256); gO resident
-            // in registers when one M chunk covers all rows.  fp32 keeps the
-            // 128-wide M chunk: 256 would hold 128 gO registers.
+            // in registers when one M chunk covers all rows.
             const bool alds = g.Mp <= 256;
 #define DCN2_COLGRAD(MCHV)                                                                      \
     do {                                                                                        \
@@ -3132,15 +3081,15 @@ static hipError_t backward_t(const Geo &g, const BwdParams &p0, void *grad_input
         else if (alds) dcn2_colgrad_kernel<T, MCHV, true, false><<<grid, 512, 0, s>>>(p);       \
         else dcn2_colgrad_kernel<T, MCHV, false, false><<<grid, 512, 0, s>>>(p);                \
     } while (0)
-            if constexpr (sizeof(T) == 2) {
-                if (g.Mp % 256 == 0) DCN2_COLGRAD(256);
-                else DCN2_COLGRAD(128);
-            } else {
-                DCN2_COLGRAD(128);
-            }
+            if (g.Mp % 256 == 0) DCN2_COLGRAD(256);
+            else DCN2_COLGRAD(128);
 #undef DCN2_COLGRAD
             if ((e = hipGetLastError()) != hipSuccess) return e;
         }
+        // grad_offset / grad_mask of groups whose chunks several workgroups
+        // share are finished from the corner sums by ring_final_kernel
+        if ((fused || sizeof(T) == 4) && csum_shape(g))
+            corner_blocks = ((long)g.B * g.G * g.KK * g.N + 255) / 256;
         prof_end(DCN2_STAGE_BWD_COLGRAD, s);
         // 3. grad_weight / grad_bias of the two-kernel path
         auto run_gradw = [&]() -> hipError_t {

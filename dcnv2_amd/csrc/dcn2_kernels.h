@@ -134,7 +134,14 @@ hipError_t launch_backward(const Geo &g, const void *xt, const void *wt, const v
                            float *csum, void *rec, int *bcnt, int *bstart, int *bcur, int *sidx,
                            float *ring, bool last, hipStream_t s);
 // Whether the fused backward kernel may serve g (2-byte type, Cout <= 256),
-// and whether it then needs the corner-sum buffer (several chunks per group).
+// and whether its column-gradient kernel (the fused one, or the fp32 one) needs
+// the corner-sum buffer (a group's channels shared by several workgroups).
 bool fused_bwd_shape(const Geo &g);
+bool csum_shape(const Geo &g);
+// Channels of one fp32 backward workgroup: two chunks of a group where they
+// pair up (and lie in one weight group), else one.
+inline int f32_chan_tile(const Geo &g) {
+    return g.Cgp % 64 == 0 && (!g.gsplit || g.cpw % 2 == 0) ? 64 : 32;
+}
 
 }  // namespace dcn2

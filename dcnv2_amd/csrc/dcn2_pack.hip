@@ -127,10 +127,9 @@ __device__ __forceinline__ void pack_input_block(const PackParams &p, int blk) {
 // W'[32*rb + lane%32][ch*kc + ks*kstep + (lane/32)*kpl + e], so one wave's
 // fragment load is one contiguous run; transpose 1 (backward): the same for
 // W'^T (rows k, reduction m): dst[((kb*(Mp/kstep) + ms)*64 + lane)][e] holds
-// W'[ms*kstep + (lane/32)*kpl + e][32*kb + lane%32].  For 2-byte types a
-// piece is the kpl = 8 elements e of one lane; for fp32 (kpl = 1) it is
-// 4 consecutive lanes.  All index math is 32-bit (the host bounds Mp*Kp
-// below 2^31).
+// W'[ms*kstep + (lane/32)*kpl + e][32*kb + lane%32].  A piece is the kpl
+// elements e of one lane (8 for 2-byte types, 4 for fp32).  All index math is
+// 32-bit (the host bounds Mp*Kp below 2^31).
 // The first nch threads also write the chunk table: for chunk ch of the K
 // order (tap, group, channel chunk of kc channels) tab[ch] = {offset/mask
 // plane g*KK + tap, row term ki*dh, column term kj*dw, channel base
@@ -153,8 +152,7 @@ __device__ __forceinline__ void pack_weight_block(const PackParams &p, int blk) 
     const int idx0 = t * EPT;
     if (idx0 >= p.Mp * p.Kp) return;
     const int kpl = p.kpl, kstep = p.kstep;
-    // fragment coordinates of element idx0: e0, lane0 and the fragment index
-    const int e0 = idx0 % kpl;
+    // fragment coordinates of element idx0: lane0 and the fragment index
     int r = idx0 / kpl;
     const int lane0 = r % 64;
     r /= 64;
@@ -171,20 +169,18 @@ __device__ __forceinline__ void pack_weight_block(const PackParams &p, int blk) 
         ch = r % nch;
         bq = r / nch; // rb
     }
-    // Across the EPT elements of a piece one coordinate steps by one and the
-    // other is fixed: for 2-byte types (kpl = 8) the K index (the channel c,
-    // within one tap and group: a piece never crosses a KC-channel chunk) in
-    // the forward layout and the row m in the transposed one; for fp32
-    // (kpl = 1, consecutive lanes) the row m in the forward layout and the K
-    // index in the transposed one.  So the divisions run once per piece.
-    const bool step_k = (kpl > 1) != (p.transpose != 0);
+    // Across the elements of a piece one coordinate steps by one and the other
+    // is fixed: the K index (the channel c, within one tap and group: a piece
+    // never crosses a KC-channel chunk) in the forward layout, the row m in the
+    // transposed one.  So the divisions run once per piece.
+    const bool step_k = p.transpose == 0;
     int m0, k0;
     if (p.transpose) {
         k0 = bq * 32 + (lane0 & 31);
-        m0 = a * kstep + (lane0 >> 5) * kpl + e0;
+        m0 = a * kstep + (lane0 >> 5) * kpl;
     } else {
         m0 = bq * 32 + (lane0 & 31);
-        k0 = ch * p.kc + ks * kstep + (lane0 >> 5) * kpl + e0;
+        k0 = ch * p.kc + ks * kstep + (lane0 >> 5) * kpl;
     }
     const int gc = p.G * p.Cgp;
     const int tap = k0 / gc, rr = k0 - tap * gc;
@@ -256,10 +252,9 @@ static hipError_t pack_t(const Geo &g, const void *input, void *xt, const void *
     p.Cw = g.Cw;
     p.mpg = g.Cout / g.WG;
     p.kc = g.KC;
-    // fp32: the forward's lanes read 4 consecutive channels, one per MFMA
-    const bool f4 = g.dtype == DCN2_F32 && !transpose;
-    p.kstep = g.dtype == DCN2_F32 ? (f4 ? 8 : 2) : 16;
-    p.kpl = g.dtype == DCN2_F32 ? (f4 ? 4 : 1) : 8;
+    // fp32: a lane reads 4 consecutive elements of the reduction, one per MFMA
+    p.kstep = g.dtype == DCN2_F32 ? 8 : 16;
+    p.kpl = g.dtype == DCN2_F32 ? 4 : 8;
     p.Mp = g.Mp;
     p.Kp = g.Kp;
     p.transpose = transpose ? 1 : 0;
