@@ -63,5 +63,7 @@ struct BwdParams {
 // dcn2_backward_f32.hip: the fp32 column gradient with its consumers
 // (grad_offset / grad_mask or the corner sums in csum, and the hand-off rows).
 hipError_t launch_colgrad_f32(const Geo &g, const BwdParams &p, hipStream_t s);
+// The fp32 grad_weight / grad_bias, added to gw_acc / gb_acc.
+hipError_t launch_gradw_f32(const Geo &g, const BwdParams &p, int ncu, hipStream_t s);
 
 }  // namespace dcn2

@@ -906,25 +906,14 @@ __global__ __launch_bounds__(512) void dcn2_colgrad_kernel(const BwdParams p) {
 // channels (blockIdx.z) x a strided subset of the pixel tiles (blockIdx.x).
 // D[m][k] = sum_n gO[m][n] * col[k][n]; A = gO straight from global memory
 // (rows are pixel-contiguous), B = re-sampled columns in LDS.
-// 2-byte types keep the LDS stage as [k][n] with the 16-byte blocks of each
+// The LDS stage is [k][n] with the 16-byte blocks of each
 // row XOR-swizzled by h(k) = ((k & 15) ^ (k >> 3)) & 15 so that both the
 // sampler's 2-byte stores and the MFMA's 16-byte reads are bank-conflict free.
-template <typename T> struct GwLayout;
-template <> struct GwLayout<float> {
-    static constexpr bool kMajor = false;
-};
-template <> struct GwLayout<f16> {
-    static constexpr bool kMajor = true;
-};
-template <> struct GwLayout<bf16> {
-    static constexpr bool kMajor = true;
-};
-
 __device__ __forceinline__ int gw_swz(int k) { return ((k & 15) ^ (k >> 3)) & 15; }
 
-// This kernel serves fp32 and gO rows that 16-byte loads cannot read (N % 8
-// != 0 or an unaligned base); 2-byte types with aligned rows take
-// dcn2_gradw_line_kernel below.  gO is read with guarded loads.
+// This kernel serves 2-byte types with gO rows that 16-byte loads cannot read
+// (N % 8 != 0 or an unaligned base); aligned rows take dcn2_gradw_line_kernel
+// below.  gO is read with guarded loads.
 template <typename T, int MB, bool MASK>
 __global__ __launch_bounds__(512) void dcn2_gradw_kernel(const BwdParams p) {
     using M = Mma<T>;
@@ -934,13 +923,10 @@ __global__ __launch_bounds__(512) void dcn2_gradw_kernel(const BwdParams p) {
     constexpr int KB = KC / 32;
     constexpr int NBLK = MB * KB;
     constexpr int BPW = NBLK >= 16 ? 2 : 1;  // blocks per wave
-    constexpr bool KMAJ = GwLayout<T>::kMajor;
-    constexpr int LDN = KMAJ ? BN : KC + 4;  // pitch of the LDS stage (elements)
-    constexpr int ROWS = KMAJ ? KC : BN;
     constexpr int CPS = KC / 4;
-    static_assert(!KMAJ || BN == 128, "swizzle assumes 16 blocks of 8 per row");
+    static_assert(sizeof(T) == 2 && BN == 128, "swizzle assumes 16 blocks of 8 per row");
 
-    __shared__ __attribute__((aligned(16))) T sC[2][ROWS][LDN];
+    __shared__ __attribute__((aligned(16))) T sC[2][KC][BN];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     int mblk, kblk0;
@@ -999,14 +985,10 @@ __global__ __launch_bounds__(512) void dcn2_gradw_kernel(const BwdParams p) {
         for (int u = 0; u < 2; ++u) {
             float v[16 / sizeof(T)];
             smp[set].blend(0, u, v);
-            if constexpr (KMAJ) {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const int k = smp[set].q * CPS + u * 8 + e;
-                    sC[buf][k][((pl >> 3) ^ gw_swz(k)) * 8 + (pl & 7)] = (T)v[e];
-                }
-            } else {
-                *reinterpret_cast<uint4 *>(&sC[buf][pl][smp[set].q * CPS + u * 4]) = pack16<T>(v);
+            for (int e = 0; e < 8; ++e) {
+                const int k = smp[set].q * CPS + u * 8 + e;
+                sC[buf][k][((pl >> 3) ^ gw_swz(k)) * 8 + (pl & 7)] = (T)v[e];
             }
         }
     };
@@ -1042,17 +1024,13 @@ __global__ __launch_bounds__(512) void dcn2_gradw_kernel(const BwdParams p) {
             }
         }
     };
-    // gO fragments of a whole tile are prefetched one step ahead for 2-byte
-    // types (8 registers of 16 bytes), in the set of the tile's parity (the
-    // loop is unrolled by two, so no register copies); fp32 (64 one-float
-    // steps) loads at use.
-    constexpr bool PREA = KPL == 8;
-    frag a_set[2][PREA ? NKS : 1];
-    auto load_a_tile = [&](frag (&a)[PREA ? NKS : 1], int t) __attribute__((always_inline)) {
-        if constexpr (PREA) {
+    // gO fragments of a whole tile are prefetched one step ahead (8 registers of
+    // 16 bytes), in the set of the tile's parity (the loop is unrolled by two, so
+    // no register copies).
+    frag a_set[2][NKS];
+    auto load_a_tile = [&](frag (&a)[NKS], int t) __attribute__((always_inline)) {
 #pragma unroll
-            for (int ks = 0; ks < NKS; ++ks) load_a(a[ks], t, ks);
-        }
+        for (int ks = 0; ks < NKS; ++ks) load_a(a[ks], t, ks);
     };
 
     auto mfma_tile = [&](auto s_c, int t) __attribute__((always_inline)) {
@@ -1060,43 +1038,21 @@ __global__ __launch_bounds__(512) void dcn2_gradw_kernel(const BwdParams p) {
         if (!active) return;
 #pragma unroll
         for (int ks = 0; ks < NKS; ++ks) {
-            frag a;
-            if constexpr (PREA) {
-                a = a_set[buf][ks];
-            } else {
-                load_a(a, t, ks);
-                if (do_bias) {
-                    if constexpr (KPL == 1) {
-                        bsum += to_f32(a);
-                    } else {
-#pragma unroll
-                        for (int e = 0; e < KPL; ++e) bsum += to_f32(a[e]);
-                    }
-                }
-            }
 #pragma unroll
             for (int i = 0; i < BPW; ++i) {
-                const int k = (kblk0 + i) * 32 + (lane & 31);
-                frag bf;
-                if constexpr (KMAJ) {
-                    const int nblk = ks * 2 + (lane >> 5);
-                    bf = *reinterpret_cast<const frag *>(&sC[buf][k][(nblk ^ gw_swz(k)) * 8]);
-                } else {
-                    bf = sC[buf][ks * KSTEP + (lane >> 5)][k];
-                }
-                acc[i] = M::mma(a, bf, acc[i]);
+                const int k = (kblk0 + i) * 32 + (lane & 31), nblk = ks * 2 + (lane >> 5);
+                const frag bf = *reinterpret_cast<const frag *>(&sC[buf][k][(nblk ^ gw_swz(k)) * 8]);
+                acc[i] = M::mma(a_set[buf][ks], bf, acc[i]);
             }
         }
         // grad_bias from the resident gO fragments, after the MFMA loop: a
         // branch between MFMAs would keep the B-fragment reads from being
         // issued ahead of them
-        if constexpr (PREA) {
-            if (do_bias) {
+        if (do_bias) {
 #pragma unroll
-                for (int ks = 0; ks < NKS; ++ks)
+            for (int ks = 0; ks < NKS; ++ks)
 #pragma unroll
-                    for (int e = 0; e < KPL; ++e) bsum += to_f32(a_set[buf][ks][e]);
-            }
+                for (int e = 0; e < KPL; ++e) bsum += to_f32(a_set[buf][ks][e]);
         }
     };
 
@@ -3094,6 +3050,11 @@ static hipError_t backward_t(const Geo &g, const BwdParams &p0, void *grad_input
         // 3. grad_weight / grad_bias of the two-kernel path
         auto run_gradw = [&]() -> hipError_t {
             prof_begin(DCN2_STAGE_BWD_GRADW, s);
+            if constexpr (sizeof(T) == 4) {
+                const hipError_t fe = launch_gradw_f32(g, p, ncu, s);
+                prof_end(DCN2_STAGE_BWD_GRADW, s);
+                return fe;
+            } else {
             // weight groups split per group (Geo::gsplit): an M chunk must lie
             // in one group, whose rows are a multiple of 128
             const int cog = g.gsplit ? g.Cout / g.WG : 0;
@@ -3134,6 +3095,7 @@ static hipError_t backward_t(const Geo &g, const BwdParams &p0, void *grad_input
             const hipError_t ge = hipGetLastError();
             prof_end(DCN2_STAGE_BWD_GRADW, s);
             return ge;
+            }
         };
         const GatherGeo gg = gather_geometry(g);
         const int nbk = (int)gg.nbuckets;

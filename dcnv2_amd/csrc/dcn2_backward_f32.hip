@@ -18,6 +18,7 @@
 // 14 x 14; 1558 -> 62 at 2048, 512, 32 x 7 x 7; 142 -> 62 at 128, 1152, 4 x 56 x 56.
 #include <algorithm>
 #include <cstddef>
+#include <type_traits>
 
 #include "dcn2_backward.h"
 #include "../../include/dcnv2_amd.h"
@@ -34,6 +35,7 @@ template <int LANES> __device__ __forceinline__ float lane_sum(float v) {
     v = dpp_add<0x4E>(v);   // quad_perm 2,3,0,1
     if constexpr (LANES >= 8) v = dpp_add<0x141>(v);   // row_half_mirror
     if constexpr (LANES >= 16) v = dpp_add<0x140>(v);  // row_mirror
+    if constexpr (LANES >= 32) v += __shfl_xor(v, 16, 64);
     return v;
 }
 
@@ -252,6 +254,236 @@ __global__ __launch_bounds__(256) void dcn2_colgrad_f32_kernel(const CgF32Params
     }
 }
 
+// ---------------------------------------------------------------------------
+// grad_weight / grad_bias (com.cu:637-706, 829-835):
+//     gW[m][c, tap] += sum_n gO[m][n] col[c, tap][n]
+// over a range of the batch's pixels, for BM rows and CT channels of one tap and
+// group.  Steps of PS pixels: grad_output rows and resampled columns of step t+1
+// are loaded while step t is multiplied, both through LDS (two stages).  A lane
+// of an MFMA covers pixels {e, e + 4} of a group of 8 (e = 0..3): the row operand
+// is one 16-byte LDS read per four MFMAs, the column operand four 4-byte reads.
+//
+// Bound: the fp32 matrix rate; then the fp32 atomics that add the ranges' partial
+// blocks (one set per workgroup).  128 x 64 blocks on 4 waves: 256 x 64 on 8 waves
+// measured the same at 256 rows and more (57.6-61.8 us) and 85-97 against 58 at 128.
+// Against the 8-wave kernel this replaces, whose rows came by one 4-byte load per
+// MFMA in the MFMA loop (us): 125 -> 66, 122 -> 57, 195 -> 58, 170 -> 58 at the
+// column gradient's four shapes.
+struct FastDiv {  // n / d for n < 2^31: (umulhi(n, mul) + n) >> shift
+    uint32_t mul, d;
+    int shift;
+};
+static FastDiv fast_div(uint32_t d) {
+    FastDiv f;
+    f.d = d;
+    f.shift = 0;
+    while ((1ull << f.shift) < d) ++f.shift;
+    f.mul = (uint32_t)(((1ull << 32) * ((1ull << f.shift) - d)) / d + 1);
+    return f;
+}
+__device__ __forceinline__ uint32_t operator/(uint32_t n, const FastDiv &f) {
+    return (__umulhi(n, f.mul) + n) >> f.shift;
+}
+
+struct GwF32Params {
+    BwdParams p;
+    int b0, total;     // first image and pixels (images * N) of this launch
+    uint32_t x_bytes;  // bytes of its images of xt
+    FastDiv dN, dWo;
+    int mtiles, ktiles, splits;  // M tiles, channel tiles walked per M tile, pixel ranges
+    int cpg;                     // channel tiles per group
+    int cpt, cpw, cog;  // channel tiles per tap; per weight group, and its rows (0: no split)
+};
+
+// GM: grad_output by 0 16-byte loads of 4 pixels (NCHW, N % 4 == 0, aligned),
+// 1 4-byte loads (NCHW), 2 4-byte loads along channels (channels-last).
+template <int IB, int WM, int CB, int GM, bool MASK>
+__global__ __launch_bounds__(64 * WM * CB) void dcn2_gradw_f32_kernel(const GwF32Params c) {
+    constexpr int NT = 64 * WM * CB, BM = 32 * IB * WM, CT = 32 * CB, LP = CT / 4;
+    constexpr int PS = NT / LP;  // pixels per step: one sampling slot per thread
+    constexpr int LDG = PS + 4, LDC = CT == 64 ? 72 : 40;
+    constexpr int GE = GM == 0 ? 4 : 1;            // pixels per grad_output load
+    constexpr int NG = BM * PS / GE / NT;          // its loads per thread and step
+    static_assert(NT * NG * GE == BM * PS && (GM != 2 || NT % BM == 0), "thread maps");
+    __shared__ __attribute__((aligned(16))) float sG[2][BM][LDG];
+    __shared__ __attribute__((aligned(16))) float sC[2][PS][LDC];
+
+    const BwdParams &p = c.p;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int cb = wave % CB, wm = wave / CB;
+    // ranges slowest: an XCD works on neighbouring pixels for all rows and channels
+    const int wi = xcd_remap(blockIdx.x, c.splits * c.ktiles * c.mtiles);
+    const int mt = wi % c.mtiles, j = wi / c.mtiles % c.ktiles, sp = wi / (c.mtiles * c.ktiles);
+    const int m0 = mt * BM;
+    int ct = j;  // channel tile (tap, group, channels)
+    if (c.cog) ct = j / c.cpw * c.cpt + m0 / c.cog * c.cpw + j % c.cpw;
+    const int N = p.Ho * p.Wo, KK = p.kh * p.kw;
+    const int cc = ct % c.cpg, tg = ct / c.cpg, tap = tg / p.G, g = tg - tap * p.G;
+    const int plane = g * KK + tap, ty = tap / p.kw * p.dh - p.ph, tx = tap % p.kw * p.dw - p.pw;
+    const int nt = ceil_div(c.total, PS);
+    const int t0 = (int)((long long)nt * sp / c.splits), t1 = (int)((long long)nt * (sp + 1) / c.splits);
+    if (t0 >= t1) return;
+
+    // grad_output
+    const int grow = GM == 2 ? tid % BM : tid / (PS / GE), gpx = GM == 2 ? tid / BM : tid % (PS / GE) * GE;
+    constexpr int GRS = GM == 2 ? 0 : NT * GE / PS, GPS = GM == 2 ? NT / BM : 0;  // row / pixel step of a load
+    const float *const go = (const float *)p.gout + (size_t)c.b0 * p.Cout * N;
+    f32x4 gr[NG];  // (only [0] used by 4-byte loads)
+    auto load_g = [&](int t) __attribute__((always_inline)) {
+        if constexpr (GM == 2) {
+#pragma unroll
+            for (int i = 0; i < NG; ++i) {
+                const int n = t * PS + gpx + i * GPS, m = m0 + grow;
+                gr[i][0] = m < p.Cout && n < c.total ? go[(size_t)n * p.Cout + m] : 0.0f;
+            }
+        } else {
+            const uint32_t n = t * PS + gpx, b = n / c.dN, nn = n - b * (uint32_t)N;
+            const float *src = go + (size_t)b * ((size_t)p.Cout * N) + nn;
+            const bool in = (int)n < c.total;  // (GE pixels together: the total is a multiple of 4 there)
+#pragma unroll
+            for (int i = 0; i < NG; ++i) {
+                const int m = m0 + grow + i * GRS;
+                gr[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                if (in && m < p.Cout) {
+                    if constexpr (GM == 0) gr[i] = *reinterpret_cast<const f32x4 *>(src + (size_t)m * N);
+                    else gr[i][0] = src[(size_t)m * N];
+                }
+            }
+        }
+    };
+    const bool do_bias = p.gb_acc != nullptr && j == 0;
+    float bsum[NG];
+#pragma unroll
+    for (int i = 0; i < NG; ++i) bsum[i] = 0.0f;
+    auto store_g = [&](int st) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NG; ++i) {
+            float *dst = &sG[st][grow + i * GRS][gpx + i * GPS];
+            if constexpr (GM == 0) *reinterpret_cast<f32x4 *>(dst) = gr[i];
+            else *dst = gr[i][0];
+            bsum[i] += GM == 0 ? (gr[i][0] + gr[i][1]) + (gr[i][2] + gr[i][3]) : gr[i][0];
+        }
+    };
+
+    // columns: LP lanes x 4 channels per pixel
+    const int spx = tid / LP, l4 = tid % LP * 4;
+    const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float *>((const float *)p.xt + (size_t)c.b0 * p.H * p.W * p.G * p.Cgp), (short)0,
+        (int)c.x_bytes, 0x00020000);
+    const int soff = (g * p.Cgp + cc * CT) * 4;
+    const float *const offp = (const float *)p.offset + c.b0 * p.off_bs + (size_t)plane * 2 * N;
+    const float *const mskp = MASK ? (const float *)p.mask + c.b0 * p.msk_bs + (size_t)plane * N : nullptr;
+    float dy, dx, mv = 1.0f;
+    auto load_om = [&](int t) __attribute__((always_inline)) {
+        const uint32_t n = min(t * PS + spx, c.total - 1), b = n / c.dN, nn = n - b * (uint32_t)N;
+        const float *o = offp + b * p.off_bs + nn;
+        dy = o[0];
+        dx = o[N];
+        if (MASK) mv = mskp[b * p.msk_bs + nn];
+    };
+    f32x4 x[4];
+    float w[4];
+    auto gather = [&](int t) __attribute__((always_inline)) {
+        const uint32_t n0 = t * PS + spx, n = min(n0, (uint32_t)c.total - 1), b = n / c.dN, nn = n - b * (uint32_t)N;
+        const bool live = n0 < (uint32_t)c.total;
+        const int oy = nn / c.dWo, ox = nn - oy * p.Wo;
+        const SamplePos s = sample_pos((float)(oy * p.sh + ty) + dy, (float)(ox * p.sw + tx) + dx, p.H, p.W);
+        const float m = MASK ? mask_value(mv, p.msk_logit) : 1.0f;
+        const float hy = (1.0f - s.ly) * m, ly = s.ly * m, hx = 1.0f - s.lx, lx = s.lx;
+        w[0] = hy * hx;
+        w[1] = hy * lx;
+        w[2] = ly * hx;
+        w[3] = ly * lx;
+        const uint32_t cs = p.G * p.Cgp * 4u, row = cs * (uint32_t)p.W;
+        const uint32_t base = (b * (uint32_t)(p.H * p.W) + (uint32_t)(s.y0 * p.W + s.x0)) * cs + l4 * 4u;
+        // (a corner outside the image, or of a pixel past the end, reads 0)
+        const uint32_t off[4] = {live && s.vy0 && s.vx0 ? base : c.x_bytes,
+                                 live && s.vy0 && s.vx1 ? base + cs : c.x_bytes,
+                                 live && s.vy1 && s.vx0 ? base + row : c.x_bytes,
+                                 live && s.vy1 && s.vx1 ? base + row + cs : c.x_bytes};
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            x[q] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(xrs, (int)off[q], soff, 0));
+    };
+    auto blend = [&](int st) __attribute__((always_inline)) {
+        f32x4 v = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = fmaf(w[q], x[q][e], v[e]);
+        *reinterpret_cast<f32x4 *>(&sC[st][spx][l4]) = v;
+    };
+
+    f32x16 acc[IB];
+#pragma unroll
+    for (int i = 0; i < IB; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][r] = 0.0f;
+    auto mma = [&](int st) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < PS / 8; ++k) {
+            f32x4 af[IB];
+#pragma unroll
+            for (int i = 0; i < IB; ++i)
+                af[i] = *reinterpret_cast<const f32x4 *>(
+                    &sG[st][(wm * IB + i) * 32 + (lane & 31)][8 * k + 4 * (lane >> 5)]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float bf = sC[st][8 * k + 4 * (lane >> 5) + e][cb * 32 + (lane & 31)];
+#pragma unroll
+                for (int i = 0; i < IB; ++i) acc[i] = Mma<float>::mma(af[i][e], bf, acc[i]);
+            }
+        }
+    };
+
+    load_g(t0);
+    load_om(t0);
+    gather(t0);
+    load_om(t0 + 1);
+    blend(0);
+    store_g(0);
+    __syncthreads();
+    auto step = [&](auto set_c, int t) __attribute__((always_inline)) {
+        constexpr int S = decltype(set_c)::value;
+        const bool more = t + 1 < t1;  // (uniform)
+        if (more) {
+            load_g(t + 1);
+            gather(t + 1);
+            load_om(t + 2);
+        }
+        mma(S);
+        if (more) {
+            store_g(S ^ 1);
+            blend(S ^ 1);
+        }
+        __syncthreads();
+    };
+    int t = t0;
+    for (; t + 1 < t1; t += 2) {
+        step(std::integral_constant<int, 0>{}, t);
+        step(std::integral_constant<int, 1>{}, t + 1);
+    }
+    if (t < t1) step(std::integral_constant<int, 0>{}, t);
+
+    const int k = ct * CT + cb * 32 + (lane & 31);
+#pragma unroll
+    for (int i = 0; i < IB; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int m = m0 + (wm * IB + i) * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+            if (m < p.Cout) unsafeAtomicAdd(p.gw_acc + (size_t)m * p.Kp + k, acc[i][r]);
+        }
+    if (do_bias) {
+#pragma unroll
+        for (int i = 0; i < NG; ++i) {
+            const int m = m0 + grow + i * GRS;
+            const float v = GM == 2 ? bsum[i] : lane_sum<PS / GE>(bsum[i]);
+            if ((GM == 2 || gpx == 0) && m < p.Cout) unsafeAtomicAdd(p.gb_acc + m, v);
+        }
+    }
+}
+
 // Images of one launch over g's images (g.B of them): the bytes of their xt and
 // their pixels stay in 32 bits (one image always fits, see make_geo).
 static int f32_images(const Geo &g) {
@@ -285,6 +517,53 @@ hipError_t launch_colgrad_f32(const Geo &g, const BwdParams &p, hipStream_t s) {
         if (CT == 32) colgrad_f32_launch<1, 1>(c, s);
         else if ((long long)ceil_div(c.total, 128) * c.ctiles >= 768) colgrad_f32_launch<2, 2>(c, s);
         else colgrad_f32_launch<1, 2>(c, s);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
+template <int IB, int WM, int CB>
+static void gradw_f32_launch(GwF32Params &c, const Geo &g, int ncu, hipStream_t s) {
+    constexpr int NT = 64 * WM * CB, PS = NT / (8 * CB);
+    c.mtiles = ceil_div(g.Cout, 32 * IB * WM);
+    const long long tiles = (long long)c.mtiles * c.ktiles;
+    // Three workgroups to a CU (of the 128-row ones), each with at least four
+    // steps.  Kernel us at 1 / 2 / 3 / 4 to a CU: 77 / 63 / 66 / 74 at Cout 256, K
+    // 64, 32 x 56 x 56; 75 / 59 / 57 / 62 at 256, 1024, 32 x 14 x 14; 80 / 59 / 58 /
+    // 63 at 2048, 512, 32 x 7 x 7; 74 / 60 / 58 / 64 at 128, 1152, 4 x 56 x 56: more
+    // ranges add more partial blocks with atomics, fewer leave gathers exposed.
+    c.splits = (int)std::max(1LL, std::min(ncu * 3LL / tiles, (long long)ceil_div(c.total, PS) / 4));
+    const unsigned grid = (unsigned)(c.splits * tiles);
+    const int gm = c.p.go_nhwc ? 2 : (g.N % 4 == 0 && ((uintptr_t)c.p.gout & 15) == 0 ? 0 : 1);
+    auto launch = [&](auto mask) {
+        constexpr bool M = decltype(mask)::value;
+        if (gm == 0) dcn2_gradw_f32_kernel<IB, WM, CB, 0, M><<<grid, NT, 0, s>>>(c);
+        else if (gm == 1) dcn2_gradw_f32_kernel<IB, WM, CB, 1, M><<<grid, NT, 0, s>>>(c);
+        else dcn2_gradw_f32_kernel<IB, WM, CB, 2, M><<<grid, NT, 0, s>>>(c);
+    };
+    if (c.p.mask) launch(std::true_type{});
+    else launch(std::false_type{});
+}
+
+hipError_t launch_gradw_f32(const Geo &g, const BwdParams &p, int ncu, hipStream_t s) {
+    GwF32Params c;
+    c.p = p;
+    const int CT = f32_chan_tile(g), nimg = f32_images(g);
+    c.dN = fast_div(g.N);
+    c.dWo = fast_div(g.Wo);
+    c.cpg = g.Cgp / CT;
+    c.cpt = g.cpt * 32 / CT;
+    c.cpw = g.cpw * 32 / CT;
+    c.cog = g.gsplit ? g.Cout / g.WG : 0;
+    c.ktiles = g.KK * c.cpw;
+    for (int b = 0; b < g.B; b += nimg) {
+        const int nb = std::min(nimg, g.B - b);
+        c.b0 = b;
+        c.total = nb * g.N;
+        c.x_bytes = (uint32_t)((long long)nb * g.H * g.W * g.cs * 4);
+        if (CT == 32) gradw_f32_launch<1, 4, 1>(c, g, ncu, s);
+        else gradw_f32_launch<2, 2, 2>(c, g, ncu, s);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
