@@ -47,6 +47,9 @@ struct BwdParams {
     // 8; both with a 16-byte aligned base)
     void *gi_out;
     int gi_nhwc, gi_vec;
+    // parts a bucket's grad_input work is split into, one workgroup each: ranges
+    // of channel chunks and (per-pixel kernel) interleaved passes of 8 pixels
+    int gi_cs, gi_rs;
     // offset / mask (and grad_offset / grad_mask) elements between images, and
     // whether the mask buffer holds logits (see mask_value; grad_mask is then
     // the gradient of the logits)

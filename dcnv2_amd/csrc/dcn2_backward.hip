@@ -2081,12 +2081,15 @@ __global__ __launch_bounds__(512) void dcn2_gi_gather_kernel(const BwdParams p) 
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int nb = p.B * p.G * p.nty * p.ntx;
-    const int bucket = xcd_remap(blockIdx.x, nb);
+    // part of the bucket's work: channel chunks [cc0, cc1), window passes qp0 + 8 k qps
+    const int id = xcd_remap(blockIdx.x, nb * p.gi_cs * p.gi_rs), part = id % (p.gi_cs * p.gi_rs);
+    const int bucket = id / (p.gi_cs * p.gi_rs);
     const int tx = bucket % p.ntx, ty = (bucket / p.ntx) % p.nty;
     const int bg = bucket / (p.ntx * p.nty), b = bg / p.G, g = bg - b * p.G;
     const int row0 = p.bstart[bucket], count = p.bstart[bucket + 1] - row0;
     const int oy = ty * TS - 1, ox = tx * TS - 1;  // pixel of local (0, 0)
     const int cpg = p.Cgp / KC;
+    const int cc0 = cpg * (part % p.gi_cs) / p.gi_cs, cc1 = cpg * (part % p.gi_cs + 1) / p.gi_cs;
     // A bucket of several batches (count > kGatherBatch) keeps its interior
     // pixels' partial sums between batches in its gi_acc slot
     // [(TS-1)^2 pixels][Cgp], slot row0 / (kGatherBatch + 1): the row ranges of
@@ -2174,10 +2177,10 @@ __global__ __launch_bounds__(512) void dcn2_gi_gather_kernel(const BwdParams p) 
         const int row_bytes = p.Cgp * (int)sizeof(R);
         // bf16 rows: this lane's 8 channels lie in 32-channel block co / 4 of the chunk
         const int sc_shift = 8 * (co >> 2);
-        for (int cc = 0; cc < cpg; ++cc) {
+        for (int cc = cc0; cc < cc1; ++cc) {
             if constexpr (kRowScaled<T>) {
                 // the chunk's scale codes of the batch's rows, in sorted order
-                if (cc > 0) __syncthreads();  // the previous chunk is done with ssc
+                if (cc > cc0) __syncthreads();  // the previous chunk is done with ssc
                 const unsigned short *rsc16 =
                     reinterpret_cast<const unsigned short *>(p.rsc) + ((size_t)row0 + base) * cpg + cc;
                 for (int i = tid; i < nrec; i += 512) ssc[i] = rsc16[(size_t)sslot[i] * cpg];
@@ -2195,7 +2198,7 @@ __global__ __launch_bounds__(512) void dcn2_gi_gather_kernel(const BwdParams p) 
             // PPW rows at a time.
             constexpr int NSEG = 2 * TW, NPASS = NSEG + (TW + PPW - 1) / PPW;
             static_assert(PPW == 8 && 1 + 8 * 2 == TW, "two 8-pixel segments per window row");
-            for (int qp = wave; qp < NPASS; qp += 8) {
+            for (int qp = wave + 8 * (part / p.gi_cs); qp < NPASS; qp += 8 * p.gi_rs) {
                 const bool seg = qp < NSEG;  // (uniform over the wave)
                 const int py = seg ? qp >> 1 : (qp - NSEG) * PPW + ps;
                 const int px = seg ? 1 + 8 * (qp & 1) + ps : 0;
@@ -2272,21 +2275,44 @@ __global__ __launch_bounds__(512) void dcn2_gi_gather_kernel(const BwdParams p) 
                 float wa[LPR], wb[LPR];
                 int oa, ob, sa, sb;
                 float xa, xb;
-                // (scheduling barriers keep each batch's loads ahead of the sums of
-                // the previous one; left alone the scheduler groups the fetches)
-                row_info(0, oa, xa, sa);
-                fetch(oa, xa, sa, ra, wa);
-                for (int j0 = 0; j0 < tot; j0 += 2 * LPR) {
-                    row_info(j0 + LPR, ob, xb, sb);
-                    fetch(ob, xb, sb, rb, wb);
-                    __builtin_amdgcn_sched_barrier(0);
-                    accumulate(ra, wa);
-                    __builtin_amdgcn_sched_barrier(0);
-                    row_info(j0 + 2 * LPR, oa, xa, sa);
+                // Batches of the wave's fullest pixel (uniform).  While one is
+                // summed the next is in flight; a pass with no rows loads nothing
+                // and the last one or two batches are peeled, so that a pixel of a
+                // few rows (one sample per pixel: 4) takes one batch, not three
+                // (49 -> 38 us at fp32 1x1, 32 x 56 x 56, C 64; 71 -> 63 at fp16 3x3,
+                // stride 2, 2 x 256 x 256, C 128).
+                // (Scheduling barriers keep each batch's loads ahead of the sums of
+                // the previous one; left alone the scheduler groups the fetches.)
+                int tmax = tot;
+#pragma unroll
+                for (int d = 8; d < 64; d <<= 1) tmax = max(tmax, __shfl_xor(tmax, d, 64));
+                const int nbat = __builtin_amdgcn_readfirstlane((tmax + LPR - 1) / LPR);
+                if (nbat > 0) {
+                    row_info(0, oa, xa, sa);
                     fetch(oa, xa, sa, ra, wa);
-                    __builtin_amdgcn_sched_barrier(0);
-                    accumulate(rb, wb);
-                    __builtin_amdgcn_sched_barrier(0);
+                    int jb = 0;
+                    for (; jb + 2 < nbat; jb += 2) {
+                        row_info((jb + 1) * LPR, ob, xb, sb);
+                        fetch(ob, xb, sb, rb, wb);
+                        __builtin_amdgcn_sched_barrier(0);
+                        accumulate(ra, wa);
+                        __builtin_amdgcn_sched_barrier(0);
+                        row_info((jb + 2) * LPR, oa, xa, sa);
+                        fetch(oa, xa, sa, ra, wa);
+                        __builtin_amdgcn_sched_barrier(0);
+                        accumulate(rb, wb);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                    if (jb + 1 < nbat) {
+                        row_info((jb + 1) * LPR, ob, xb, sb);
+                        fetch(ob, xb, sb, rb, wb);
+                        __builtin_amdgcn_sched_barrier(0);
+                        accumulate(ra, wa);
+                        __builtin_amdgcn_sched_barrier(0);
+                        accumulate(rb, wb);
+                    } else {
+                        accumulate(ra, wa);
+                    }
                 }
                 // Interior pixels (reachable from this tile's cells only) are this
                 // block's alone.  With one batch their sums are final; with
@@ -2394,6 +2420,8 @@ __global__ __launch_bounds__(512) void dcn2_gi_gather_kernel(const BwdParams p) 
 // (com.cu:553-609).
 // Mean samples per bucket from which the host takes dcn2_gi_push_kernel.
 constexpr int kPushMinPerBucket = 1024;
+// ... and (bucket, channel chunk) pairs from which it does.
+constexpr int kPushMinPairs = 128;
 
 template <typename T>
 __global__ __launch_bounds__(512) void dcn2_gi_push_kernel(const BwdParams p) {
@@ -2420,12 +2448,14 @@ __global__ __launch_bounds__(512) void dcn2_gi_push_kernel(const BwdParams p) {
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int nb = p.B * p.G * p.nty * p.ntx;
-    const int bucket = xcd_remap(blockIdx.x, nb);
+    // part of the bucket's work: channel chunks [cc0, cc1)
+    const int id = xcd_remap(blockIdx.x, nb * p.gi_cs), part = id % p.gi_cs, bucket = id / p.gi_cs;
     const int tx = bucket % p.ntx, ty = (bucket / p.ntx) % p.nty;
     const int bg = bucket / (p.ntx * p.nty), b = bg / p.G, g = bg - b * p.G;
     const int row0 = p.bstart[bucket], count = p.bstart[bucket + 1] - row0;
     const int oy = ty * TS - 1, ox = tx * TS - 1;  // pixel of local (0, 0)
     const int cpg = p.Cgp / KC;
+    const int cc0 = cpg * part / p.gi_cs, cc1 = cpg * (part + 1) / p.gi_cs;
     const int co = lane % LPR, gq = lane / LPR;
     const int row_bytes = p.Cgp * (int)sizeof(R);
     const int slice = co * 16 * NLD;
@@ -2436,14 +2466,14 @@ __global__ __launch_bounds__(512) void dcn2_gi_push_kernel(const BwdParams p) {
     };
     typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
-    for (int cc = 0; cc < cpg; ++cc) {
-        if (cc > 0) __syncthreads();  // the previous chunk's window is written out
+    for (int cc = cc0; cc < cc1; ++cc) {
+        if (cc > cc0) __syncthreads();  // the previous chunk's window is written out
         for (int i = tid; i < TW * TW * KC / 4; i += 512)
             reinterpret_cast<f32x4 *>(win)[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
         for (int base = 0; base < count; base += kGatherBatch) {
             const int nrec = min(count - base, kGatherBatch);
             __syncthreads();  // the window is clear / the previous batch is done with the LDS arrays
-            if (cc == 0 || count > kGatherBatch) {
+            if (cc == cc0 || count > kGatherBatch) {
                 // 1. counting sort by cell (cell = local row * TS + local column)
                 const BucketRec *__restrict__ recs = p.rec + (size_t)row0 + base;
                 for (int i = tid; i < NCELL; i += 512) ccnt[i] = 0;
@@ -3111,8 +3141,17 @@ static hipError_t backward_t(const Geo &g, const BwdParams &p0, void *grad_input
         p.gi_nhwc = g.nhwc;
         const int align16 = ((uintptr_t)grad_input & 15) == 0;
         p.gi_vec = align16 && (g.nhwc ? g.C % 8 == 0 && g.Cg % 8 == 0 : g.W % 8 == 0);
+        // Few buckets: their channel chunks (and, per pixel, their window passes)
+        // are shared out over workgroups until every CU has one; each part sorts
+        // the bucket's records itself.  Kernel us, one workgroup per bucket against
+        // this rule: 337 -> 49 (32 buckets of 32 chunks, fp32 1x1 at 32 x 14 x 14),
+        // 85 -> 15 (32 of 16, 32 x 7 x 7), by cells 65 -> 23 (64 of 4, fp32 3x3 at 4 x
+        // 56 x 56), 115 -> 35 (12 of 4, bf16 3x3 at 2 x 25 x 42).  Two or four to a CU
+        // measured 50-55, 17-22, 23, 35: the sorts repeat.
+        const int gcpg = g.Cgp / g.KC;
         if (gg.by_cells) {
-            dcn2_gi_push_kernel<T><<<nbk, 512, 0, s>>>(p);
+            p.gi_cs = std::min(gcpg, ceil_div(ncu, nbk));
+            dcn2_gi_push_kernel<T><<<nbk * p.gi_cs, 512, 0, s>>>(p);
         } else {
             // At most two workgroups per CU (extra LDS reserved at launch when
             // the static LDS leaves room for three): each bucket's rows are read
@@ -3124,7 +3163,9 @@ static hipError_t backward_t(const Geo &g, const BwdParams &p0, void *grad_input
                                       dev) != hipSuccess)
                 lds_cu = 0;
             const int pad = std::max(0, lds_cu / 3 + 256 - gather_static_lds(kRowScaled<T>));
-            dcn2_gi_gather_kernel<T><<<nbk, 512, pad, s>>>(p);
+            p.gi_cs = std::min(gcpg, ceil_div(ncu, nbk));
+            p.gi_rs = std::min(4, std::max(1, ncu / (nbk * p.gi_cs)));
+            dcn2_gi_gather_kernel<T><<<nbk * p.gi_cs * p.gi_rs, 512, pad, s>>>(p);
         }
         if ((e = hipGetLastError()) != hipSuccess) return e;
         // the tile-boundary pixels from the border rings, and grad_weight /
@@ -3170,9 +3211,13 @@ GatherGeo gather_geometry(const Geo &g) {
     // full enough to amortise a block's fixed work; per pixel otherwise.
     // Option DCN2_OPT_GI_PUSH = 1 / 0 forces either.  Measured: c2 68
     // against 72 us, c3 ~190 against 282 us (2304 samples per bucket); c4
-    // (576 per bucket) ~118 against 73 us.
+    // (576 per bucket) ~118 against 73 us.  With few (bucket, channel chunk)
+    // pairs the per-pixel kernel's passes still split four ways: 24 against 43
+    // us for the stage at 48 pairs (bf16 3x3, 2 x 25 x 42, C 256), 33 against 31
+    // at 256 (fp32 3x3, 4 x 56 x 56, C 128).
     gg.by_cells = g.opt_push >= 0 ? g.opt_push != 0
-                                  : gg.rows >= (long)kPushMinPerBucket * gg.nbuckets;
+                                  : gg.rows >= (long)kPushMinPerBucket * gg.nbuckets &&
+                                        gg.nbuckets * (g.Cgp / g.KC) >= kPushMinPairs;
     gg.acc_bytes = gg.rows / (kGatherBatch + 1) * (long)(kCellTile - 1) * (kCellTile - 1) * g.Cgp *
                    (long)sizeof(float);
     return gg;
@@ -3237,6 +3282,7 @@ hipError_t launch_backward(const Geo &g, const void *xt, const void *wt, const v
     p.ring = ring;
     p.gi_out = nullptr;  // (set by the by-cells grad_input)
     p.gi_nhwc = p.gi_vec = 0;
+    p.gi_cs = p.gi_rs = 1;
     switch (g.dtype) {
     case DCN2_F16: return backward_t<f16>(g, p, grad_input, grad_weight, grad_bias, last, s);
     case DCN2_BF16: return backward_t<bf16>(g, p, grad_input, grad_weight, grad_bias, last, s);
