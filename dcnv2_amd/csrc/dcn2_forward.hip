@@ -1,28 +1,14 @@
-// Fused DCNv2 forward for gfx950: bilinear, mask-modulated sampling into LDS
-// feeding a 32x32 MFMA GEMM, never materialising the column matrix.
+// Fused DCNv2 forward for gfx950, persistent role-specialised kernel (2-byte
+// types): bilinear, mask-modulated sampling into LDS feeding a 32x32 MFMA GEMM,
+// never materialising the column matrix.
 //
 // Reference: im2colcuda + dcn_bilinear_cuda write columns[B][C*kh*kw][N] to
 // HBM (com.cu:119-195), then gemm_cuda reads them back (com.cu:46-117).  Here
-// one workgroup owns a BM x BN output tile (all of Cout when Cout <= 256) and
-// walks K in chunks of KC channels of one (tap, group):
-//
-//   for chunk ch:                       (double-buffered LDS stage sB[2])
-//     load offset/mask of ch+3                       -- raw bits, used next step
-//     issue A (weight) fragment loads for ch+1      -- global/L2, 16 B per lane
-//     descriptors + corner gathers for ch+2          -- channels-last xt
-//     MFMA over sB[ch&1]                             -- matrix cores
-//     bilinear blend of ch+1 (gathered one step ago) -> sB[(ch+1)&1]
-//     barrier
-//
-// so a corner gather has a whole step (an MFMA phase and a barrier) to land
-// before its blend, and its offsets were loaded a step before that.
-// Each sampled value is produced once per workgroup and reused by every output
-// channel of the tile.
-//
-// Threads: 512 (8 waves) as WM x WN waves, each wave owning a 64x64 output
-// sub-tile = 2x2 MFMA 32x32 blocks.  Sampling slot = (pixel, quarter of the
-// chunk): 4 lanes cover one pixel's KC channels, so one corner of one pixel is
-// read as a contiguous KC*sizeof(T)-byte run across 4 adjacent lanes.
+// one workgroup owns an output tile (all of Cout when Cout <= 256) and walks K in
+// chunks of KC channels of one (tap, group); each sampled value is produced once
+// per workgroup and reused by every output channel of the tile.  Few-tile shapes
+// and fp32 take dcn2_forward_tiles.hip.
+#include <algorithm>
 #include <type_traits>
 
 #include "dcn2_common.h"
@@ -50,242 +36,6 @@ struct FwdParams {
     long long off_bs, msk_bs;   // offset / mask elements between images
     int msk_logit;              // mask buffer holds logits (see mask_value)
 };
-
-template <typename T, int WM, int WN, int IB, int JB, bool MASK>
-__global__ __launch_bounds__(512) void dcn2_fwd_kernel(const FwdParams p) {
-    using M = Mma<T>;
-    using frag = typename M::frag;
-    constexpr int KC = M::KC, KPL = M::KPL, KSTEP = M::KSTEP, NKS = KC / KSTEP;
-    constexpr int BN = 32 * JB * WN;            // each wave: 32*IB rows x 32*JB pixels
-    constexpr int BM = 32 * IB * WM;
-    static_assert(WM * WN == 8, "8 waves");
-    constexpr int CPS = KC / 4;                 // channels per sampling slot
-    constexpr int U4 = CPS * sizeof(T) / 16;    // 16-byte registers per corner per slot (2)
-    constexpr int SPT = BN * 4 / 512;           // sampling slots per thread
-    constexpr int LDK = KC + 16 / sizeof(T);    // LDS pitch (elements) of one pixel row
-    static_assert(U4 == 2, "slot is 32 bytes per corner");
-
-    // LDS: the two sampled-column stages during the K loop; afterwards the
-    // same memory stages each wave's output tile for 16-byte row stores.
-    constexpr int LDO = 32 * JB + 16 / sizeof(T);  // pitch (elements) of an output row
-    constexpr size_t kStageBytes = sizeof(T) * 2 * BN * LDK;
-    constexpr size_t kOutBytes = sizeof(T) == 2 ? sizeof(T) * 8 * 32 * IB * LDO : 0;
-    __shared__ __attribute__((aligned(16))) char smem[kStageBytes > kOutBytes ? kStageBytes
-                                                                              : kOutBytes];
-    T(&sB)[2][BN][LDK] = *reinterpret_cast<T(*)[2][BN][LDK]>(smem);
-
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave / WN, wn = wave - wm * WN;
-    // Tiles are numbered (image, pixel tile, M tile) and handed to XCDs in
-    // contiguous ranges: consecutive workgroup ids go round-robin over the 8
-    // XCDs, so XCD x receives the ids x, x+8, ... and is given the x-th range.
-    // Neighbouring tiles of one image then share that XCD's L2 for their
-    // corner gathers.
-    const int t = xcd_remap(blockIdx.x, p.tiles);
-    const int mt = t % p.mtiles, nt = (t / p.mtiles) % p.ntiles, b = t / (p.mtiles * p.ntiles);
-    const int n0 = nt * BN, m0 = (p.mt_base + mt) * BM;
-    const int N = p.Ho * p.Wo, KK = p.kh * p.kw, cs = p.G * p.Cgp;
-    const int nch_all = p.Kp / KC;         // chunks of the packed weight rows
-    const int nch = p.nch_eff, last = nch - 1;  // chunks walked (see FwdParams)
-    // j-th chunk of the walk -> packed chunk index
-    auto chmap = [&](int j) __attribute__((always_inline)) {
-        j = min(j, last);
-        const int tap = j / p.cpw;
-        return tap * p.cpt + p.cb + (j - tap * p.cpw);
-    };
-
-    const T *__restrict__ xt = (const T *)p.xt + (size_t)b * p.H * p.W * cs;
-    const T *__restrict__ offs = (const T *)p.offset + (size_t)b * p.off_bs;
-    const T *__restrict__ msk = MASK ? (const T *)p.mask + (size_t)b * p.msk_bs : nullptr;
-    const ChunkEnt *__restrict__ tab = (const ChunkEnt *)p.tab;
-
-    SampleGeo sg;
-    sg.H = p.H; sg.W = p.W; sg.kh = p.kh; sg.kw = p.kw; sg.sh = p.sh; sg.sw = p.sw;
-    sg.ph = p.ph; sg.pw = p.pw; sg.dh = p.dh; sg.dw = p.dw; sg.G = p.G; sg.Cgp = p.Cgp;
-    sg.Wo = p.Wo; sg.N = N; sg.cs = cs; sg.KK = KK; sg.msk_logit = p.msk_logit;
-
-    // Chunk c lives in set c % 2 of every pipeline buffer: offset/mask bits
-    // om, corner gathers smp, A fragments a and the LDS stage sB.  The loop
-    // is unrolled by two so that every set index is a compile-time constant,
-    // and stages past the last chunk re-read the last chunk (clamped table
-    // index) instead of branching, so one step is one basic block and the
-    // scheduler can interleave its MFMA with the VALU work of the next chunk.
-    Sampler<T, SPT, MASK> smp[2];
-    smp[0].init(tid);
-    smp[1].init(tid);
-    SlotOM<T, SPT> om[2];
-    frag a[2][IB][NKS];
-
-    auto ent = [&](int ch) __attribute__((always_inline)) { return tab[chmap(ch)]; };
-
-    // Bilinear blend of sampler set SET, stored to LDS stage SET as
-    // [pixel][channel] rows (the MFMA B-operand order).
-    auto store_stage = [&](auto set_c) __attribute__((always_inline)) {
-        constexpr int SET = decltype(set_c)::value;
-#pragma unroll
-        for (int s = 0; s < SPT; ++s) {
-            const int pl = (tid + s * 512) >> 2;
-            uint4 *dst = reinterpret_cast<uint4 *>(&sB[SET][pl][smp[SET].q * CPS]);
-#pragma unroll
-            for (int u = 0; u < U4; ++u) {
-                float v[16 / sizeof(T)];
-                smp[SET].blend(s, u, v);
-                dst[u] = pack16<T>(v);
-            }
-        }
-    };
-
-    // A (weight) fragments of rows m0 + wm*64 + i*32 + lane%32, packed in
-    // fragment order (pack_weight_kernel layout 0): the fragment (row block
-    // rb, chunk ch, step ks) is 64 lanes x KPL contiguous elements.
-    const T *wfrag[IB];
-#pragma unroll
-    for (int i = 0; i < IB; ++i)
-        wfrag[i] = (const T *)p.wp + ((size_t)((m0 + wm * 32 * IB + i * 32) / 32) * nch_all * NKS * 64 +
-                                      lane) * KPL;
-    auto load_a = [&](auto set_c, int ch) __attribute__((always_inline)) {
-        constexpr int SET = decltype(set_c)::value;
-        const int c = chmap(ch) * NKS * 64 * KPL;
-#pragma unroll
-        for (int i = 0; i < IB; ++i)
-#pragma unroll
-            for (int ks = 0; ks < NKS; ++ks)
-                a[SET][i][ks] = *reinterpret_cast<const frag *>(wfrag[i] + c + ks * 64 * KPL);
-    };
-
-    // The accumulators start at the bias of their output row, so the
-    // epilogue only rounds and stores.
-    f32x16 acc[IB][JB];
-    const T *bias = (const T *)p.bias;
-#pragma unroll
-    for (int i = 0; i < IB; ++i)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int m = m0 + wm * 32 * IB + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-            const float bv = (bias && m < p.Cout) ? to_f32(bias[m]) : 0.0f;
-#pragma unroll
-            for (int j = 0; j < JB; ++j) acc[i][j][r] = bv;
-        }
-
-    auto mfma_chunk = [&](auto set_c) __attribute__((always_inline)) {
-        constexpr int SET = decltype(set_c)::value;
-        frag bf[NKS][JB];
-#pragma unroll
-        for (int ks = 0; ks < NKS; ++ks)
-#pragma unroll
-            for (int j = 0; j < JB; ++j)
-                bf[ks][j] = *reinterpret_cast<const frag *>(
-                    &sB[SET][(wn * JB + j) * 32 + (lane & 31)][ks * KSTEP + (lane >> 5) * KPL]);
-#pragma unroll
-        for (int ks = 0; ks < NKS; ++ks)
-#pragma unroll
-            for (int i = 0; i < IB; ++i)
-#pragma unroll
-                for (int j = 0; j < JB; ++j)
-                    acc[i][j] = M::mma(a[SET][i][ks], bf[ks][j], acc[i][j]);
-    };
-
-    // One pipeline step for chunk ch, set S = ch % 2, O = S ^ 1:
-    //   offset/mask bits of ch+3 -> om[O]     A fragments of ch+1 -> a[O]
-    //   corner gathers of ch+2 (om[S]) -> smp[S]
-    //   MFMA of ch (a[S], sB[S])              blend of ch+1 (smp[O]) -> sB[O]
-    // Chunk-table entries of ch+2 and ch+3 are held in scalar registers and
-    // the entry of ch+4 is fetched one step ahead, so no step starts by
-    // waiting for a scalar load.
-    ChunkEnt e2 = ent(2), e3 = ent(3);
-    auto step = [&](auto s_c, int ch) __attribute__((always_inline)) {
-        constexpr int S = decltype(s_c)::value;
-        constexpr int O = S ^ 1;
-        // Loads whose results the next step consumes go first, so that the
-        // in-order load counter lets the next step wait for them without
-        // also waiting for this step's corner gathers.
-        smp[0].load_om(n0, e3.x, sg, tid, offs, msk, om[O]);
-        load_a(std::integral_constant<int, O>{}, ch + 1);
-        const ChunkEnt e4 = ent(ch + 4);
-        __builtin_amdgcn_sched_barrier(0);
-        smp[S].issue(e2, sg, xt, om[S]);
-        mfma_chunk(std::integral_constant<int, S>{});
-        store_stage(std::integral_constant<int, O>{});
-        // Interleave: each MFMA (32 cycles of the matrix core) is followed by
-        // a slice of the blend / descriptor VALU work and one LDS read.
-        __builtin_amdgcn_sched_group_barrier(0x100, JB * NKS, 0);  // all B-fragment reads
-#pragma unroll
-        for (int i = 0; i < IB * JB * NKS; ++i) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-            __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);  // VALU
-        }
-        __syncthreads();
-        e2 = e3;
-        e3 = e4;
-    };
-
-    // Prologue: offset/mask bits of chunks 0, 1, 2; gathers of chunks 0 and
-    // 1; chunk 0 blended into stage 0.
-    {
-        const ChunkEnt e0 = ent(0), e1 = ent(1);
-        smp[0].load_om(n0, e0.x, sg, tid, offs, msk, om[0]);
-        smp[0].load_om(n0, e1.x, sg, tid, offs, msk, om[1]);
-        load_a(std::integral_constant<int, 0>{}, 0);
-        smp[0].issue(e0, sg, xt, om[0]);
-        smp[0].load_om(n0, e2.x, sg, tid, offs, msk, om[0]);
-        smp[1].issue(e1, sg, xt, om[1]);
-        store_stage(std::integral_constant<int, 0>{});
-        __syncthreads();
-    }
-    int ch = 0;
-    for (; ch + 1 < nch; ch += 2) {
-        step(std::integral_constant<int, 0>{}, ch);
-        step(std::integral_constant<int, 1>{}, ch + 1);
-    }
-    if (ch < nch) step(std::integral_constant<int, 0>{}, ch);
-
-    // Epilogue: round to T and store.  For 2-byte types with an NCHW output
-    // of aligned, 8-divisible rows each wave stages its 32*IB x 32*JB tile in
-    // LDS (the K loop's stages are free after its last barrier) and writes
-    // whole 16-byte row segments; otherwise every lane stores its own elements.
-    T *out = (T *)p.out + (size_t)b * p.Cout * N;
-    if constexpr (sizeof(T) == 2) {
-        if (p.out_vec) {
-            T *so = reinterpret_cast<T *>(smem) + (size_t)wave * 32 * IB * LDO;
-#pragma unroll
-            for (int i = 0; i < IB; ++i)
-#pragma unroll
-                for (int j = 0; j < JB; ++j)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                        so[(i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * LDO + j * 32 +
-                           (lane & 31)] = from_f32<T>(acc[i][j][r]);
-            // each row is 32*JB elements = 4*JB segments of 8; a wave
-            // instruction covers 64 segments
-            constexpr int SEG = 4 * JB, ROWS = 32 * IB;
-#pragma unroll
-            for (int it = 0; it < ROWS * SEG / 64; ++it) {
-                const int sidx = it * 64 + lane;
-                const int row = sidx / SEG, seg = sidx - row * SEG;
-                const int m = m0 + wm * ROWS + row, n = n0 + wn * 32 * JB + seg * 8;
-                const uint4 v = *reinterpret_cast<const uint4 *>(so + row * LDO + seg * 8);
-                if (m < p.Cout && n < N)  // N % 8 == 0: a segment is all in or all out
-                    *reinterpret_cast<uint4 *>(out + (size_t)m * N + n) = v;
-            }
-            return;
-        }
-    }
-    // element stores: NCHW (m * N + n) or channels-last (n * Cout + m)
-    const size_t ms = p.out_nhwc ? 1 : (size_t)N, ns = p.out_nhwc ? (size_t)p.Cout : 1;
-#pragma unroll
-    for (int i = 0; i < IB; ++i) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int m = m0 + wm * 32 * IB + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-            if (m >= p.Cout) continue;
-#pragma unroll
-            for (int j = 0; j < JB; ++j) {
-                const int n = n0 + (wn * JB + j) * 32 + (lane & 31);
-                if (n < N) out[m * ms + n * ns] = from_f32<T>(acc[i][j][r]);
-            }
-        }
-    }
-}
 
 // ---------------------------------------------------------------------------
 // Warp-specialised forward for 2-byte types (f16, bf16).
@@ -353,8 +103,9 @@ template <typename T> struct Blend8 {
     }
 };
 
-// Rows of the LDS bias table of the warp-specialised forward.
-constexpr int kBiasRows = 1024;
+// Rows of the LDS bias table of the warp-specialised forward (32 KB: one workgroup
+// to a CU either way), and so of a launch.
+constexpr int kBiasRows = 8192;
 
 // MASK: 0 no mask (all ones), 1 mask values, 2 mask logits (sigmoid on load);
 // a compile-time mode keeps the descriptor code free of branches, so it can
@@ -547,12 +298,14 @@ __global__ __launch_bounds__(512) void dcn2_fwd_ws_kernel(const FwdParams p) {
         f32x16 acc[IB][JB];
         const T *bias = (const T *)p.bias;
         const T *wbase = (const T *)p.wp + (size_t)lane * KPL;
-        // Bias of this wave's rows of every M tile in LDS (fp32, 0 past Cout;
-        // the host guarantees Mp <= kBiasRows), so starting a tile never waits
+        // Bias of this wave's rows of every M tile of the launch in LDS (fp32, 0
+        // past Cout; the host keeps a launch within kBiasRows rows), so starting a tile never waits
         // on a global load queued behind the A loads in flight.  Each wave
         // writes and reads only its own rows: no barrier needed.
-        for (int m = lane; m < p.Mp; m += 64)
-            if ((m / ROWS) % 4 == rw) sBias[m] = (bias && m < p.Cout) ? to_f32(bias[m]) : 0.0f;
+        const int mrow0 = p.mt_base * 4 * ROWS;
+        for (int r = lane; r < p.mtiles * 4 * ROWS; r += 64)
+            if ((r / ROWS) % 4 == rw)
+                sBias[r] = (bias && mrow0 + r < p.Cout) ? to_f32(bias[mrow0 + r]) : 0.0f;
         // The MFMAs compute the transposed tile D^T[n][m] (the weight
         // fragment is the B operand, the sampled columns the A operand; both
         // operands have the same register layout), so lane l holds output
@@ -570,7 +323,7 @@ __global__ __launch_bounds__(512) void dcn2_fwd_ws_kernel(const FwdParams p) {
 #pragma unroll
                     for (int rq = 0; rq < 4; ++rq) {
                         const f32x4 b4 = *reinterpret_cast<const f32x4 *>(
-                            &sBias[m0 + rw * ROWS + i * 32 + 8 * rq + 4 * (lane >> 5)]);
+                            &sBias[m0 - mrow0 + rw * ROWS + i * 32 + 8 * rq + 4 * (lane >> 5)]);
 #pragma unroll
                         for (int j = 0; j < JB; ++j)
 #pragma unroll
@@ -580,7 +333,7 @@ __global__ __launch_bounds__(512) void dcn2_fwd_ws_kernel(const FwdParams p) {
                 typedef unsigned long long u64x8 __attribute__((ext_vector_type(8)));
 #pragma unroll
                 for (int i = 0; i < IB; ++i) {
-                    const uint32_t bb = __float_as_uint(sBias[m0 + rw * ROWS + i * 32 + (lane & 31)]);
+                    const uint32_t bb = __float_as_uint(sBias[m0 - mrow0 + rw * ROWS + i * 32 + (lane & 31)]);
                     const unsigned long long b2 = ((unsigned long long)bb << 32) | bb;
 #pragma unroll
                     for (int j = 0; j < JB; ++j) acc[i][j] = __builtin_bit_cast(f32x16, u64x8(b2));
@@ -878,19 +631,6 @@ __global__ __launch_bounds__(512) void dcn2_fwd_ws_kernel(const FwdParams p) {
     }
 }
 
-template <typename T, int WM, int WN, int IB, int JB>
-static hipError_t launch_fwd_t(const Geo &g, const FwdParams &p0, hipStream_t s) {
-    FwdParams p = p0;
-    p.ntiles = ceil_div(g.N, 32 * JB * WN);
-    p.tiles = g.B * p.ntiles * p.mtiles;
-    p.out_vec = !p.out_nhwc && (g.N % 8 == 0) && (((uintptr_t)p.out & 15) == 0);
-    if (p.mask)
-        dcn2_fwd_kernel<T, WM, WN, IB, JB, true><<<p.tiles, 512, 0, s>>>(p);
-    else
-        dcn2_fwd_kernel<T, WM, WN, IB, JB, false><<<p.tiles, 512, 0, s>>>(p);
-    return hipGetLastError();
-}
-
 // Warp-specialised kernel for 2-byte types: persistent grid of one
 // workgroup per CU (at most one tile per workgroup more than the average).
 template <typename T, int IB>
@@ -939,24 +679,33 @@ static bool ws_two_waves_per_simd() {
     return ok;
 }
 
-// One launch over the output rows [row0, row0 + rows) with M tile bm (256 or
-// 128 rows; rows and row0 are multiples of it).  fp32 (and 2-byte types with
-// more than kBiasRows padded output rows): block tile 256x128 (8 waves of
-// 32x128) when bm is 256, else 128x128 (8 waves of 64x32); both sample 128
-// pixels, one slot per thread.
+// The tile kernels serve this kernel's shapes when it would have few tiles (of 128
+// pixels of one image x 256 rows, or 128 up to 128 rows) per launch, or a register
+// count that would let three waves share a SIMD.
+// Measured (us, this kernel against those, fp16 3x3): 53.8 against 45.4 at 128 tiles
+// (Cout 256, C 256), 56.0 against 61.2 at 192; 27.2 against 20.5 at 128 (Cout 128, C
+// 128), 29.6 against 32.8 at 256; 19.9 against 14.0 at 128 (Cout 64, C 64), 33.2
+// against 38.6 at 512.
+constexpr int kWsMinTiles = 160;
+static bool ws_few_tiles(const Geo &g) {
+    const int rows = std::min(g.gsplit ? g.Cout / g.WG : g.Cout, kBiasRows);
+    if ((long long)g.B * ceil_div(g.N, 128) * ceil_div(rows, rows > 128 ? 256 : 128) < kWsMinTiles) return true;
+    return g.dtype == DCN2_F16 ? !(ws_two_waves_per_simd<f16, 1>() && ws_two_waves_per_simd<f16, 2>())
+                               : !(ws_two_waves_per_simd<bf16, 1>() && ws_two_waves_per_simd<bf16, 2>());
+}
+
+// The output rows [row0, row0 + rows) with M tile bm (256 or 128 rows; rows and
+// row0 are multiples of it), at most kBiasRows to a launch.
 template <typename T>
 static hipError_t launch_fwd_dt(const Geo &g, FwdParams p, int bm, int row0, int rows,
                                 hipStream_t s) {
-    p.mt_base = row0 / bm;
-    p.mtiles = rows / bm;
-    if (g.Mp <= kBiasRows) {
-        if (bm == 256 && ws_two_waves_per_simd<T, 2>()) return launch_fwd_ws<T, 2>(g, p, s);
-        if (bm == 128 && ws_two_waves_per_simd<T, 1>()) return launch_fwd_ws<T, 1>(g, p, s);
+    for (int r = 0; r < rows; r += kBiasRows) {
+        p.mt_base = (row0 + r) / bm;
+        p.mtiles = std::min(kBiasRows, rows - r) / bm;
+        const hipError_t e = bm == 256 ? launch_fwd_ws<T, 2>(g, p, s) : launch_fwd_ws<T, 1>(g, p, s);
+        if (e != hipSuccess) return e;
     }
-    // more than kBiasRows output rows (or a register count that would let
-    // three waves share a SIMD): the non-specialised kernel
-    if (bm == 256) return launch_fwd_t<T, 8, 1, 1, 4>(g, p, s);
-    return launch_fwd_t<T, 2, 4, 2, 1>(g, p, s);
+    return hipSuccess;
 }
 
 // Ungrouped (or not splittable): one launch over every row and chunk.  With
@@ -987,8 +736,8 @@ hipError_t launch_forward(const Geo &g, const void *xt, const void *wp, const vo
                           const void *offset, const void *mask, const void *bias, void *out,
                           hipStream_t s) {
     if (g.B == 0) return hipSuccess;
-    if (g.dtype == DCN2_F32)
-        return launch_forward_f32(g, xt, wp, tab, offset, mask, bias, out, s);
+    if (g.dtype == DCN2_F32 || ws_few_tiles(g))
+        return launch_forward_tiles(g, xt, wp, tab, offset, mask, bias, out, s);
     FwdParams p;
     p.xt = xt;
     p.wp = wp;

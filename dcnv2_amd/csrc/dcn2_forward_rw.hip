@@ -543,7 +543,12 @@ void dcn2_fwd_rw_kernel(const RwParams p) {
     for (int it = 0; it < 8; it += 2) flush_out(prv, it);
 }
 
+// Fewer than 48 tiles of 128 pixels leave most CUs without one, and each workgroup
+// first loads the whole weight: dcn2_forward_tiles.hip takes them (us, this kernel
+// against that, Cout 256, C 64: 13.6 / 10.9 at 8 tiles, 14.2 / 11.8 at 32, 14.9 / 15.3
+// at 64).
 bool rw_eligible(const Geo &g) {
+    if ((long long)g.B * ceil_div(g.N, 128) < 48) return false;
     return g.dtype == DCN2_F16 && g.G == 1 && g.Cgp == 64 && g.KK == kRwTaps && g.Mp == 256 &&
            g.WG == 1 && (g.out_nhwc ? g.Cout % 8 == 0 : g.N % 8 == 0) &&
            (long long)g.Cout * g.N * 2 < 0x7fffffffLL;

@@ -1,33 +1,37 @@
-// Fused DCNv2 forward for fp32: bilinear, mask-modulated sampling into LDS
-// feeding 32x32x2 fp32 MFMAs (the reference's im2colcuda + gemm_cuda,
-// com.cu:46-195, without the column matrix in HBM).
+// Fused DCNv2 forward in small tiles: bilinear, mask-modulated sampling into LDS
+// feeding 32x32 MFMAs (the reference's im2colcuda + gemm_cuda, com.cu:46-195,
+// without the column matrix in HBM).  Serves every fp32 shape, and the 2-byte
+// shapes that have too few 128-pixel tiles for the persistent kernels of
+// dcn2_forward.hip / dcn2_forward_rw.hip or more rows than those hold.
 //
-// Bound: the fp32 matrix rate.  One 32x32x2 MFMA holds the matrix core for 64
-// cycles, so a wave needs few operand reads per cycle, and small workgroups of
-// 4 waves, several to a CU, hide the sampling behind each other's MFMAs
-// without role-specialised waves.  What cost the time before (8-wave workgroups
-// of 128 pixels of one image, one to a CU) was idle CUs and padding: a 14 x 14
-// map filled 196 of 256 tile pixels and ran two workgroups per image.  So:
+// Bound: for fp32 the matrix rate (a 32x32x2 MFMA holds the matrix core for 64
+// cycles, so workgroups of 4 or 8 waves hide their sampling behind each other's
+// MFMAs without role-specialised waves); for the small problems the chain of
+// gathers, blend and barrier of a step (about 1.2 us at one workgroup to a CU;
+// issuing the gathers two steps ahead and fetching table entries a step early
+// both measured the same).  What cost the time before was idle CUs and padding: a
+// 14 x 14 map filled 196 of 256 tile pixels and ran two workgroups per image.  So:
 //   * output pixels are numbered through the whole batch (pixel i of the launch
 //     is pixel i % N of image i / N), and a tile may span images;
-//   * the tile is chosen by how many workgroups it gives (launch_forward_f32),
-//     and where they are few K is split over the waves of a workgroup (WK).
-// Measured against the 8-wave kernel this replaces (us): 79.0 -> 64.7 at Cout 256,
-// K 64, 32 x 56 x 56; 174.9 -> 49.9 at 256, 1024, 32 x 14 x 14; 100.2 -> 48.7 at
-// 2048, 512, 32 x 7 x 7; 111.2 -> 59.9 at 128, 1152, 4 x 56 x 56 (3x3); 31.3 ->
-// 9.6 at 32, 144, 32 x 32 (3x3).  The 3.29 GFLOP of the first three take 21 us at
-// the 154 TFLOP/s a large fp32 matrix product reaches here.
+//   * the tile is chosen by how many workgroups it gives (forward_tiles), and where
+//     they are few K is split over the waves of a workgroup (WK).
+// Measured against the kernels this replaces (us): fp32 79.0 -> 64.7 at Cout 256,
+// K 64, 32 x 56 x 56; 174.9 -> 50.7 at 256, 1024, 32 x 14 x 14; 100.2 -> 48.7 at
+// 2048, 512, 32 x 7 x 7; 111.2 -> 59.4 at 128, 1152, 4 x 56 x 56 (3x3); 31.3 -> 9.6
+// at 32, 144, 32 x 32 (3x3).  The 3.29 GFLOP of the first three take 21 us at the
+// 154 TFLOP/s a large fp32 matrix product reaches here.  16 bits, 3x3: 50.5 -> 32.8
+// at 256, 2304, 50 x 84; 65.3 -> 24.3 at 256, 2304, 2 x 25 x 42; 92.3 -> 32.0 at
+// 512, 4608, 32 x 32; 25.7 -> 13.5 at 128, 1152, 64 x 64.
 //
 // A workgroup owns 32*IB*WM output rows x 32*JB*WN pixels and walks K in steps
-// of WK chunks (32 channels of one tap and group each).  Step s:
+// of WK chunks (128 bytes of channels of one tap and group each).  Step s:
 //   weight fragments and corner gathers of step s+1, offsets of step s+2 issued
 //   MFMAs of step s over its LDS stage
 //   blend of step s+1 into the other stage; barrier
-// An MFMA multiplies K pairs {e, e + 4} of an 8-channel group (e = 0..3): both
-// operands of four MFMAs are then one 16-byte read per lane, four consecutive
-// channels of the lane's row (weight, straight from the fragment-ordered pack)
-// or pixel (LDS, pitch 36 floats: the 16-byte reads of 16 lanes cover all banks
-// once).
+// Operands are one 16-byte read per lane: a row's piece from the fragment-ordered
+// weight, a pixel's from LDS (pitch 144 bytes: the reads of 16 lanes cover all
+// banks once).  For 2-byte types that is one 32x32x16 MFMA; for fp32 four 32x32x2
+// ones, the e-th multiplying channels e and e + 4 of a group of 8.
 #include <algorithm>
 #include <type_traits>
 
@@ -38,10 +42,10 @@
 
 namespace dcn2 {
 
-struct F32FwdParams {
-    const float *xt, *wp, *offset, *mask, *bias;
+struct TileParams {
+    const void *xt, *wp, *offset, *mask, *bias;
     const int4 *tab;
-    float *out;
+    void *out;
     int H, W, Cout, N, Wo, sh, sw, ph, pw, cs;
     int nch_all;  // chunks of the packed weight rows
     // chunk walk of this launch (see FwdParams of dcn2_forward.hip): the
@@ -54,10 +58,10 @@ struct F32FwdParams {
     int msk_logit;
 };
 
-constexpr int kF32Pitch = 36;  // floats per pixel of an LDS stage (32 channels)
+constexpr int kTilePitch = 144;  // bytes per pixel of an LDS stage (one chunk: 128 bytes)
 
-template <int IB, int JB, int WM, int WN, int WK, bool MASK, bool ONHWC>
-__global__ __launch_bounds__(64 * WM * WN * WK) void dcn2_fwd_f32_kernel(const F32FwdParams p) {
+template <typename T, int IB, int JB, int WM, int WN, int WK, bool MASK, bool ONHWC>
+__global__ __launch_bounds__(64 * WM * WN * WK) void dcn2_fwd_tile_kernel(const TileParams p) {
     constexpr int NT = 64 * WM * WN * WK;
     constexpr int BM = 32 * IB * WM, BN = 32 * JB * WN;
     constexpr int PPP = NT / 8;            // (pixel, chunk) pairs sampled per pass
@@ -65,9 +69,9 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void dcn2_fwd_f32_kernel(const F
     static_assert(BN * WK % PPP == 0 && (BN % PPP == 0 || PPP % BN == 0), "whole passes");
     static_assert(WK == 1 || IB * JB * 4 % WK == 0, "the K split's reduction shares row quads out evenly");
     // the two sampled stages; after the last one the K split's partial blocks
-    constexpr int kStage = 2 * WK * BN * kF32Pitch, kRed = WK > 1 ? WK * WM * WN * 4 * 64 * 4 : 0;
-    __shared__ __attribute__((aligned(16))) float smem[kStage > kRed ? kStage : kRed];
-    float(&sB)[2][WK][BN][kF32Pitch] = *reinterpret_cast<float(*)[2][WK][BN][kF32Pitch]>(smem);
+    constexpr int kStage = 2 * WK * BN * kTilePitch, kRed = WK > 1 ? WK * WM * WN * 4 * 64 * 16 : 0;
+    __shared__ __attribute__((aligned(16))) char smem[kStage > kRed ? kStage : kRed];
+    char(&sB)[2][WK][BN][kTilePitch] = *reinterpret_cast<char(*)[2][WK][BN][kTilePitch]>(smem);
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -101,7 +105,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void dcn2_fwd_f32_kernel(const F
         return c;
     };
 
-    // Slot i of a thread: chunk slot_k(i) of the step, pixel slot_px(i), channels 4*(tid % 8) ..; 8 lanes read one 128-byte corner line.
+    // Slot i of a thread: chunk slot_k(i) of the step, pixel slot_px(i), 16-byte piece tid % 8 of the chunk; 8 lanes read one 128-byte corner line.
     const int cq = tid & 7;
     auto slot_px = [&](int i) __attribute__((always_inline)) { return (PPP * i + (tid >> 3)) % BN; };
     // (uniform over the wave)
@@ -119,42 +123,43 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void dcn2_fwd_f32_kernel(const F
         const int oy = nn / (unsigned)p.Wo, ox = nn - oy * p.Wo;
         by[i] = oy * p.sh - p.ph;
         bx[i] = ox * p.sw - p.pw;
-        ooff[i] = (b * (uint32_t)p.off_bs + nn) * 4u;
-        moff[i] = MASK ? (b * (uint32_t)p.msk_bs + nn) * 4u : 0u;
+        ooff[i] = (b * (uint32_t)p.off_bs + nn) * (uint32_t)sizeof(T);
+        moff[i] = MASK ? (b * (uint32_t)p.msk_bs + nn) * (uint32_t)sizeof(T) : 0u;
         ximg[i] = b * (uint32_t)(p.H * p.W);
     }
     const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<float *>(p.xt), (short)0, (int)p.x_bytes, 0x00020000);
+        const_cast<void *>(p.xt), (short)0, (int)p.x_bytes, 0x00020000);
     typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
     // Sampling state of a slot: the plane its descriptor (corner byte offsets
     // and mask-folded weights) is of, and the offsets loaded for the next one.
     // Chunks of one plane (the channel chunks of a group) share a descriptor.
-    float dy[SPT], dx[SPT], mv[SPT], w[SPT][4];
+    T dy[SPT], dx[SPT], mv[SPT];
+    float w[SPT][4];
     uint32_t co[SPT][4];
     int plane_d[SPT], plane_o[SPT];
     auto load_om = [&](int i, const Cursor &c) __attribute__((always_inline)) {
         const int plane = tab[4 * c.ch];
         if (plane == plane_d[i] || plane == plane_o[i]) return;
         plane_o[i] = plane;
-        const char *ob = (const char *)(p.offset + (size_t)plane * 2 * p.N);
-        dy[i] = *(const float *)(ob + ooff[i]);
-        dx[i] = *(const float *)(ob + (size_t)p.N * 4 + ooff[i]);
-        if (MASK) mv[i] = *(const float *)((const char *)(p.mask + (size_t)plane * p.N) + moff[i]);
+        const char *ob = (const char *)((const T *)p.offset + (size_t)plane * 2 * p.N);
+        dy[i] = *(const T *)(ob + ooff[i]);
+        dx[i] = *(const T *)(ob + (size_t)p.N * sizeof(T) + ooff[i]);
+        if (MASK) mv[i] = *(const T *)((const char *)((const T *)p.mask + (size_t)plane * p.N) + moff[i]);
     };
-    f32x4 raw[SPT][4];
+    u32x4 raw[SPT][4];
     auto gather = [&](int i, const Cursor &c) __attribute__((always_inline)) {
         const ConstTab e = tab + 4 * c.ch;
         if (e[0] != plane_d[i]) {
             plane_d[i] = e[0];
-            const float y = (float)(by[i] + e[1]) + dy[i];
-            const float x = (float)(bx[i] + e[2]) + dx[i];
-            float m = MASK ? mask_value(mv[i], p.msk_logit) : 1.0f;
+            const float y = (float)(by[i] + e[1]) + to_f32(dy[i]);
+            const float x = (float)(bx[i] + e[2]) + to_f32(dx[i]);
+            float m = MASK ? mask_value(to_f32(mv[i]), p.msk_logit) : 1.0f;
             m = live[i] ? m : 0.0f;
             const SamplePos sp = sample_pos(y, x, p.H, p.W);
             const float hy = (1.0f - sp.ly) * m, ly = sp.ly * m, hx = 1.0f - sp.lx, lx = sp.lx;
-            const uint32_t base = (ximg[i] + (uint32_t)(sp.y0 * p.W + sp.x0)) * (uint32_t)(p.cs * 4) + cq * 16u;
-            const uint32_t px = (uint32_t)p.cs * 4u, row = px * (uint32_t)p.W, out = p.x_bytes;
+            const uint32_t base = (ximg[i] + (uint32_t)(sp.y0 * p.W + sp.x0)) * (uint32_t)(p.cs * sizeof(T)) + cq * 16u;
+            const uint32_t px = (uint32_t)p.cs * (uint32_t)sizeof(T), row = px * (uint32_t)p.W, out = p.x_bytes;
             co[i][0] = sp.vy0 && sp.vx0 ? base : out;
             co[i][1] = sp.vy0 && sp.vx1 ? base + px : out;
             co[i][2] = sp.vy1 && sp.vx0 ? base + row : out;
@@ -167,31 +172,34 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void dcn2_fwd_f32_kernel(const F
         // (a corner outside the image has an offset past the buffer and reads 0)
 #pragma unroll
         for (int q = 0; q < 4; ++q)
-            raw[i][q] = __builtin_bit_cast(
-                f32x4, __builtin_amdgcn_raw_buffer_load_b128(xrs, (int)co[i][q], e[3] * 4, 0));
+            raw[i][q] = __builtin_amdgcn_raw_buffer_load_b128(xrs, (int)co[i][q], e[3] * (int)sizeof(T), 0);
     };
     auto blend = [&](int st) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < SPT; ++i) {
-            f32x4 v = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            constexpr int E = 16 / sizeof(T);
+            float v[E];
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
+            for (int e = 0; e < E; ++e) v[e] = 0.0f;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = fmaf(w[i][q], raw[i][q][e], v[e]);
-            *reinterpret_cast<f32x4 *>(&sB[st][slot_k(i)][slot_px(i)][cq * 4]) = v;
+            for (int q = 0; q < 4; ++q) {
+                float x[E];
+                Unpack<T>::run(make_uint4(raw[i][q].x, raw[i][q].y, raw[i][q].z, raw[i][q].w), x);
+#pragma unroll
+                for (int e = 0; e < E; ++e) v[e] = fmaf(w[i][q], x[e], v[e]);
+            }
+            *reinterpret_cast<uint4 *>(&sB[st][slot_k(i)][slot_px(i)][cq * 16]) = pack16<T>(v);
         }
     };
-    // weight fragments: row block rb, chunk ch, 8-channel group k8 -> 64 lanes x 4 floats
-    f32x4 a[2][IB][4];
-    const float *wrow = p.wp + (size_t)(m0 / 32) * p.nch_all * 1024 + lane * 4;
+    // weight fragments: row block rb, chunk ch, quarter ks of it -> 64 lanes x 16 bytes
+    u32x4 a[2][IB][4];
+    const u32x4 *wrow = (const u32x4 *)p.wp + (size_t)(m0 / 32) * p.nch_all * 256 + lane;
     auto load_a = [&](int set, const Cursor &cur) __attribute__((always_inline)) {
-        const size_t c = (size_t)cur.ch * 1024;
+        const u32x4 *src = wrow + (size_t)cur.ch * 256;
 #pragma unroll
         for (int i = 0; i < IB; ++i)
 #pragma unroll
-            for (int k8 = 0; k8 < 4; ++k8)
-                a[set][i][k8] = *reinterpret_cast<const f32x4 *>(
-                    wrow + (size_t)i * p.nch_all * 1024 + c + k8 * 256);
+            for (int ks = 0; ks < 4; ++ks) a[set][i][ks] = src[(size_t)i * p.nch_all * 256 + ks * 64];
     };
     f32x16 acc[IB][JB];
 #pragma unroll
@@ -203,21 +211,32 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void dcn2_fwd_f32_kernel(const F
     // Channels-last output: the operands swap, so that a lane holds one row
     // (m = lane % 32) of 16 pixels and stores run along the channels.
     auto mma = [&](int set) __attribute__((always_inline)) {
+        typedef typename Mma<T>::frag frag;
 #pragma unroll
-        for (int k8 = 0; k8 < 4; ++k8) {
-            f32x4 bf[JB];
+        for (int ks = 0; ks < 4; ++ks) {
+            u32x4 bf[JB];
 #pragma unroll
             for (int j = 0; j < JB; ++j)
-                bf[j] = *reinterpret_cast<const f32x4 *>(
-                    &sB[set][wk][(wn * JB + j) * 32 + (lane & 31)][k8 * 8 + 4 * (lane >> 5)]);
+                bf[j] = *reinterpret_cast<const u32x4 *>(
+                    &sB[set][wk][(wn * JB + j) * 32 + (lane & 31)][ks * 32 + 16 * (lane >> 5)]);
+            auto mul = [&](auto af, auto bv, int i, int j) __attribute__((always_inline)) {
+                acc[i][j] = ONHWC ? Mma<T>::mma(bv, af, acc[i][j]) : Mma<T>::mma(af, bv, acc[i][j]);
+            };
+            if constexpr (sizeof(T) == 4) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int i = 0; i < IB; ++i)
+#pragma unroll
+                        for (int j = 0; j < JB; ++j)
+                            mul(__uint_as_float(a[set][i][ks][e]), __uint_as_float(bf[j][e]), i, j);
+            } else {
 #pragma unroll
                 for (int i = 0; i < IB; ++i)
 #pragma unroll
                     for (int j = 0; j < JB; ++j)
-                        acc[i][j] = ONHWC ? Mma<float>::mma(bf[j][e], a[set][i][k8][e], acc[i][j])
-                                         : Mma<float>::mma(a[set][i][k8][e], bf[j][e], acc[i][j]);
+                        mul(__builtin_bit_cast(frag, a[set][i][ks]), __builtin_bit_cast(frag, bf[j]), i, j);
+            }
         }
     };
 
@@ -276,21 +295,21 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void dcn2_fwd_f32_kernel(const F
         if constexpr (ONHWC) {
             const int m = mb + lc;
             if (m >= p.m_end) return;
-            const float bv = p.bias ? p.bias[m] : 0.0f;
+            const float bv = p.bias ? to_f32(((const T *)p.bias)[m]) : 0.0f;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const int pl = pb + 8 * rq + lr + e;
-                if (pl < live_px) p.out[(size_t)(n0 + pl) * p.Cout + m] = v[e] + bv;
+                if (pl < live_px) ((T *)p.out)[(size_t)(n0 + pl) * p.Cout + m] = from_f32<T>(v[e] + bv);
             }
         } else {
             const int pl = pb + lc;
             if (pl >= live_px) return;
             const unsigned n = n0 + pl, b = n / (unsigned)p.N;
-            float *o = p.out + (size_t)b * p.Cout * p.N + (n - b * (unsigned)p.N);
+            T *o = (T *)p.out + (size_t)b * p.Cout * p.N + (n - b * (unsigned)p.N);
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const int m = mb + 8 * rq + lr + e;
-                if (m < p.m_end) o[(size_t)m * p.N] = v[e] + (p.bias ? p.bias[m] : 0.0f);
+                if (m < p.m_end) o[(size_t)m * p.N] = from_f32<T>(v[e] + (p.bias ? to_f32(((const T *)p.bias)[m]) : 0.0f));
             }
         }
     };
@@ -331,26 +350,26 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void dcn2_fwd_f32_kernel(const F
     }
 }
 
-template <int IB, int JB, int WM, int WN, int WK>
-static hipError_t launch_fwd_f32_t(F32FwdParams p, int rows, bool nhwc, hipStream_t s) {
+template <typename T, int IB, int JB, int WM, int WN, int WK>
+static hipError_t launch_tile(TileParams p, int rows, bool nhwc, hipStream_t s) {
     constexpr int NT = 64 * WM * WN * WK;
     p.mtiles = ceil_div(rows, 32 * IB * WM);
     p.tiles = ceil_div(p.total, 32 * JB * WN) * p.mtiles;
-    if (p.mask && nhwc) dcn2_fwd_f32_kernel<IB, JB, WM, WN, WK, true, true><<<p.tiles, NT, 0, s>>>(p);
-    else if (p.mask) dcn2_fwd_f32_kernel<IB, JB, WM, WN, WK, true, false><<<p.tiles, NT, 0, s>>>(p);
-    else if (nhwc) dcn2_fwd_f32_kernel<IB, JB, WM, WN, WK, false, true><<<p.tiles, NT, 0, s>>>(p);
-    else dcn2_fwd_f32_kernel<IB, JB, WM, WN, WK, false, false><<<p.tiles, NT, 0, s>>>(p);
+    if (p.mask && nhwc) dcn2_fwd_tile_kernel<T, IB, JB, WM, WN, WK, true, true><<<p.tiles, NT, 0, s>>>(p);
+    else if (p.mask) dcn2_fwd_tile_kernel<T, IB, JB, WM, WN, WK, true, false><<<p.tiles, NT, 0, s>>>(p);
+    else if (nhwc) dcn2_fwd_tile_kernel<T, IB, JB, WM, WN, WK, false, true><<<p.tiles, NT, 0, s>>>(p);
+    else dcn2_fwd_tile_kernel<T, IB, JB, WM, WN, WK, false, false><<<p.tiles, NT, 0, s>>>(p);
     return hipGetLastError();
 }
 
-hipError_t launch_forward_f32(const Geo &g, const void *xt, const void *wp, const void *tab,
+template <typename T>
+static hipError_t forward_tiles(const Geo &g, const void *xt, const void *wp, const void *tab,
                               const void *offset, const void *mask, const void *bias, void *out,
                               hipStream_t s) {
-    if (g.B == 0) return hipSuccess;
-    F32FwdParams p;
-    p.wp = (const float *)wp;
+    TileParams p;
+    p.wp = wp;
     p.tab = (const int4 *)tab;
-    p.bias = (const float *)bias;
+    p.bias = bias;
     p.H = g.H;
     p.W = g.W;
     p.Cout = g.Cout;
@@ -368,7 +387,7 @@ hipError_t launch_forward_f32(const Geo &g, const void *xt, const void *wp, cons
     p.msk_logit = mask ? g.msk_logit : 0;
     // Images per launch: the input, offset and mask bytes and the pixel count of
     // a launch stay in 32 bits (one image always fits, see make_geo).
-    const long long img = std::max({(long long)g.H * g.W * g.cs * 4, g.off_bs * 4, g.msk_bs * 4, 2LL * g.N});
+    const long long img = std::max({(long long)g.H * g.W * g.cs * g.esz, g.off_bs * g.esz, g.msk_bs * g.esz, 2LL * g.N});
     const int nimg = (int)std::max(1LL, std::min((long long)g.B, 0xffff0000LL / img));
     // One launch over all rows and chunks, or one per weight group over the
     // group's rows (a multiple of 128) and chunks.
@@ -378,45 +397,53 @@ hipError_t launch_forward_f32(const Geo &g, const void *xt, const void *wp, cons
     for (int b = 0; b < g.B; b += nimg) {
         const int nb = std::min(nimg, g.B - b);
         p.total = nb * g.N;
-        p.x_bytes = (uint32_t)((long long)nb * g.H * g.W * g.cs * 4);
-        p.xt = (const float *)xt + (size_t)b * g.H * g.W * g.cs;
-        p.offset = (const float *)offset + (size_t)b * g.off_bs;
-        p.mask = mask ? (const float *)mask + (size_t)b * g.msk_bs : nullptr;
-        p.out = (float *)out + (size_t)b * g.Cout * g.N;
+        p.x_bytes = (uint32_t)((long long)nb * g.H * g.W * g.cs * g.esz);
+        p.xt = (const T *)xt + (size_t)b * g.H * g.W * g.cs;
+        p.offset = (const T *)offset + (size_t)b * g.off_bs;
+        p.mask = mask ? (const T *)mask + (size_t)b * g.msk_bs : nullptr;
+        p.out = (T *)out + (size_t)b * g.Cout * g.N;
         for (int w = 0; w < groups; ++w) {
             p.cb = w * p.cpw;
             p.m_base = w * rows;
             p.m_end = p.m_base + rows;
-            // Tile rule: the largest tile that keeps the CUs busy.  Measured (us at
-            // Cout, K, pixels; tiles in brackets):
-            //   256x64, 8 waves: a pixel is sampled once for 256 rows.  64.7 against
-            //     71.1 for 128x64 at 256, 64, 100352 [1568]; 48.7 against 51.7 at
-            //     2048, 512, 1568 [200]; 79.9 against 57.7 at 256, 1024, 6272 [98].
-            //   128x64: with K split over 8 waves when tiles are few and K long:
-            //     49.9 against 57.7 at 256, 1024, 6272 [196] and 59.9 against 66.3
-            //     at 128, 1152, 12544 [196]; 98.8 against 71.1 at K = 64 [3136].
-            //   32 pixels, K split: 9.6 (64x32) against 11.6 (128x32) and 18.7
-            //     (128x64) at 32, 288, 1024.
+            // Tile rule, measured in us (rows, K, pixels; tile: rows x pixels, all with
+            // 8 waves and one or two workgroups to a CU unless noted):
+            //   64x32, K over 4 groups of waves, while one workgroup to a CU does: fp16
+            //     13.5 against 16.2 (128x32) at 128, 1152, 4096; 32 against 39 at 512,
+            //     4608, 1024; fp32 9.6 against 11.6 at 32, 288, 1024.  Past that 38
+            //     against 24 at 256, 2304, 2100.
+            //   128x32, K over 2, while two and a half do: fp16 33 against 43 (256x64)
+            //     at 256, 2304, 8192, but 60 against 45 at 16384; fp32 50.7 against 79.9
+            //     at 256, 1024, 6272.
+            //   256x64 (a pixel is sampled once for 256 rows): fp32 64.7 against 71.1
+            //     for 128x64 at 256, 64, 100352; 48.7 against 51.7 at 2048, 512, 1568.
+            //   128x64 and 64x64 (4 waves): the rest, whose rows 256x64 would pad.
             auto tiles = [&](int bm, int bn) { return (long long)ceil_div(rows, bm) * ceil_div(p.total, bn); };
             hipError_t e;
-            if (rows > 128 && tiles(256, 64) >= 192)
-                e = launch_fwd_f32_t<1, 2, 8, 1, 1>(p, rows, g.out_nhwc, s);
-            else if (rows > 64 && (tiles(128, 64) >= 512 || (tiles(128, 64) >= 160 && p.nch < 8)))
-                e = launch_fwd_f32_t<1, 2, 4, 1, 1>(p, rows, g.out_nhwc, s);
-            else if (rows > 64 && tiles(128, 64) >= 160)
-                e = launch_fwd_f32_t<1, 2, 4, 1, 2>(p, rows, g.out_nhwc, s);
-            else if (rows > 64 && tiles(128, 32) >= 128)
-                e = launch_fwd_f32_t<1, 1, 4, 1, 2>(p, rows, g.out_nhwc, s);
-            else if (rows <= 64 && tiles(64, 64) >= 256)
-                e = launch_fwd_f32_t<1, 1, 2, 2, 1>(p, rows, g.out_nhwc, s);
-            else if (rows > 32)
-                e = launch_fwd_f32_t<1, 1, 2, 1, 4>(p, rows, g.out_nhwc, s);
+            if (tiles(64, 32) <= 256)
+                e = launch_tile<T, 1, 1, 2, 1, 4>(p, rows, g.out_nhwc, s);
+            else if (rows > 64 && tiles(128, 32) <= 640)
+                e = launch_tile<T, 1, 1, 4, 1, 2>(p, rows, g.out_nhwc, s);
+            else if (rows > 128)
+                e = launch_tile<T, 1, 2, 8, 1, 1>(p, rows, g.out_nhwc, s);
+            else if (rows > 64)
+                e = launch_tile<T, 1, 2, 4, 1, 1>(p, rows, g.out_nhwc, s);
             else
-                e = launch_fwd_f32_t<1, 1, 1, 1, 4>(p, rows, g.out_nhwc, s);
+                e = launch_tile<T, 1, 1, 2, 2, 1>(p, rows, g.out_nhwc, s);
             if (e != hipSuccess) return e;
         }
     }
     return hipSuccess;
+}
+
+hipError_t launch_forward_tiles(const Geo &g, const void *xt, const void *wp, const void *tab,
+                                const void *offset, const void *mask, const void *bias, void *out,
+                                hipStream_t s) {
+    switch (g.dtype) {
+    case DCN2_F16: return forward_tiles<f16>(g, xt, wp, tab, offset, mask, bias, out, s);
+    case DCN2_BF16: return forward_tiles<bf16>(g, xt, wp, tab, offset, mask, bias, out, s);
+    default: return forward_tiles<float>(g, xt, wp, tab, offset, mask, bias, out, s);
+    }
 }
 
 }  // namespace dcn2

@@ -111,10 +111,11 @@ hipError_t launch_forward(const Geo &g, const void *xt, const void *wp, const vo
                           const void *offset, const void *mask, const void *bias, void *out,
                           hipStream_t s);
 
-// dcn2_forward_f32.hip: the fp32 forward (launch_forward calls it).
-hipError_t launch_forward_f32(const Geo &g, const void *xt, const void *wp, const void *tab,
-                              const void *offset, const void *mask, const void *bias, void *out,
-                              hipStream_t s);
+// dcn2_forward_tiles.hip: small tiles over the batch's pixels; every fp32 forward
+// and the 2-byte ones of few tiles (launch_forward calls it).
+hipError_t launch_forward_tiles(const Geo &g, const void *xt, const void *wp, const void *tab,
+                                const void *offset, const void *mask, const void *bias, void *out,
+                                hipStream_t s);
 
 // dcn2_forward_rw.hip: the resident-weight forward and its eligibility (f16,
 // one deformable group of <= 64 channels, 3x3, 128 < Cout <= 256, no weight

@@ -17,13 +17,13 @@ SHAPES = [
     (3, 40, 65, 67, 257, 1, 1, 1, 1, False),    # 256x64, one row past a tile
     (70, 33, 7, 7, 2048, 1, 1, 1, 1, False),    # 256x64, 49-pixel images
     (2, 64, 129, 131, 65, 1, 1, 1, 1, False),   # 128x64, many tiles
-    (3, 160, 61, 60, 100, 1, 1, 1, 1, True),    # 128x64, short K
+    (3, 160, 61, 60, 100, 1, 1, 1, 1, True),    # 128x64, 5 chunks
     (3, 96, 61, 60, 128, 3, 1, 1, 1, False),    # 128x64, K split
     (5, 32, 31, 29, 127, 3, 1, 1, 1, True),     # 128x32, K split, 9 chunks
     (9, 16, 45, 43, 33, 3, 1, 2, 1, False),     # 64x64
     (3, 70, 9, 5, 34, 3, 2, 1, 1, True),        # 64x32, K split
-    (1, 3, 4, 3, 1, 1, 1, 1, 1, False),         # 32x32, K split, one chunk
-    (2, 16, 13, 11, 32, 5, 1, 4, 1, True),      # 32x32, 100 chunks
+    (1, 3, 4, 3, 1, 1, 1, 1, 1, False),         # 64x32, K split, one chunk
+    (2, 16, 13, 11, 32, 5, 1, 4, 1, True),      # 64x32, 100 chunks
     (2, 64, 33, 35, 256, 3, 1, 1, 2, False),    # weight groups, one launch each
 ]
 
