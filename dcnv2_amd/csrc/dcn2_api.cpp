@@ -220,6 +220,8 @@ BwdWorkspace bwd_workspace(const Geo &g0) {
         w.ring = o;
         o += ring_bytes;
     }
+    w.gop = o;
+    if (go_padded(g)) o += align256((size_t)g.B * g.Cout * go_pitch(g) * g.esz);
     w.total = o;
     return w;
 }
@@ -349,7 +351,9 @@ static int backward_impl(const Geo &g0, const void *input, const void *weight, c
         clr.n[3] = ws.rec > ws.csum && gs.B > 0 ? (size_t)gs.B * g.G * g.KK * g.N * 4 : 0;
         prof_begin(DCN2_STAGE_BWD_PACK, s);
         if ((rc = check_launch(launch_pack(gs, g.xt_direct ? nullptr : in_s, (void *)xt,
-                                           first ? weight : nullptr, wt, tab, true, s, &clr),
+                                           first ? weight : nullptr, wt, tab, true, s, &clr,
+                                           gs.B > 0 && go_padded(gs) ? at(grad_output, go_img) : nullptr,
+                                           base + ws.gop),
                                "pack")))
             return rc;
         prof_end(DCN2_STAGE_BWD_PACK, s);
@@ -362,7 +366,8 @@ static int backward_impl(const Geo &g0, const void *input, const void *weight, c
                                  base + ws.cgm, base + ws.rsc, (float *)(base + ws.csum), base + ws.rec,
                                  (int *)(base + ws.bcnt),
                                  (int *)(base + ws.bstart), (int *)(base + ws.bcur),
-                                 (int *)(base + ws.sidx), (float *)(base + ws.ring), last, s),
+                                 (int *)(base + ws.sidx), (float *)(base + ws.ring), base + ws.gop,
+                                 last, s),
                  "backward")))
             return rc;
         b0 += gs.B;

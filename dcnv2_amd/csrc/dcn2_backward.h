@@ -26,6 +26,7 @@ struct BwdParams {
     // (NCHW, N % 8 == 0) or channels of a pixel (channels-last, Cout % 8 == 0),
     // from a 16-byte aligned base
     int go_vec;
+    int go_n;  // elements between rows of NCHW grad_output: N, or more in a padded copy (zeros past N)
     // grad_input gather: cell-tile buckets (see dcn2_gi_gather_kernel).  The
     // rows of all buckets are packed back to back, bucket k owning rows
     // [bstart[k], bstart[k+1]); there are at most B*G*KK*N of them (one per

@@ -101,7 +101,7 @@ __device__ __forceinline__ float row_unscale(unsigned code) { return __int_as_fl
 
 // Buffer offset at or past one image's gO bytes (a load there reads 0); the
 // kernels that read gO through it require Cout*N*sizeof(T) <= kGoOutOfRange.
-constexpr int kGoOutOfRange = 0x7ffffff0;
+constexpr int kGoOutOfRange = (int)kGoMaxBytes;
 
 // Cell tiles of the grad_input gather: a sample with floor corner (y0, x0)
 // belongs to cell (y0+1, x0+1) of the (H+1) x (W+1) cell grid, and cells are
@@ -487,7 +487,7 @@ __global__ __launch_bounds__(512) void dcn2_colgrad_kernel(const BwdParams p) {
     const T *__restrict__ xt = (const T *)p.xt + (size_t)b * p.H * p.W * cs;
     const T *__restrict__ offs = (const T *)p.offset + (size_t)b * p.off_bs;
     const T *__restrict__ msk = p.mask ? (const T *)p.mask + (size_t)b * p.msk_bs : nullptr;
-    const T *__restrict__ go = (const T *)p.gout + (size_t)b * p.Cout * N;
+    const T *__restrict__ go = (const T *)p.gout + (size_t)b * p.Cout * p.go_n;
     const T *__restrict__ wt = (const T *)p.wt;
     T *__restrict__ goff = (T *)p.goff + (size_t)b * p.off_bs;
     T *__restrict__ gmask = p.gmask ? (T *)p.gmask + (size_t)b * p.msk_bs : nullptr;
@@ -515,7 +515,7 @@ __global__ __launch_bounds__(512) void dcn2_colgrad_kernel(const BwdParams p) {
 #pragma unroll
                 for (int e = 0; e < KPL; ++e) {
                     const int m = m0s + e;
-                    const T v = (n < N && m < p.Cout) ? go[(size_t)m * N + n] : (T)0.0f;
+                    const T v = (n < N && m < p.Cout) ? go[(size_t)m * p.go_n + n] : (T)0.0f;
                     FragSet<T, KPL>::set(gfr[s], e, v);
                 }
             }
@@ -535,15 +535,15 @@ __global__ __launch_bounds__(512) void dcn2_colgrad_kernel(const BwdParams p) {
     // distinct banks.  Rows past Cout and pixels past N read 0 (buffer range).
     constexpr int GQ = (sizeof(T) == 2 ? MCH * (BN / 8) : 512) / 512;  // 16-byte pieces per thread
     const bool go_stage = ONEM && sizeof(T) == 2 && p.go_vec && !p.go_nhwc &&
-                          (size_t)p.Cout * N * sizeof(T) <= (size_t)kGoOutOfRange;
+                          (size_t)p.Cout * p.go_n * sizeof(T) <= (size_t)kGoOutOfRange;
     uint4 gst[GQ];
     auto go_stage_issue = [&]() __attribute__((always_inline)) {
         const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<T *>(go), (short)0, (int)((size_t)p.Cout * N * sizeof(T)), 0x00020000);
+            const_cast<T *>(go), (short)0, (int)((size_t)p.Cout * p.go_n * sizeof(T)), 0x00020000);
 #pragma unroll
         for (int q = 0; q < GQ; ++q) {
             const int idx = tid + 512 * q, m = idx / (BN / 8), n = n0 + (idx % (BN / 8)) * 8;
-            const int off = (int)(((unsigned)m * (unsigned)N + (unsigned)n) * sizeof(T));
+            const int off = (int)(((unsigned)m * (unsigned)p.go_n + (unsigned)n) * sizeof(T));
             gst[q] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
                                                    rs, n < N ? off : kGoOutOfRange, 0, 0));
         }
@@ -1200,7 +1200,7 @@ __global__ __launch_bounds__(512) void dcn2_gradw_line_kernel(const BwdParams p)
     };
 
     // one image's gO (the host keeps it within kGoOutOfRange bytes)
-    const uint32_t go_bytes = (uint32_t)((size_t)p.Cout * N * sizeof(T));
+    const uint32_t go_bytes = (uint32_t)((size_t)p.Cout * p.go_n * sizeof(T));
     const int lg = lane >> 3, lc = lane & 7;
     uint4 ga[NKS];  // gO of the next tile, loaded by line; stored to LDS at the end of the step
     // NCHW: lanes 8g..8g+7 read one 128-byte line (8 pixels of a row) per
@@ -1209,7 +1209,7 @@ __global__ __launch_bounds__(512) void dcn2_gradw_line_kernel(const BwdParams p)
     auto load_a_tile = [&](uint4 (&a)[NKS], int t) __attribute__((always_inline)) {
         const int b = t / p.tiles_per_img, n0 = (t - b * p.tiles_per_img) * BN;
         const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<T *>((const T *)p.gout + (size_t)b * p.Cout * N), (short)0, (int)go_bytes,
+            const_cast<T *>((const T *)p.gout + (size_t)b * p.Cout * p.go_n), (short)0, (int)go_bytes,
             0x00020000);
 #pragma unroll
         for (int j = 0; j < NKS; ++j) {
@@ -1223,7 +1223,7 @@ __global__ __launch_bounds__(512) void dcn2_gradw_line_kernel(const BwdParams p)
             } else {
                 const unsigned row = (unsigned)(rbase + 8 * (j & 3) + lg);
                 const int n = n0 + 64 * (j >> 2) + 8 * lc;
-                off = n < N ? (int)((row * (unsigned)N + (unsigned)n) * sizeof(T)) : kGoOutOfRange;
+                off = n < N ? (int)((row * (unsigned)p.go_n + (unsigned)n) * sizeof(T)) : kGoOutOfRange;
             }
             a[j] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0));
         }
@@ -1489,10 +1489,10 @@ void dcn2_bwd_fused_kernel(const BwdParams p) {
         const int b = t / tpi;
         return TileId{b, (t - b * tpi) * BN};
     };
-    const uint32_t go_bytes = (uint32_t)((size_t)p.Cout * N * sizeof(T));
+    const uint32_t go_bytes = (uint32_t)((size_t)p.Cout * p.go_n * sizeof(T));
     auto go_rsrc = [&](const TileId &id) __attribute__((always_inline)) {
         return __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<T *>((const T *)p.gout + (size_t)id.b * p.Cout * N), (short)0, (int)go_bytes,
+            const_cast<T *>((const T *)p.gout + (size_t)id.b * p.Cout * p.go_n), (short)0, (int)go_bytes,
             0x00020000);
     };
     // Load q of the wave's rows: NCHW rows RPW wave + 8q + l/8, 8 pieces of 8
@@ -1513,7 +1513,7 @@ void dcn2_bwd_fused_kernel(const BwdParams p) {
         } else {
             const int r = RPW * wave + 8 * q + (lane >> 3);
             const int n = 8 * ((lane & 7) ^ fused_swz(r));
-            go_lo[q] = (r * N + n) * (int)sizeof(T);
+            go_lo[q] = (r * p.go_n + n) * (int)sizeof(T);
             go_px[q] = n;
             go_ok[q] = r < p.Cout;
         }
@@ -3113,7 +3113,7 @@ static hipError_t backward_t(const Geo &g, const BwdParams &p0, void *grad_input
                else DCN2_GRADW(KERN, 4, false __VA_ARGS__); }                                    \
     } while (0)
             if constexpr (sizeof(T) == 2) {
-                if (p.go_vec && (long long)g.Cout * g.N * (long long)sizeof(T) <= kGoOutOfRange) {
+                if (p.go_vec && (long long)g.Cout * p.go_n * (long long)sizeof(T) <= kGoOutOfRange) {
                     if (p.go_nhwc) DCN2_GRADW_MB(dcn2_gradw_line_kernel, , true);
                     else DCN2_GRADW_MB(dcn2_gradw_line_kernel, , false);
                     line = true;
@@ -3229,14 +3229,15 @@ hipError_t launch_backward(const Geo &g, const void *xt, const void *wt, const v
                            void *grad_offset, void *grad_mask, void *grad_weight, void *grad_bias,
                            float *gi_acc, float *gw_acc, float *gb_acc, void *cgm, void *rsc,
                            float *csum, void *rec, int *bcnt, int *bstart, int *bcur, int *sidx,
-                           float *ring, bool last, hipStream_t s) {
+                           float *ring, const void *gop, bool last, hipStream_t s) {
     BwdParams p;
     p.xt = xt;
     p.wt = wt;
     p.tab = tab;
     p.offset = offset;
     p.mask = mask;
-    p.gout = grad_out;
+    const bool padded = go_padded(g);  // (copied by the pack launch)
+    p.gout = padded ? gop : grad_out;
     p.goff = grad_offset;
     p.gmask = grad_mask;
     p.off_bs = g.off_bs;
@@ -3266,8 +3267,9 @@ hipError_t launch_backward(const Geo &g, const void *xt, const void *wt, const v
     p.Mp = g.Mp;
     p.tiles_per_img = ceil_div(g.N, 128);
     p.splits = 1;
-    p.go_nhwc = g.out_nhwc;
-    p.go_vec = (g.out_nhwc ? g.Cout % 8 == 0 : g.N % 8 == 0) && (((uintptr_t)grad_out & 15) == 0);
+    p.go_nhwc = padded ? 0 : g.out_nhwc;
+    p.go_n = padded ? go_pitch(g) : g.N;
+    p.go_vec = padded || ((g.out_nhwc ? g.Cout % 8 == 0 : g.N % 8 == 0) && (((uintptr_t)grad_out & 15) == 0));
     const GatherGeo gg = gather_geometry(g);
     p.cgm = cgm;
     p.rsc = (unsigned char *)rsc;

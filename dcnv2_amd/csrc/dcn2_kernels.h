@@ -66,7 +66,7 @@ struct FwdWorkspace {
 FwdWorkspace fwd_workspace(const Geo &g);
 
 struct BwdWorkspace {
-    size_t xt, wt, tab, gi_acc, gw_acc, gb_acc, cgm, rsc, csum, rec, bcnt, bstart, bcur, sidx, ring, total;
+    size_t xt, wt, tab, gi_acc, gw_acc, gb_acc, cgm, rsc, csum, rec, bcnt, bstart, bcur, sidx, ring, gop, total;
 };
 // Carves the backward workspace of one slice of g.Bs images.
 // Border-ring pixels of one grad_input gather window (4 x the cell tile side).
@@ -103,8 +103,24 @@ struct ClearList {
     float *p[kClearBufs];
     size_t n[kClearBufs];
 };
+// With `go`, it also copies the 2-byte grad_output of g.B images to `gop`, NCHW with
+// rows of go_pitch(g) elements, zeros past the N pixels (see go_padded).
 hipError_t launch_pack(const Geo &g, const void *input, void *xt, const void *weight, void *wp,
-                       void *tab, bool transpose, hipStream_t s, const ClearList *clear = nullptr);
+                       void *tab, bool transpose, hipStream_t s, const ClearList *clear = nullptr,
+                       const void *go = nullptr, void *gop = nullptr);
+
+// grad_output whose rows 16-byte loads cannot read whatever its address (NCHW with
+// N % 8, or channels-last with Cout % 8): the backward reads a padded NCHW copy,
+// so that the kernels with 16-byte loads (the fused one among them) serve it too.
+// Measured at bf16 3x3, C 256 -> 256, 2 x 25 x 42 (N = 1050): 32 us in the fused
+// kernel against 118 + 47 in the two that read such rows by elements; the copy
+// adds 2 us to the pack launch.
+constexpr long long kGoMaxBytes = 0x7ffffff0;  // one image of grad_output those kernels address
+inline int go_pitch(const Geo &g) { return (g.N + 7) / 8 * 8; }
+inline bool go_padded(const Geo &g) {
+    return g.esz == 2 && (g.out_nhwc ? g.Cout : g.N) % 8 != 0 &&
+           (long long)g.Cout * go_pitch(g) * g.esz <= kGoMaxBytes;
+}
 
 // dcn2_forward.hip
 hipError_t launch_forward(const Geo &g, const void *xt, const void *wp, const void *tab,
@@ -133,7 +149,7 @@ hipError_t launch_backward(const Geo &g, const void *xt, const void *wt, const v
                            void *grad_offset, void *grad_mask, void *grad_weight, void *grad_bias,
                            float *gi_acc, float *gw_acc, float *gb_acc, void *cgm, void *rsc,
                            float *csum, void *rec, int *bcnt, int *bstart, int *bcur, int *sidx,
-                           float *ring, bool last, hipStream_t s);
+                           float *ring, const void *gop, bool last, hipStream_t s);
 // Whether the fused backward kernel may serve g (2-byte type, Cout <= 256),
 // and whether its column-gradient kernel (the fused one, or the fp32 one) needs
 // the corner-sum buffer (a group's channels shared by several workgroups).

@@ -12,7 +12,8 @@
 //
 // Blocks [0, nw) pack 256 16-byte pieces of the weight each; blocks
 // [nw, nw + nin) transpose 64 pixels x CT channels of the input each (CT*esz
-// = 128 bytes, one channel chunk of a pixel); the rest clear accumulators.
+// = 128 bytes, one channel chunk of a pixel); the rest clear accumulators and copy
+// grad_output rows that need padding (go_padded).
 // The halves are independent, so the (small, latency bound) weight packing,
 // dispatched first, overlaps the (bandwidth bound) input transpose.
 #include "dcn2_common.h"
@@ -37,6 +38,10 @@ struct PackParams {
     float4 *clr[kClearBufs];       // buffers to zero, 16-byte pieces each
     long clr_n4[kClearBufs];
     int clr_blk[kClearBufs + 1];   // first clearing block of each buffer (prefix sums)
+    const void *go;                // grad_output to copy in padded rows (go_padded), and its copy
+    void *gop;
+    int N, go_nhwc;
+    long ngo;                      // its 16-byte pieces, 256 to a block
 };
 constexpr int kClearPieces = 1024;  // 16-byte pieces zeroed per clearing block
 
@@ -199,6 +204,35 @@ __device__ __forceinline__ void pack_weight_block(const PackParams &p, int blk) 
     *reinterpret_cast<uint4 *>(dst + idx0) = __builtin_bit_cast(uint4, v);
 }
 
+// One 16-byte piece (8 pixels of one channel) of the padded NCHW copy of
+// grad_output per thread; consecutive threads take consecutive pieces of a row, or
+// (channels-last source) channels of 8 pixels, so that the reads are contiguous.
+template <typename T>
+__device__ __forceinline__ void pack_go_block(const PackParams &p, long blk) {
+    const long idx = blk * 256 + threadIdx.x;
+    if (idx >= p.ngo) return;
+    const int np = (p.N + 7) / 8;
+    int m, pc;
+    long b;
+    if (p.go_nhwc) {
+        m = (int)(idx % p.Cout);
+        pc = (int)(idx / p.Cout % np);
+        b = idx / p.Cout / np;
+    } else {
+        pc = (int)(idx % np);
+        m = (int)(idx / np % p.Cout);
+        b = idx / np / p.Cout;
+    }
+    const T *src = (const T *)p.go + b * (long)p.Cout * p.N;
+    T v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const int n = pc * 8 + e;
+        v[e] = n < p.N ? (p.go_nhwc ? src[(size_t)n * p.Cout + m] : src[(size_t)m * p.N + n]) : (T)0.0f;
+    }
+    *reinterpret_cast<uint4 *>((T *)p.gop + ((b * p.Cout + m) * np + pc) * 8) = __builtin_bit_cast(uint4, v);
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void pack_kernel(const PackParams p) {
     // weight blocks first: they are latency bound, so they are dispatched
@@ -211,6 +245,8 @@ __global__ __launch_bounds__(256) void pack_kernel(const PackParams p) {
             pack_input_block_nhwc<T>(p, blk - p.nw);
         else
             pack_input_block<T>(p, blk - p.nw);
+    } else if (blk - p.nw - p.nin >= p.clr_blk[kClearBufs]) {
+        if constexpr (sizeof(T) == 2) pack_go_block<T>(p, blk - p.nw - p.nin - p.clr_blk[kClearBufs]);
     } else {
         // zero kClearPieces 16-byte pieces of one of the clear-list buffers
         const int cb = blk - p.nin - p.nw;
@@ -225,7 +261,8 @@ __global__ __launch_bounds__(256) void pack_kernel(const PackParams p) {
 
 template <typename T>
 static hipError_t pack_t(const Geo &g, const void *input, void *xt, const void *weight,
-                         void *wp, void *tab, bool transpose, hipStream_t s, const ClearList *clear) {
+                         void *wp, void *tab, bool transpose, hipStream_t s, const ClearList *clear,
+                         const void *go, void *gop) {
     constexpr int E = 16 / sizeof(T), CT = 128 / sizeof(T);
     PackParams p;
     p.in = input;
@@ -271,18 +308,24 @@ static hipError_t pack_t(const Geo &g, const void *input, void *xt, const void *
         p.clr_n4[i] = (long)((n + 3) / 4);
         p.clr_blk[i + 1] = p.clr_blk[i] + (int)((p.clr_n4[i] + kClearPieces - 1) / kClearPieces);
     }
-    const long blocks = p.nin + nw + p.clr_blk[kClearBufs];
+    p.go = go;
+    p.gop = gop;
+    p.N = g.N;
+    p.go_nhwc = g.out_nhwc;
+    p.ngo = go ? (long)g.B * g.Cout * (go_pitch(g) / 8) : 0;
+    const long blocks = p.nin + nw + p.clr_blk[kClearBufs] + (p.ngo + 255) / 256;
     pack_kernel<T><<<(unsigned)blocks, 256, 0, s>>>(p);
     return hipGetLastError();
 }
 
 hipError_t launch_pack(const Geo &g, const void *input, void *xt, const void *weight, void *wp,
-                       void *tab, bool transpose, hipStream_t s, const ClearList *clear) {
+                       void *tab, bool transpose, hipStream_t s, const ClearList *clear,
+                       const void *go, void *gop) {
     if (g.B == 0) input = nullptr;  // weight packing only (also for an input read in place)
     switch (g.dtype) {
-    case DCN2_F16: return pack_t<f16>(g, input, xt, weight, wp, tab, transpose, s, clear);
-    case DCN2_BF16: return pack_t<bf16>(g, input, xt, weight, wp, tab, transpose, s, clear);
-    default: return pack_t<float>(g, input, xt, weight, wp, tab, transpose, s, clear);
+    case DCN2_F16: return pack_t<f16>(g, input, xt, weight, wp, tab, transpose, s, clear, go, gop);
+    case DCN2_BF16: return pack_t<bf16>(g, input, xt, weight, wp, tab, transpose, s, clear, go, gop);
+    default: return pack_t<float>(g, input, xt, weight, wp, tab, transpose, s, clear, go, gop);
     }
 }
 
