@@ -101,7 +101,22 @@ def _err(prefix: str) -> RuntimeError:
 
 
 def _ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
+
+
+def _launch(name, entry, device, *args):
+    """entry(*args, current stream of `device`) with `device` current; raises on a
+    status other than 0.  Small layers are bound by the host, so the device guard
+    is entered only when another GPU is current, and the stream handle is read
+    without building a Stream object (3 us of a call of 18)."""
+    index = device.index
+    if torch.cuda.current_device() == index:
+        rc = entry(*args, torch._C._cuda_getCurrentRawStream(index))
+    else:
+        with torch.cuda.device(index):
+            rc = entry(*args, torch._C._cuda_getCurrentRawStream(index))
+    if rc != 0:
+        raise _err(name)
 
 
 def _layout(t):
@@ -123,8 +138,8 @@ _input_layout = _layout
 
 def make_desc(input, weight, stride_h, stride_w, pad_h, pad_w, dilation_h, dilation_w,
               deformable_groups, input_layout=0, output_layout=0) -> Desc:
-    B, C, H, W = (int(v) for v in input.shape)
-    Cout, Cw, kh, kw = (int(v) for v in weight.shape)
+    B, C, H, W = input.shape
+    Cout, Cw, kh, kw = weight.shape
     # weight groups follow from weight.shape[1], as in torchvision's deform_conv2d
     return Desc(B, C, H, W, Cout, kh, kw, int(stride_h), int(stride_w), int(pad_h), int(pad_w),
                 int(dilation_h), int(dilation_w), int(deformable_groups), _DTYPES[input.dtype],
@@ -133,11 +148,15 @@ def make_desc(input, weight, stride_h, stride_w, pad_h, pad_w, dilation_h, dilat
 
 def _empty_out(shape, like, layout):
     """The output tensor: channels_last when `layout` is 1."""
-    fmt = torch.channels_last if layout else torch.contiguous_format
-    return torch.empty(shape, dtype=like.dtype, device=like.device, memory_format=fmt)
+    if layout:
+        return torch.empty(shape, dtype=like.dtype, device=like.device,
+                           memory_format=torch.channels_last)
+    return torch.empty(shape, dtype=like.dtype, device=like.device)
 
 
-def _validate(name, input, weight, mask, offset, bias, extra=()):
+def _check_tensors(name, input, weight, mask, offset, bias, extra):
+    """Raises for the first argument that is not a GPU tensor of input's device and
+    a supported dtype."""
     tensors = {"input": input, "weight": weight, "offset": offset}
     if mask is not None:
         tensors["mask"] = mask
@@ -158,6 +177,21 @@ def _validate(name, input, weight, mask, offset, bias, extra=()):
     if input.dtype not in _DTYPES:
         raise RuntimeError(f"{name}: unsupported dtype {input.dtype} "
                            "(float32, float16 and bfloat16 are supported)")
+
+
+def _validate(name, input, weight, mask, offset, bias, extra=()):
+    try:  # one pass over the usual case; anything else is named by _check_tensors
+        dev, dt = input.device, input.dtype
+        ok = dt in _DTYPES and input.is_cuda
+        for t in (weight, offset):
+            ok = ok and isinstance(t, torch.Tensor) and t.device == dev and t.dtype == dt
+        for t in (mask, bias, *(t for _, t in extra)):
+            ok = ok and (t is None or (t.device == dev and t.dtype == dt))
+        ok = ok and all(t is not None for _, t in extra)
+    except AttributeError:
+        ok = False
+    if not ok:
+        _check_tensors(name, input, weight, mask, offset, bias, extra)
     if input.dim() != 4 or weight.dim() != 4 or offset.dim() != 4:
         raise RuntimeError(f"{name}: input, weight and offset must be 4-D")
     # reference com.cu:760-761 requires weight.shape[1] == C; torchvision's weight
@@ -186,10 +220,8 @@ def _geometry(name, desc, input, mask, offset):
 
 def _workspace(nbytes, device):
     # 256 extra bytes so the start can be aligned to 256 whatever the allocator returns
-    buf = torch.empty(int(nbytes) + 256, dtype=torch.uint8, device=device)
-    addr = buf.data_ptr()
-    aligned = (addr + 255) & ~255
-    return buf, aligned, int(nbytes)
+    buf = torch.empty(nbytes + 256, dtype=torch.uint8, device=device)
+    return buf, (buf.data_ptr() + 255) & ~255, nbytes
 
 
 def dcn_v2_forward(input, weight, mask, offset, bias, stride_h, stride_w, pad_h, pad_w,
@@ -207,15 +239,10 @@ def dcn_v2_forward(input, weight, mask, offset, bias, stride_h, stride_w, pad_h,
     ho, wo = _geometry(name, desc, input, mask, offset)
     L = lib()
     out = _empty_out((desc.batch, desc.out_channels, ho, wo), input, layout)
-    with torch.cuda.device(input.device):
-        ws_buf, ws, ws_bytes = _workspace(L.dcn2_forward_workspace_bytes(ctypes.byref(desc)),
-                                          input.device)
-        stream = torch.cuda.current_stream(input.device).cuda_stream
-        rc = L.dcn2_forward(ctypes.byref(desc), _ptr(input), _ptr(weight), _ptr(mask),
-                            _ptr(offset), _ptr(bias), _ptr(out), ctypes.c_void_p(ws), ws_bytes,
-                            ctypes.c_void_p(stream))
-    if rc != 0:
-        raise _err(name)
+    ref = ctypes.byref(desc)
+    ws_buf, ws, ws_bytes = _workspace(L.dcn2_forward_workspace_bytes(ref), input.device)
+    _launch(name, L.dcn2_forward, input.device, ref, _ptr(input), _ptr(weight), _ptr(mask),
+            _ptr(offset), _ptr(bias), _ptr(out), ws, ws_bytes)
     del ws_buf  # returned to torch's caching allocator in stream order
     return out
 
@@ -245,17 +272,11 @@ def dcn_v2_backward(input, weight, mask, offset, bias, grad_output, stride_h, st
     grad_weight = torch.empty_like(weight)
     grad_bias = torch.empty((desc.out_channels,), dtype=input.dtype, device=input.device) \
         if bias is not None else None
-    with torch.cuda.device(input.device):
-        ws_buf, ws, ws_bytes = _workspace(L.dcn2_backward_workspace_bytes(ctypes.byref(desc)),
-                                          input.device)
-        stream = torch.cuda.current_stream(input.device).cuda_stream
-        rc = L.dcn2_backward(ctypes.byref(desc), _ptr(input), _ptr(weight), _ptr(mask),
-                             _ptr(offset), _ptr(grad_output), _ptr(grad_input),
-                             _ptr(grad_offset), _ptr(grad_mask), _ptr(grad_weight),
-                             _ptr(grad_bias), ctypes.c_void_p(ws), ws_bytes,
-                             ctypes.c_void_p(stream))
-    if rc != 0:
-        raise _err(name)
+    ref = ctypes.byref(desc)
+    ws_buf, ws, ws_bytes = _workspace(L.dcn2_backward_workspace_bytes(ref), input.device)
+    _launch(name, L.dcn2_backward, input.device, ref, _ptr(input), _ptr(weight), _ptr(mask),
+            _ptr(offset), _ptr(grad_output), _ptr(grad_input), _ptr(grad_offset), _ptr(grad_mask),
+            _ptr(grad_weight), _ptr(grad_bias), ws, ws_bytes)
     del ws_buf
     return [grad_input, grad_offset, grad_mask, grad_weight, grad_bias]
 
@@ -288,15 +309,10 @@ def dcn_v2_forward_om(input, weight, om, bias, stride_h, stride_w, pad_h, pad_w,
     ho, wo = _om_geometry(name, desc, om)
     L = lib()
     out = _empty_out((desc.batch, desc.out_channels, ho, wo), input, layout)
-    with torch.cuda.device(input.device):
-        ws_buf, ws, ws_bytes = _workspace(L.dcn2_forward_workspace_bytes(ctypes.byref(desc)),
-                                          input.device)
-        stream = torch.cuda.current_stream(input.device).cuda_stream
-        rc = L.dcn2_forward_om(ctypes.byref(desc), _ptr(input), _ptr(weight), _ptr(om),
-                               _ptr(bias), _ptr(out), ctypes.c_void_p(ws), ws_bytes,
-                               ctypes.c_void_p(stream))
-    if rc != 0:
-        raise _err(name)
+    ref = ctypes.byref(desc)
+    ws_buf, ws, ws_bytes = _workspace(L.dcn2_forward_workspace_bytes(ref), input.device)
+    _launch(name, L.dcn2_forward_om, input.device, ref, _ptr(input), _ptr(weight), _ptr(om),
+            _ptr(bias), _ptr(out), ws, ws_bytes)
     del ws_buf
     return out
 
@@ -323,16 +339,11 @@ def dcn_v2_backward_om(input, weight, om, bias, grad_output, stride_h, stride_w,
     grad_weight = torch.empty_like(weight)
     grad_bias = torch.empty((desc.out_channels,), dtype=input.dtype, device=input.device) \
         if bias is not None else None
-    with torch.cuda.device(input.device):
-        ws_buf, ws, ws_bytes = _workspace(L.dcn2_backward_workspace_bytes(ctypes.byref(desc)),
-                                          input.device)
-        stream = torch.cuda.current_stream(input.device).cuda_stream
-        rc = L.dcn2_backward_om(ctypes.byref(desc), _ptr(input), _ptr(weight), _ptr(om),
-                                _ptr(grad_output), _ptr(grad_input), _ptr(grad_om),
-                                _ptr(grad_weight), _ptr(grad_bias), ctypes.c_void_p(ws),
-                                ws_bytes, ctypes.c_void_p(stream))
-    if rc != 0:
-        raise _err(name)
+    ref = ctypes.byref(desc)
+    ws_buf, ws, ws_bytes = _workspace(L.dcn2_backward_workspace_bytes(ref), input.device)
+    _launch(name, L.dcn2_backward_om, input.device, ref, _ptr(input), _ptr(weight), _ptr(om),
+            _ptr(grad_output), _ptr(grad_input), _ptr(grad_om), _ptr(grad_weight), _ptr(grad_bias),
+            ws, ws_bytes)
     del ws_buf
     return [grad_input, grad_om, grad_weight, grad_bias]
 
