@@ -14,8 +14,8 @@
 // per chunk there.  Here every (pixel tile, channel tile) is its own 4-wave
 // workgroup, several to a CU, and pixels are numbered through the batch.  Measured
 // (us, old -> new; 3.3-3.7 GFLOP each, 21-24 us at the 154 TFLOP/s of a large
-// product): 203 -> 62 at Cout 256, K 64, 32 x 56 x 56; 392 -> 60 at 256, 1024, 32 x
-// 14 x 14; 1558 -> 62 at 2048, 512, 32 x 7 x 7; 142 -> 62 at 128, 1152, 4 x 56 x 56.
+// product): 203 -> 54 at Cout 256, K 64, 32 x 56 x 56; 392 -> 50 at 256, 1024, 32 x
+// 14 x 14; 1558 -> 60 at 2048, 512, 32 x 7 x 7; 142 -> 58 at 128, 1152, 4 x 56 x 56.
 #include <algorithm>
 #include <cstddef>
 #include <type_traits>
@@ -49,11 +49,11 @@ struct CgF32Params {
 
 constexpr int kCgM = 32;  // rows of grad_output per step
 
-// JB x (CB == 2 ? 2 : 4) blocks of 32 pixels, CB blocks of 32 channels.  GN:
+// 4 / CB blocks of 32 pixels x CB blocks of 32 channels, one per wave.  GN:
 // grad_output is channels-last.
-template <int JB, int CB, bool GN>
+template <int CB, bool GN>
 __global__ __launch_bounds__(256) void dcn2_colgrad_f32_kernel(const CgF32Params c) {
-    constexpr int NW = 4 / CB, NT = 32 * JB * NW, CT = 32 * CB;
+    constexpr int NT = 32 * (4 / CB), CT = 32 * CB;
     constexpr int LDG = NT + 8;  // floats per staged row: the two lane halves read rows 4 apart, on other banks
     constexpr int LDC = CT + 4;
     constexpr int NG = NT * kCgM / 256;
@@ -72,7 +72,7 @@ __global__ __launch_bounds__(256) void dcn2_colgrad_f32_kernel(const CgF32Params
     const BwdParams &p = c.p;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int cb = wave % CB, nb = wave / CB * JB;
+    const int cb = wave % CB, nb = wave / CB;
     // the channel tiles of one pixel tile are neighbours, on one XCD: they read the same grad_output
     const int t = xcd_remap(blockIdx.x, c.ptiles * c.ctiles);
     const int ct = t % c.ctiles, n0 = t / c.ctiles * NT;
@@ -164,11 +164,9 @@ __global__ __launch_bounds__(256) void dcn2_colgrad_f32_kernel(const CgF32Params
 
     // Even and odd steps sum apart: half as long a chain of fp32 additions (the
     // error of a 2048-row sum against 64 bits: 8.2e-7 in one chain, 5.8e-7 in two).
-    f32x16 acc[2][JB];
+    f32x16 acc[2];
 #pragma unroll
-    for (int j = 0; j < JB; ++j)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[0][j][r] = acc[1][j][r] = 0.0f;
+    for (int r = 0; r < 16; ++r) acc[0][r] = acc[1][r] = 0.0f;
     store_g(0);
     __syncthreads();
     auto step = [&](auto set_c, int m0) __attribute__((always_inline)) {
@@ -182,10 +180,8 @@ __global__ __launch_bounds__(256) void dcn2_colgrad_f32_kernel(const CgF32Params
         for (int k = 0; k < kCgM / 8; ++k)
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-#pragma unroll
-                for (int j = 0; j < JB; ++j)
-                    acc[S][j] = Mma<float>::mma(
-                        a[S][k][e], sG[S][8 * k + 4 * (lane >> 5) + e][(nb + j) * 32 + (lane & 31)], acc[S][j]);
+                acc[S] = Mma<float>::mma(a[S][k][e], sG[S][8 * k + 4 * (lane >> 5) + e][nb * 32 + (lane & 31)],
+                                         acc[S]);
         if (more) store_g(S ^ 1);
         __syncthreads();
     };
@@ -197,14 +193,11 @@ __global__ __launch_bounds__(256) void dcn2_colgrad_f32_kernel(const CgF32Params
     if (m0 < mend) step(std::integral_constant<int, 0>{}, m0);
 
     // acc[4*rq + e] of lane l: channel 8*rq + 4*(l/32) + e of pixel l%32
+    const f32x16 cg = acc[0] + acc[1];
 #pragma unroll
-    for (int j = 0; j < JB; ++j) {
-        const f32x16 v = acc[0][j] + acc[1][j];
-#pragma unroll
-        for (int rq = 0; rq < 4; ++rq)
-            *reinterpret_cast<f32x4 *>(&sC[(nb + j) * 32 + (lane & 31)][cb * 32 + 8 * rq + 4 * (lane >> 5)]) =
-                f32x4{v[4 * rq], v[4 * rq + 1], v[4 * rq + 2], v[4 * rq + 3]};
-    }
+    for (int rq = 0; rq < 4; ++rq)
+        *reinterpret_cast<f32x4 *>(&sC[nb * 32 + (lane & 31)][cb * 32 + 8 * rq + 4 * (lane >> 5)]) =
+            f32x4{cg[4 * rq], cg[4 * rq + 1], cg[4 * rq + 2], cg[4 * rq + 3]};
     __syncthreads();
 
     // Consumers: LP lanes x 4 channels per pixel.
@@ -491,11 +484,11 @@ static int f32_images(const Geo &g) {
     return (int)std::max(1LL, std::min((long long)g.B, 0xffff0000LL / img));
 }
 
-template <int JB, int CB>
+template <int CB>
 static void colgrad_f32_launch(CgF32Params &c, hipStream_t s) {
-    c.ptiles = ceil_div(c.total, 32 * JB * (4 / CB));
-    if (c.p.go_nhwc) dcn2_colgrad_f32_kernel<JB, CB, true><<<c.ptiles * c.ctiles, 256, 0, s>>>(c);
-    else dcn2_colgrad_f32_kernel<JB, CB, false><<<c.ptiles * c.ctiles, 256, 0, s>>>(c);
+    c.ptiles = ceil_div(c.total, 32 * (4 / CB));
+    if (c.p.go_nhwc) dcn2_colgrad_f32_kernel<CB, true><<<c.ptiles * c.ctiles, 256, 0, s>>>(c);
+    else dcn2_colgrad_f32_kernel<CB, false><<<c.ptiles * c.ctiles, 256, 0, s>>>(c);
 }
 
 hipError_t launch_colgrad_f32(const Geo &g, const BwdParams &p, hipStream_t s) {
@@ -511,12 +504,11 @@ hipError_t launch_colgrad_f32(const Geo &g, const BwdParams &p, hipStream_t s) {
         c.b0 = b;
         c.total = nb * g.N;
         c.x_bytes = (uint32_t)((long long)nb * g.H * g.W * g.cs * 4);
-        // 128-pixel tiles (the weight read once for twice the pixels) where three
-        // to a CU remain, else 64: at 2048, 512, 32 x 7 x 7 the 128-pixel tiles
-        // would be 104 workgroups, the 64-pixel ones are 200.
-        if (CT == 32) colgrad_f32_launch<1, 1>(c, s);
-        else if ((long long)ceil_div(c.total, 128) * c.ctiles >= 768) colgrad_f32_launch<2, 2>(c, s);
-        else colgrad_f32_launch<1, 2>(c, s);
+        // 64 pixels x 64 channels (or 128 x 32): 128 x 64 reads the weight once for
+        // twice the pixels but leaves three workgroups to a CU, 62 against 54 us at
+        // Cout 256, K 64, 32 x 56 x 56 and 58 against 50 at 256, 1024, 32 x 14 x 14.
+        if (CT == 32) colgrad_f32_launch<1>(c, s);
+        else colgrad_f32_launch<2>(c, s);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
