@@ -2177,20 +2177,26 @@ __global__ __launch_bounds__(512) void dcn2_gi_gather_kernel(const BwdParams p) 
         const int row_bytes = p.Cgp * (int)sizeof(R);
         // bf16 rows: this lane's 8 channels lie in 32-channel block co / 4 of the chunk
         const int sc_shift = 8 * (co >> 2);
-        for (int cc = cc0; cc < cc1; ++cc) {
+        // A pass takes all its channel chunks in turn, so that its record ranges (and,
+        // when one batch holds the rows, their offsets and weights) are worked out
+        // once and the next chunk's rows are in flight while one is summed.  bf16
+        // rows go chunk by chunk: their scale codes are staged per chunk.
+        constexpr bool kByChunk = kRowScaled<T>;
+        for (int oc = cc0; oc < (kByChunk ? cc1 : cc0 + 1); ++oc) {
+            const int ib = kByChunk ? oc : cc0, ie = kByChunk ? oc + 1 : cc1;  // chunks of the passes below
             if constexpr (kRowScaled<T>) {
                 // the chunk's scale codes of the batch's rows, in sorted order
-                if (cc > cc0) __syncthreads();  // the previous chunk is done with ssc
+                if (oc > cc0) __syncthreads();  // the previous chunk is done with ssc
                 const unsigned short *rsc16 =
-                    reinterpret_cast<const unsigned short *>(p.rsc) + ((size_t)row0 + base) * cpg + cc;
+                    reinterpret_cast<const unsigned short *>(p.rsc) + ((size_t)row0 + base) * cpg + oc;
                 for (int i = tid; i < nrec; i += 512) ssc[i] = rsc16[(size_t)sslot[i] * cpg];
                 __syncthreads();
             }
-            // buffer over the batch's rows from this chunk's first channel (uniform);
-            // the lane's slice goes into the offset
-            const R *rows = (const R *)p.cgm + ((size_t)row0 + base) * p.Cgp + cc * KC;
+            // buffer over the batch's rows from chunk ib's first channel (uniform); the
+            // lane's slice goes into the offset, the chunk into the scalar offset
+            const R *rows = (const R *)p.cgm + ((size_t)row0 + base) * p.Cgp + ib * KC;
             const __amdgpu_buffer_rsrc_t rrs = __builtin_amdgcn_make_buffer_rsrc(
-                const_cast<R *>(rows), (short)0, nrec * row_bytes, 0x00020000);
+                const_cast<R *>(rows), (short)0, max(0, nrec * row_bytes - ib * KC * (int)sizeof(R)), 0x00020000);
             const int slice = co * 16 * NLD;
             // Passes of PPW pixels: pass qp < NSEG takes window row qp / 2,
             // columns 1 + 8 (qp % 2) .. +7 (8 of the tile's own pixels, 8-aligned
@@ -2217,8 +2223,10 @@ __global__ __launch_bounds__(512) void dcn2_gi_gather_kernel(const BwdParams p) 
                 }
                 const int e1 = len[0], e2 = e1 + len[1], e3 = e2 + len[2], tot = e3 + len[3];
                 float sum[EPL];
+                auto clear_sum = [&]() __attribute__((always_inline)) {
 #pragma unroll
-                for (int e = 0; e < EPL; ++e) sum[e] = 0.0f;
+                    for (int e = 0; e < EPL; ++e) sum[e] = 0.0f;
+                };
                 // Row j of the pixel's corner-ordered record ranges: its record
                 // position, weight and row offset (out of range past the pixel's
                 // count), by selects only.  Lane co of the pixel's 8-lane group
@@ -2241,7 +2249,7 @@ __global__ __launch_bounds__(512) void dcn2_gi_gather_kernel(const BwdParams p) 
                     off = ok ? (int)sslot[pos] * row_bytes : kGatherOutOfRange;
                     sc = kRowScaled<T> ? (int)ssc[kRowScaled<T> ? pos : 0] : 0;
                 };
-                auto fetch = [&](int off, float w, int sc, u32x4 (&raw)[LPR][NLD], float (&wgt)[LPR]) __attribute__((always_inline)) {
+                auto fetch = [&](int off, float w, int sc, int soff, u32x4 (&raw)[LPR][NLD], float (&wgt)[LPR]) __attribute__((always_inline)) {
                     static_for<0, LPR>([&](auto uc) __attribute__((always_inline)) {
                         constexpr int u = decltype(uc)::value;
                         const int ou = __builtin_amdgcn_ds_swizzle(off, (u << 5) | 0x18);
@@ -2255,7 +2263,7 @@ __global__ __launch_bounds__(512) void dcn2_gi_gather_kernel(const BwdParams p) 
                         // in keeps either in range
 #pragma unroll
                         for (int h = 0; h < NLD; ++h)
-                            raw[u][h] = __builtin_amdgcn_raw_buffer_load_b128(rrs, ou | (slice + 16 * h), 0, 0);
+                            raw[u][h] = __builtin_amdgcn_raw_buffer_load_b128(rrs, ou | (slice + 16 * h), soff, 0);
                     });
                 };
                 auto accumulate = [&](const u32x4 (&raw)[LPR][NLD], const float (&wgt)[LPR]) __attribute__((always_inline)) {
@@ -2287,109 +2295,152 @@ __global__ __launch_bounds__(512) void dcn2_gi_gather_kernel(const BwdParams p) 
 #pragma unroll
                 for (int d = 8; d < 64; d <<= 1) tmax = max(tmax, __shfl_xor(tmax, d, 64));
                 const int nbat = __builtin_amdgcn_readfirstlane((tmax + LPR - 1) / LPR);
-                if (nbat > 0) {
-                    row_info(0, oa, xa, sa);
-                    fetch(oa, xa, sa, ra, wa);
-                    int jb = 0;
-                    for (; jb + 2 < nbat; jb += 2) {
-                        row_info((jb + 1) * LPR, ob, xb, sb);
-                        fetch(ob, xb, sb, rb, wb);
-                        __builtin_amdgcn_sched_barrier(0);
-                        accumulate(ra, wa);
-                        __builtin_amdgcn_sched_barrier(0);
-                        row_info((jb + 2) * LPR, oa, xa, sa);
-                        fetch(oa, xa, sa, ra, wa);
-                        __builtin_amdgcn_sched_barrier(0);
-                        accumulate(rb, wb);
-                        __builtin_amdgcn_sched_barrier(0);
+                auto sum_rows = [&](int cc) __attribute__((always_inline)) {
+                    const int soff = (cc - ib) * KC * (int)sizeof(R);
+                    clear_sum();
+                    if (nbat > 0) {
+                        row_info(0, oa, xa, sa);
+                        fetch(oa, xa, sa, soff, ra, wa);
+                        int jb = 0;
+                        for (; jb + 2 < nbat; jb += 2) {
+                            row_info((jb + 1) * LPR, ob, xb, sb);
+                            fetch(ob, xb, sb, soff, rb, wb);
+                            __builtin_amdgcn_sched_barrier(0);
+                            accumulate(ra, wa);
+                            __builtin_amdgcn_sched_barrier(0);
+                            row_info((jb + 2) * LPR, oa, xa, sa);
+                            fetch(oa, xa, sa, soff, ra, wa);
+                            __builtin_amdgcn_sched_barrier(0);
+                            accumulate(rb, wb);
+                            __builtin_amdgcn_sched_barrier(0);
+                        }
+                        if (jb + 1 < nbat) {
+                            row_info((jb + 1) * LPR, ob, xb, sb);
+                            fetch(ob, xb, sb, soff, rb, wb);
+                            __builtin_amdgcn_sched_barrier(0);
+                            accumulate(ra, wa);
+                            __builtin_amdgcn_sched_barrier(0);
+                            accumulate(rb, wb);
+                        } else {
+                            accumulate(ra, wa);
+                        }
                     }
-                    if (jb + 1 < nbat) {
-                        row_info((jb + 1) * LPR, ob, xb, sb);
-                        fetch(ob, xb, sb, rb, wb);
-                        __builtin_amdgcn_sched_barrier(0);
-                        accumulate(ra, wa);
-                        __builtin_amdgcn_sched_barrier(0);
-                        accumulate(rb, wb);
-                    } else {
-                        accumulate(ra, wa);
-                    }
-                }
-                // Interior pixels (reachable from this tile's cells only) are this
-                // block's alone.  With one batch their sums are final; with
-                // several, the batches before the last keep the partial sums in
-                // the bucket's gi_acc slot (the first writes them, so it needs
-                // no clearing) and the last adds them back.  The accumulator's padding channels
-                // (Cg..Cgp of a group) are never read back, so whole 16-byte
-                // pieces are written.
-                const bool inner = py >= 1 && py <= TS - 1 && px >= 1 && px <= TS - 1;
-                if (inner) {
-                    if (live && (first || last || tot > 0)) {
-                        f32x4 *d4 =
-                            reinterpret_cast<f32x4 *>(gi + ((py - 1) * (TS - 1) + px - 1) * p.Cgp + cc * KC + co * EPL);
-#pragma unroll
+                };
+                // The pass's sums of chunk cc.
+                auto emit = [&](int cc) __attribute__((always_inline)) {
+                    // Interior pixels (reachable from this tile's cells only) are this
+                    // block's alone.  With one batch their sums are final; with
+                    // several, the batches before the last keep the partial sums in
+                    // the bucket's gi_acc slot (the first writes them, so it needs
+                    // no clearing) and the last adds them back.  The accumulator's padding channels
+                    // (Cg..Cgp of a group) are never read back, so whole 16-byte
+                    // pieces are written.
+                    const bool inner = py >= 1 && py <= TS - 1 && px >= 1 && px <= TS - 1;
+                    if (inner) {
+                        if (live && (first || last || tot > 0)) {
+                            f32x4 *d4 =
+                                reinterpret_cast<f32x4 *>(gi + ((py - 1) * (TS - 1) + px - 1) * p.Cgp + cc * KC + co * EPL);
+    #pragma unroll
+                            for (int i = 0; i < EPL / 4; ++i) {
+                                f32x4 v = f32x4{sum[4 * i], sum[4 * i + 1], sum[4 * i + 2], sum[4 * i + 3]};
+                                if (!first) v += d4[i];
+                                if (!last) d4[i] = v;
+    #pragma unroll
+                                for (int k = 0; k < 4; ++k) sum[4 * i + k] = v[k];
+                            }
+                        }
+                    } else if (inwin) {
+                        // border ring: written in full every call (zeros included),
+                        // summed by ring_final_kernel, no atomics.  Later batches add
+                        // to it; this lane wrote the same entry in every earlier batch.
+                        f32x4 *r4 = reinterpret_cast<f32x4 *>(
+                            p.ring + ((size_t)bucket * kRing + ring_index(py, px)) * p.Cgp + cc * KC + co * EPL);
+    #pragma unroll
                         for (int i = 0; i < EPL / 4; ++i) {
                             f32x4 v = f32x4{sum[4 * i], sum[4 * i + 1], sum[4 * i + 2], sum[4 * i + 3]};
-                            if (!first) v += d4[i];
-                            if (!last) d4[i] = v;
-#pragma unroll
+                            if (!first) v += r4[i];
+                            r4[i] = v;
+    #pragma unroll
                             for (int k = 0; k < 4; ++k) sum[4 * i + k] = v[k];
                         }
                     }
-                } else if (inwin) {
-                    // border ring: written in full every call (zeros included),
-                    // summed by ring_final_kernel, no atomics.  Later batches add
-                    // to it; this lane wrote the same entry in every earlier batch.
-                    f32x4 *r4 = reinterpret_cast<f32x4 *>(
-                        p.ring + ((size_t)bucket * kRing + ring_index(py, px)) * p.Cgp + cc * KC + co * EPL);
-#pragma unroll
-                    for (int i = 0; i < EPL / 4; ++i) {
-                        f32x4 v = f32x4{sum[4 * i], sum[4 * i + 1], sum[4 * i + 2], sum[4 * i + 3]};
-                        if (!first) v += r4[i];
-                        r4[i] = v;
-#pragma unroll
-                        for (int k = 0; k < 4; ++k) sum[4 * i + k] = v[k];
+                    // After the last batch, the pass's 8 pixels of the tile's own
+                    // 16 x 16 block (window rows and columns 1 .. TS) go straight to
+                    // grad_input in the caller's type and layout: the interior ones
+                    // final, those on window row or column TS (tile boundary) partial,
+                    // to be overwritten by ring_final_kernel.
+                    if (last && seg && py >= 1) {
+                        T *const gout = (T *)p.gi_out;
+                        const int C = p.G * p.Cg, c0 = cc * KC + co * EPL;
+                        if (p.gi_nhwc) {
+                            // lane: its EPL channels of its pixel
+                            if (live && c0 < p.Cg) {
+                                T *dst = gout + (((size_t)b * p.H + Y) * p.W + X) * C + g * p.Cg + c0;
+                                if (p.gi_vec && c0 + EPL <= p.Cg) {
+                                    *reinterpret_cast<uint4 *>(dst) = pack16<T>(sum);
+                                } else {
+    #pragma unroll
+                                    for (int e = 0; e < EPL; ++e)
+                                        if (c0 + e < p.Cg) dst[e] = from_f32<T>(sum[e]);
+                                }
+                            }
+                        } else {
+                            // transposed through this wave's LDS: lane l then holds
+                            // KC/8 consecutive pixels (from LPX) of channel l % KC
+                            *reinterpret_cast<uint4 *>(&stage[wave][ps * KC + co * EPL]) = pack16<T>(sum);
+                            constexpr int PPL = KC / 8;  // pixels per lane: 16 bytes
+                            const int cl = lane % KC, lpx = (lane / KC) * PPL;
+                            T v[PPL];
+    #pragma unroll
+                            for (int e = 0; e < PPL; ++e) v[e] = stage[wave][(lpx + e) * KC + cl];
+                            const int X0 = ox + 1 + 8 * (qp & 1) + lpx, cgi = cc * KC + cl;
+                            if (Y < p.H && X0 < p.W && cgi < p.Cg) {
+                                T *dst = gout + (((size_t)b * C + g * p.Cg + cgi) * p.H + Y) * p.W + X0;
+                                if (p.gi_vec && X0 + PPL <= p.W) {
+                                    *reinterpret_cast<uint4 *>(dst) = __builtin_bit_cast(uint4, v);
+                                } else {
+    #pragma unroll
+                                    for (int e = 0; e < PPL; ++e)
+                                        if (X0 + e < p.W) dst[e] = v[e];
+                                }
+                            }
+                        }
                     }
-                }
-                // After the last batch, the pass's 8 pixels of the tile's own
-                // 16 x 16 block (window rows and columns 1 .. TS) go straight to
-                // grad_input in the caller's type and layout: the interior ones
-                // final, those on window row or column TS (tile boundary) partial,
-                // to be overwritten by ring_final_kernel.
-                if (last && seg && py >= 1) {
-                    T *const gout = (T *)p.gi_out;
-                    const int C = p.G * p.Cg, c0 = cc * KC + co * EPL;
-                    if (p.gi_nhwc) {
-                        // lane: its EPL channels of its pixel
-                        if (live && c0 < p.Cg) {
-                            T *dst = gout + (((size_t)b * p.H + Y) * p.W + X) * C + g * p.Cg + c0;
-                            if (p.gi_vec && c0 + EPL <= p.Cg) {
-                                *reinterpret_cast<uint4 *>(dst) = pack16<T>(sum);
-                            } else {
+                };
+                if (!kByChunk && nbat == 1 && ie - ib > 1) {
+                    row_info(0, oa, xa, sa);
+                    int ou[LPR];
+                    static_for<0, LPR>([&](auto uc) __attribute__((always_inline)) {
+                        constexpr int u = decltype(uc)::value;
+                        ou[u] = __builtin_amdgcn_ds_swizzle(oa, (u << 5) | 0x18) | slice;
+                        wa[u] = __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(xa), (u << 5) | 0x18));
+                    });
+                    auto load = [&](int cc, u32x4 (&raw)[LPR][NLD]) __attribute__((always_inline)) {
+                        const int soff = (min(cc, ie - 1) - ib) * KC * (int)sizeof(R);
 #pragma unroll
-                                for (int e = 0; e < EPL; ++e)
-                                    if (c0 + e < p.Cg) dst[e] = from_f32<T>(sum[e]);
-                            }
-                        }
-                    } else {
-                        // transposed through this wave's LDS: lane l then holds
-                        // KC/8 consecutive pixels (from LPX) of channel l % KC
-                        *reinterpret_cast<uint4 *>(&stage[wave][ps * KC + co * EPL]) = pack16<T>(sum);
-                        constexpr int PPL = KC / 8;  // pixels per lane: 16 bytes
-                        const int cl = lane % KC, lpx = (lane / KC) * PPL;
-                        T v[PPL];
+                        for (int u = 0; u < LPR; ++u)
 #pragma unroll
-                        for (int e = 0; e < PPL; ++e) v[e] = stage[wave][(lpx + e) * KC + cl];
-                        const int X0 = ox + 1 + 8 * (qp & 1) + lpx, cgi = cc * KC + cl;
-                        if (Y < p.H && X0 < p.W && cgi < p.Cg) {
-                            T *dst = gout + (((size_t)b * C + g * p.Cg + cgi) * p.H + Y) * p.W + X0;
-                            if (p.gi_vec && X0 + PPL <= p.W) {
-                                *reinterpret_cast<uint4 *>(dst) = __builtin_bit_cast(uint4, v);
-                            } else {
-#pragma unroll
-                                for (int e = 0; e < PPL; ++e)
-                                    if (X0 + e < p.W) dst[e] = v[e];
-                            }
-                        }
+                            for (int h = 0; h < NLD; ++h)
+                                raw[u][h] = __builtin_amdgcn_raw_buffer_load_b128(rrs, ou[u] | (16 * h), soff, 0);
+                    };
+                    load(ib, ra);
+                    for (int cc = ib; cc < ie; cc += 2) {
+                        load(cc + 1, rb);
+                        __builtin_amdgcn_sched_barrier(0);
+                        clear_sum();
+                        accumulate(ra, wa);
+                        emit(cc);
+                        if (cc + 1 >= ie) break;
+                        load(cc + 2, ra);
+                        __builtin_amdgcn_sched_barrier(0);
+                        clear_sum();
+                        accumulate(rb, wa);
+                        emit(cc + 1);
+                    }
+                } else {
+                    for (int cc = ib; cc < ie; ++cc) {
+                        sum_rows(cc);
+                        emit(cc);
                     }
                 }
             }
