@@ -1405,7 +1405,9 @@ __device__ __forceinline__ int fused_swz_c(int n) { return ((n & 3) << 1) | ((n 
 constexpr int kFusedTrashLane = 32;
 
 
-template <typename T, bool GN, int MP>
+// CG16 (f16): the corner sums take the column gradient rounded to f16.  Off for a
+// padded grad_output, whose shapes kept it in fp32 before this kernel served them.
+template <typename T, bool GN, int MP, bool CG16>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void dcn2_bwd_fused_kernel(const BwdParams p) {
     static_assert(sizeof(T) == 2, "2-byte types");
@@ -1714,14 +1716,14 @@ void dcn2_bwd_fused_kernel(const BwdParams p) {
         }
         at(0);
         // corner sums over the lane's 8 channels, then over the 4 lanes of the
-        // pixel.  f16: 2-element dot products (v_dot2_f32_f16) of the corner
+        // pixel.  CG16: 2-element dot products (v_dot2_f32_f16) of the corner
         // values with the column gradient rounded to f16, accumulated in fp32
         // (the rounding is that of the f16 grad_offset / grad_mask outputs).
         f32x4 S;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             float s = 0.0f;
-            if constexpr (std::is_same<T, f16>::value) {
+            if constexpr (CG16) {
                 typedef f16 h2 __attribute__((ext_vector_type(2)));
                 typedef float f2 __attribute__((ext_vector_type(2)));
                 const f16x8 x = __builtin_bit_cast(f16x8, raw[q]);
@@ -3095,8 +3097,10 @@ static hipError_t backward_t(const Geo &g, const BwdParams &p0, void *grad_input
                     const int grid = pf.splits * nch;
 #define DCN2_FUSED(MPV)                                                                     \
     do {                                                                                    \
-        if (p.go_nhwc) dcn2_bwd_fused_kernel<T, true, MPV><<<grid, 512, 0, s>>>(pf);       \
-        else dcn2_bwd_fused_kernel<T, false, MPV><<<grid, 512, 0, s>>>(pf);                \
+        constexpr bool F16 = std::is_same<T, f16>::value;                                   \
+        if (p.go_nhwc) dcn2_bwd_fused_kernel<T, true, MPV, F16><<<grid, 512, 0, s>>>(pf);  \
+        else if (go_padded(g)) dcn2_bwd_fused_kernel<T, false, MPV, false><<<grid, 512, 0, s>>>(pf); \
+        else dcn2_bwd_fused_kernel<T, false, MPV, F16><<<grid, 512, 0, s>>>(pf);           \
     } while (0)
                     if (g.Mp == 256) DCN2_FUSED(256);
                     else DCN2_FUSED(128);

@@ -33,7 +33,8 @@
  * fp16 (fp16 calls) or to fp16 with one power-of-two scale per 32 channels
  * (bf16 calls: an 11-bit significand over bf16's exponent range); for fp16
  * the one multiplied into the corner sums of grad_offset / grad_mask is
- * rounded to fp16 too (products and sums stay fp32); fp32 has none.
+ * rounded to fp16 too where the fused kernel reads grad_output in place
+ * (products and sums stay fp32); fp32 has none.
  *
  * Return value of every int function: 0 = success, otherwise a DCN2_E* code;
  * dcn2_last_error() then describes the failure.  This replaces the reference's
