@@ -223,6 +223,9 @@ __global__ __launch_bounds__(256) void dcn2_colgrad_f32_kernel(const CgF32Params
 #pragma unroll
         for (int q = 0; q < 4; ++q)
             S[q] = lane_sum<LP>(fmaf(v[0], x[q][0], fmaf(v[1], x[q][1], fmaf(v[2], x[q][2], v[3] * x[q][3]))));
+        // (nothing from a corner outside, also where the column gradient is not finite)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) S[q] = d.off[q] != c.x_bytes ? S[q] : 0.0f;
         if (l4 == 0) sS[px] = S;
     }
     __syncthreads();
@@ -384,17 +387,20 @@ __global__ __launch_bounds__(64 * WM * CB) void dcn2_gradw_f32_kernel(const GwF3
         const SamplePos s = sample_pos((float)(oy * p.sh + ty) + dy, (float)(ox * p.sw + tx) + dx, p.H, p.W);
         const float m = MASK ? mask_value(mv, p.msk_logit) : 1.0f;
         const float hy = (1.0f - s.ly) * m, ly = s.ly * m, hx = 1.0f - s.lx, lx = s.lx;
-        w[0] = hy * hx;
-        w[1] = hy * lx;
-        w[2] = ly * hx;
-        w[3] = ly * lx;
         const uint32_t cs = p.G * p.Cgp * 4u, row = cs * (uint32_t)p.W;
         const uint32_t base = (b * (uint32_t)(p.H * p.W) + (uint32_t)(s.y0 * p.W + s.x0)) * cs + l4 * 4u;
-        // (a corner outside the image, or of a pixel past the end, reads 0)
-        const uint32_t off[4] = {live && s.vy0 && s.vx0 ? base : c.x_bytes,
-                                 live && s.vy0 && s.vx1 ? base + cs : c.x_bytes,
-                                 live && s.vy1 && s.vx0 ? base + row : c.x_bytes,
-                                 live && s.vy1 && s.vx1 ? base + row + cs : c.x_bytes};
+        // A corner outside the image, or of a pixel past the end, reads 0 and has
+        // weight 0 (0 times a mask that is not finite is not 0).
+        const bool v[4] = {live && s.vy0 && s.vx0, live && s.vy0 && s.vx1, live && s.vy1 && s.vx0,
+                           live && s.vy1 && s.vx1};
+        const uint32_t o[4] = {base, base + cs, base + row, base + row + cs};
+        const float wq[4] = {hy * hx, hy * lx, ly * hx, ly * lx};
+        uint32_t off[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            off[q] = v[q] ? o[q] : c.x_bytes;
+            w[q] = v[q] ? wq[q] : 0.0f;
+        }
 #pragma unroll
         for (int q = 0; q < 4; ++q)
             x[q] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(xrs, (int)off[q], soff, 0));

@@ -160,14 +160,15 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void dcn2_fwd_tile_kernel(const 
             const float hy = (1.0f - sp.ly) * m, ly = sp.ly * m, hx = 1.0f - sp.lx, lx = sp.lx;
             const uint32_t base = (ximg[i] + (uint32_t)(sp.y0 * p.W + sp.x0)) * (uint32_t)(p.cs * sizeof(T)) + cq * 16u;
             const uint32_t px = (uint32_t)p.cs * (uint32_t)sizeof(T), row = px * (uint32_t)p.W, out = p.x_bytes;
-            co[i][0] = sp.vy0 && sp.vx0 ? base : out;
-            co[i][1] = sp.vy0 && sp.vx1 ? base + px : out;
-            co[i][2] = sp.vy1 && sp.vx0 ? base + row : out;
-            co[i][3] = sp.vy1 && sp.vx1 ? base + row + px : out;
-            w[i][0] = hy * hx;
-            w[i][1] = hy * lx;
-            w[i][2] = ly * hx;
-            w[i][3] = ly * lx;
+            // (weight 0 as well outside: 0 times a mask that is not finite is not 0)
+            const bool v[4] = {sp.vy0 && sp.vx0, sp.vy0 && sp.vx1, sp.vy1 && sp.vx0, sp.vy1 && sp.vx1};
+            const uint32_t o[4] = {base, base + px, base + row, base + row + px};
+            const float wq[4] = {hy * hx, hy * lx, ly * hx, ly * lx};
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                co[i][q] = v[q] ? o[q] : out;
+                w[i][q] = v[q] ? wq[q] : 0.0f;
+            }
         }
         // (a corner outside the image has an offset past the buffer and reads 0)
 #pragma unroll
