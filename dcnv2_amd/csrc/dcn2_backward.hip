@@ -9,7 +9,7 @@
 //  bucket passes   each sample (image, offset plane, pixel) gets a row in the
 //                  bucket of the 16x16 cell tile its bilinear cell lies in
 //                  (count, scan, place; the rows are sized exactly)
-//  fused kernel    (2-byte types, 128 < Cout <= 256, one K chunk per group)
+//  fused kernel    (2-byte types, Cout <= 256)
 //     cg[k][n] = sum_m Wt[k][m] * gO[m][n]            MFMA, kept on chip (LDS)
 //     grad_mask / grad_offset  via the corner sums    S_q = sum_c cg_c * x_c(corner q)
 //         grad_mask = sum_q w_q S_q,  grad_off_y = mask * sum_q dw_q/dy S_q, ...
@@ -19,7 +19,8 @@
 //     gW[m][k] += sum_n gO[m][n] * col[k][n]           MFMA over the columns
 //       blended from the same corner gathers; grad_bias from the same gO
 //  otherwise       dcn2_colgrad_kernel (all but grad_weight) and a grad_weight
-//                  kernel that re-samples the columns
+//                  kernel that re-samples the columns (fp32: both in
+//                  dcn2_backward_f32.hip)
 //  grad_input      per cell tile, from the tile's bucket rows (no atomics):
 //                  summed by cells or pulled per pixel, written straight to
 //                  grad_input in the caller's type and layout; then the
@@ -161,9 +162,6 @@ __device__ __forceinline__ int bucket_append(bool want, int key, int *ctr) {
 }
 
 template <typename T, int KPL> struct FragSet;
-template <typename T> struct FragSet<T, 1> {
-    template <typename F> static __device__ __forceinline__ void set(F &f, int, T v) { f = v; }
-};
 template <typename T> struct FragSet<T, 8> {
     template <typename F> static __device__ __forceinline__ void set(F &f, int e, T v) { f[e] = v; }
 };
@@ -423,7 +421,7 @@ constexpr int kTrashBytes = 64 * 1024;
 __device__ __attribute__((aligned(16))) unsigned char dcn2_trash[kTrashBytes];
 
 // ---------------------------------------------------------------------------
-// Column-gradient kernel: grad_offset, grad_mask and grad_input.
+// Column-gradient kernel (2-byte types): grad_offset, grad_mask and grad_input.
 // 512 threads; BN = 128 output pixels of one image per block.
 // ALDS: the W'^T fragments of a chunk (Mp*128 bytes, Mp <= 256) are staged in
 // LDS two chunks ahead; otherwise every wave reads its fragments from memory.
@@ -448,7 +446,8 @@ __global__ __launch_bounds__(512) void dcn2_colgrad_kernel(const BwdParams p) {
     using frag = typename M::frag;
     constexpr int KC = M::KC, KPL = M::KPL, KSTEP = M::KSTEP;
     constexpr int BN = 128;
-    constexpr int NB = (KC / 32) * (BN / 32);  // 32x32 blocks of one chunk (8 or 4)
+    static_assert(sizeof(T) == 2, "fp32 takes dcn2_colgrad_f32_kernel");
+    constexpr int NB = (KC / 32) * (BN / 32);  // 32x32 blocks of one chunk
     constexpr int WPB = 8 / NB;                // waves sharing one block's M reduction
     constexpr int MPW = MCH / WPB;             // M range of one wave per M chunk
     constexpr int NMS = MPW / KSTEP;           // MFMA steps per wave per M chunk
@@ -533,8 +532,8 @@ __global__ __launch_bounds__(512) void dcn2_colgrad_kernel(const BwdParams p) {
     // receives rows 0..3 of that half at pixel i.  Row m keeps its 32-byte
     // blocks XOR-permuted by m%4, which puts the 4 rows of one read on
     // distinct banks.  Rows past Cout and pixels past N read 0 (buffer range).
-    constexpr int GQ = (sizeof(T) == 2 ? MCH * (BN / 8) : 512) / 512;  // 16-byte pieces per thread
-    const bool go_stage = ONEM && sizeof(T) == 2 && p.go_vec && !p.go_nhwc &&
+    constexpr int GQ = MCH * (BN / 8) / 512;  // 16-byte pieces per thread
+    const bool go_stage = ONEM && p.go_vec && !p.go_nhwc &&
                           (size_t)p.Cout * p.go_n * sizeof(T) <= (size_t)kGoOutOfRange;
     uint4 gst[GQ];
     auto go_stage_issue = [&]() __attribute__((always_inline)) {
@@ -558,23 +557,19 @@ __global__ __launch_bounds__(512) void dcn2_colgrad_kernel(const BwdParams p) {
         }
     };
     auto go_stage_read = [&]() __attribute__((always_inline)) {
-        if constexpr (sizeof(T) == 2) {
-            typedef short s16x4 __attribute__((ext_vector_type(4)));
-            const int g = lane >> 4, li = lane & 15;
+        typedef short s16x4 __attribute__((ext_vector_type(4)));
+        const int g = lane >> 4, li = lane & 15;
 #pragma unroll
-            for (int s = 0; s < NMS; ++s) {
-                s16x4 h[2];
+        for (int s = 0; s < NMS; ++s) {
+            s16x4 h[2];
 #pragma unroll
-                for (int hh = 0; hh < 2; ++hh) {
-                    const int m = wr * MPW + s * KSTEP + 8 * (g >> 1) + 4 * hh + (li >> 2);
-                    const int nl = nb * 32 + 16 * (g & 1) + 4 * (li & 3);
-                    h[hh] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                        (__attribute__((address_space(3))) s16x4 *)(gstg + m * BN +
-                                                                    (nl ^ ((m & 3) << 4))));
-                }
-                gfr[s] = __builtin_bit_cast(frag, __builtin_shufflevector(h[0], h[1], 0, 1, 2, 3, 4, 5,
-                                                                           6, 7));
+            for (int hh = 0; hh < 2; ++hh) {
+                const int m = wr * MPW + s * KSTEP + 8 * (g >> 1) + 4 * hh + (li >> 2);
+                const int nl = nb * 32 + 16 * (g & 1) + 4 * (li & 3);
+                h[hh] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                    (__attribute__((address_space(3))) s16x4 *)(gstg + m * BN + (nl ^ ((m & 3) << 4))));
             }
+            gfr[s] = __builtin_bit_cast(frag, __builtin_shufflevector(h[0], h[1], 0, 1, 2, 3, 4, 5, 6, 7));
         }
     };
 
