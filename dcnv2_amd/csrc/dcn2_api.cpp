@@ -90,6 +90,7 @@ int make_geo(const dcn2_desc *d, Geo &g) {
     g.opt_fused = g_opt_fused.load(std::memory_order_relaxed);
     g.opt_push = g_opt_push.load(std::memory_order_relaxed);
     g.Bs = g.B;
+    g.by_cells = 0;  // (plan_backward)
     g.esz = g.dtype == DCN2_F32 ? 4 : 2;
     g.KC = g.dtype == DCN2_F32 ? 32 : 64;
     g.Cg = g.C / g.G;
@@ -189,7 +190,7 @@ BwdWorkspace bwd_workspace(const Geo &g0) {
     o += align256((size_t)(g.Kp / g.KC) * 16);
     const GatherGeo gg = gather_geometry(g);
     w.gi_acc = o;  // (by pixels only: partial sums of buckets of several record batches)
-    if (!gg.by_cells) o += align256((size_t)gg.acc_bytes);
+    o += align256((size_t)gg.acc_bytes);
     w.gw_acc = o;
     o += align256((size_t)g.Mp * g.Kp * sizeof(float));
     w.gb_acc = o;
@@ -245,6 +246,19 @@ static int bwd_slice_images(const Geo &g) {
     }
     const int nslices = (g.B + lo - 1) / lo;
     return (g.B + nslices - 1) / nslices;
+}
+
+// Chooses the grad_input kernel and the slices of a backward call.  The kernel is
+// the one for a full slice; a shorter last slice takes it too, since its buffers
+// are those of the full slice's layout (by cells has no gi_acc) and the slice
+// sizes follow from that layout.
+static void plan_backward(Geo &g) {
+    g.by_cells = gather_by_cells(g, g.B);
+    g.Bs = bwd_slice_images(g);
+    if (g.by_cells && !gather_by_cells(g, g.Bs)) {
+        g.by_cells = 0;
+        g.Bs = bwd_slice_images(g);
+    }
 }
 
 static int check_launch(hipError_t e, const char *what) {
@@ -306,7 +320,7 @@ static int backward_impl(const Geo &g0, const void *input, const void *weight, c
     if ((mask == nullptr) != (grad_mask == nullptr))
         return fail(DCN2_EINVAL, "dcn2_backward: grad_mask must be given exactly when mask is");
     Geo g = g0;
-    g.Bs = bwd_slice_images(g0);
+    plan_backward(g);
     const BwdWorkspace ws = bwd_workspace(g);
     if (!workspace || workspace_bytes < ws.total || ((uintptr_t)workspace & 255))
         return fail(DCN2_EWORKSPACE,
@@ -400,7 +414,7 @@ size_t dcn2_forward_workspace_bytes(const dcn2_desc *d) {
 size_t dcn2_backward_workspace_bytes(const dcn2_desc *d) {
     Geo g;
     if (make_geo(d, g)) return 0;
-    g.Bs = bwd_slice_images(g);
+    plan_backward(g);
     return bwd_workspace(g).total;
 }
 

@@ -3199,7 +3199,7 @@ static hipError_t backward_t(const Geo &g, const BwdParams &p0, void *grad_input
         // 56 x 56), 115 -> 35 (12 of 4, bf16 3x3 at 2 x 25 x 42).  Two or four to a CU
         // measured 50-55, 17-22, 23, 35: the sorts repeat.
         const int gcpg = g.Cgp / g.KC;
-        if (gg.by_cells) {
+        if (g.by_cells) {
             p.gi_cs = std::min(gcpg, ceil_div(ncu, nbk));
             dcn2_gi_push_kernel<T><<<nbk * p.gi_cs, 512, 0, s>>>(p);
         } else {
@@ -3257,20 +3257,28 @@ GatherGeo gather_geometry(const Geo &g) {
     gg.row_scaled = row_scaled(g.dtype) ? 1 : 0;
     gg.batch_bytes = (long)kGatherBatch * g.Cgp * gg.row_esz;
     gg.max_batch_bytes = kGatherOutOfRange;
-    // By cells (each row read once, one block per CU) when the buckets are
-    // full enough to amortise a block's fixed work; per pixel otherwise.
-    // Option DCN2_OPT_GI_PUSH = 1 / 0 forces either.  Measured: c2 68
-    // against 72 us, c3 ~190 against 282 us (2304 samples per bucket); c4
-    // (576 per bucket) ~118 against 73 us.  With few (bucket, channel chunk)
-    // pairs the per-pixel kernel's passes still split four ways: 24 against 43
-    // us for the stage at 48 pairs (bf16 3x3, 2 x 25 x 42, C 256), 33 against 31
-    // at 256 (fp32 3x3, 4 x 56 x 56, C 128).
-    gg.by_cells = g.opt_push >= 0 ? g.opt_push != 0
-                                  : gg.rows >= (long)kPushMinPerBucket * gg.nbuckets &&
-                                        gg.nbuckets * (g.Cgp / g.KC) >= kPushMinPairs;
-    gg.acc_bytes = gg.rows / (kGatherBatch + 1) * (long)(kCellTile - 1) * (kCellTile - 1) * g.Cgp *
-                   (long)sizeof(float);
+    gg.acc_bytes = g.by_cells ? 0
+                              : gg.rows / (kGatherBatch + 1) * (long)(kCellTile - 1) * (kCellTile - 1) *
+                                    g.Cgp * (long)sizeof(float);
     return gg;
+}
+
+// By cells (each row read once, one block per CU) when the buckets are full enough
+// to amortise a block's fixed work; per pixel otherwise.  Option DCN2_OPT_GI_PUSH =
+// 1 / 0 forces either.  Measured: c2 68 against 72 us, c3 ~190 against 282 us (2304
+// samples per bucket); c4 (576 per bucket) ~118 against 73 us.  With few (bucket,
+// channel chunk) pairs the per-pixel kernel's passes still split four ways.  Whole
+// backward, us by cells / per pixel, at 47 x 47 maps of 9 buckets, 128 rows out, one to
+// 16 images of one or four chunks: at 108 pairs 102 / 89 (fp16 3x3), 181 / 161
+// (5x5), 313 / 283 (7x7), 132 / 128, 252 / 243 and 451 / 444 (fp32); at 144 pairs 115
+// / 113, 213 / 216, 412 / 454, 135 / 137, 270 / 288 and 508 / 548.
+bool gather_by_cells(const Geo &g, int images) {
+    if (g.opt_push >= 0) return g.opt_push != 0;
+    Geo t = g;
+    t.B = images;
+    const GatherGeo gg = gather_geometry(t);
+    return gg.rows >= (long)kPushMinPerBucket * gg.nbuckets &&
+           gg.nbuckets * (g.Cgp / g.KC) >= kPushMinPairs;
 }
 
 hipError_t launch_backward(const Geo &g, const void *xt, const void *wt, const void *tab,

@@ -46,8 +46,10 @@ struct Geo {
     // grad_input by cells (-1 auto, 0 per pixel, 1 by cells).
     long long slice_bytes;
     int opt_fused, opt_push;
-    // The images of one backward slice (B when the batch runs in one piece).
-    int Bs;
+    // The images of one backward slice (B when the batch runs in one piece), and
+    // whether grad_input goes by cells: one decision for all slices of a call,
+    // which also lays out their common workspace (plan_backward).
+    int Bs, by_cells;
 };
 
 // dcn2_api.cpp: the descriptor check shared by every entry point, the forward
@@ -82,16 +84,16 @@ struct GatherGeo {
     int row_scaled;  // bf16 rows carry one scale byte per 32 channels
     long nbuckets, rows;
     long batch_bytes, max_batch_bytes;
-    // grad_input by cells (dcn2_gi_push_kernel) or by pixels
-    // (dcn2_gi_gather_kernel, which keeps the partial sums of a bucket of
-    // several record batches in an fp32 accumulator, gi_acc); both write the
-    // caller's grad_input directly
-    bool by_cells;
-    // bytes of gi_acc (by pixels): one slot of interior pixels per bucket of
-    // several record batches, at most rows / (batch + 1) of them
+    // bytes of gi_acc: one slot of interior pixels per bucket of several record
+    // batches, at most rows / (batch + 1) of them (none by cells)
     long acc_bytes;
 };
 GatherGeo gather_geometry(const Geo &g);
+// Whether grad_input of a slice of `images` images is faster by cells
+// (dcn2_gi_push_kernel) than by pixels (dcn2_gi_gather_kernel, which keeps the
+// partial sums of a bucket of several record batches in an fp32 accumulator,
+// gi_acc); both write the caller's grad_input directly.
+bool gather_by_cells(const Geo &g, int images);
 
 // dcn2_pack.hip: input -> xt (skipped when input is null) and weight -> wp +
 // chunk table (skipped when weight is null) in one launch; transpose selects the backward's W'^T fragment

@@ -141,3 +141,32 @@ def test_backward_om_in_slices(dtype):
     check("grad_om[logits] (sliced)", gom[:, 2 * kk:], r_gmask * m * (1.0 - m), tol)
     check("grad_weight (om, sliced)", gw, r_gw, tol)
     check("grad_bias (om, sliced)", gb, r_gb, tol)
+
+
+@pytest.mark.parametrize("dtype,B,C,slices", [
+    # 3 x 3 cell tiles x chunks: (bucket, channel chunk) pairs of a full slice and of the last one
+    (torch.float16, 3, 512, 2),   # 144, 72: by cells, though the last alone would go by pixels
+    (torch.bfloat16, 3, 512, 2),
+    (torch.float32, 3, 256, 2),
+    (torch.float16, 5, 256, 3),   # 72, 36 (180 in all): by pixels
+], ids=["f16_by_cells", "bf16_by_cells", "f32_by_cells", "f16_per_pixel"])
+def test_short_last_slice_automatic_kernel(dtype, B, C, slices):
+    """The last slice holds fewer images than the others and the grad_input kernel is
+    chosen by the library; the first tile's bucket holds 16 * 16 * 25 samples, more
+    than one batch (4096), so by pixels keeps partial sums in the workspace."""
+    print(f"case {dtype} {B} {C}", flush=True)
+    w = CONFIGS[0].with_(B=B, C=C, H=32, W=32, Cout=16, k=5, stride=1, pad=2, dil=1, groups=1,
+                         seed=59, offset_dist="normal:0.5", backward=True)
+    t = make_inputs(w, dtype=dtype)
+    geo = w.geometry()
+    rg = oracle.dcn_backward(*(t[k] for k in IN5), t["grad_output"], pos_f32=True, **geo)
+    dev = [t[k].to(DEV) for k in IN5]
+    go = t["grad_output"].to(DEV)
+    args = (1, 1, 2, 2, 1, 1, 1)
+    d = _C.make_desc(dev[0][:2], dev[1], *args)
+    budget = _C.lib().dcn2_backward_workspace_bytes(ctypes.byref(d))  # two images
+    with _C.option("bwd_slice_bytes", budget):
+        grads, n = _sliced(lambda: _C.dcn_v2_backward(*dev, go, *args))
+    assert n == slices
+    for name, g, r in zip(GRADS, grads, rg):
+        check(f"{name} (short last slice)", g, r, TOL[dtype])

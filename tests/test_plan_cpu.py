@@ -1,0 +1,70 @@
+"""What the library's host code plans for a call, read on the CPU through
+``plan_probe.cpp``: every slice of a backward call uses no more of the workspace than
+its layout holds, and all slices take the same grad_input kernel."""
+import glob
+import os
+import subprocess
+
+import pytest
+
+from dcnv2_amd import build
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+DEFAULT_BUDGET = 192 << 20
+F32, F16 = 0, 1
+
+
+@pytest.fixture(scope="module")
+def probe(tmp_path_factory):
+    objs = glob.glob(os.path.join(build.BUILD, "*.o"))
+    if len(objs) != len([f for f in os.listdir(build.CSRC) if f.endswith((".hip", ".cpp"))]):
+        build.build(verbose=False)
+        objs = glob.glob(os.path.join(build.BUILD, "*.o"))
+    exe = str(tmp_path_factory.mktemp("plan") / "plan_probe")
+    hipcc = [build.HIPCC, f"--offload-arch={build.ARCH}"]
+    for cmd in ([*hipcc, "-std=c++17", "-c", os.path.join(HERE, "plan_probe.cpp"), "-o", exe + ".o"],
+                [*hipcc, "-Wl,--allow-multiple-definition", exe + ".o", *objs, "-o", exe]):
+        subprocess.run(cmd, check=True, capture_output=True)
+
+    def run(budget, push, desc):
+        r = subprocess.run([exe], input=" ".join(str(v) for v in (budget, push, *desc)), text=True,
+                           capture_output=True, check=True)
+        return [[int(v) for v in ln.split()] for ln in r.stdout.splitlines() if ln]
+
+    return run
+
+
+def _desc(dtype, B, C, H, W, Cout, k, dg=1):
+    return (B, C, H, W, Cout, k, k, 1, 1, k // 2, k // 2, 1, 1, dg, dtype, 1, 0, 0)
+
+
+# The last slice is shorter than the others, so that it alone has fewer than 128
+# (bucket, channel chunk) pairs, the count from which grad_input goes by cells; each
+# bucket of its interior holds more than one batch (4096) of samples.
+@pytest.mark.parametrize("case,slices,pairs", [
+    ((F16, 7, 128, 63, 63, 128, 5), (4, 3), 32),      # 4 images by cells: 128 pairs
+    ((F16, 5, 64, 104, 104, 64, 5), (3, 2), 49),      # 147
+    ((F32, 7, 128, 63, 63, 64, 5), (3, 3, 1), 64),    # 192
+    ((F16, 11, 64, 47, 47, 64, 7, 2), (4, 4, 3), 18), # 72: by pixels throughout
+], ids=str)
+def test_short_last_slice_keeps_the_kernel(probe, case, slices, pairs):
+    got = probe(DEFAULT_BUDGET, -1, _desc(*case))
+    assert tuple(r[0] for r in got) == slices
+    assert {r[1] for r in got} == {int(slices[0] * pairs >= 128)}
+    for r in got:
+        for need, room in zip(r[2::2], r[3::2]):
+            assert need <= room
+
+
+def test_slices_fit_their_layout(probe):
+    """The same over batches, budgets and both forced kernels."""
+    for case in ((F16, 64, 63, 63, 128, 5), (F16, 128, 63, 63, 300, 5), (F32, 96, 40, 90, 64, 7),
+                 (F16, 192, 33, 20, 64, 3), (F32, 512, 14, 14, 64, 1)):
+        for B in range(1, 24, 2):
+            for budget in (16 << 20, 100 << 20, DEFAULT_BUDGET):
+                for push in (-1, 0, 1):
+                    got = probe(budget, push, _desc(case[0], B, *case[1:]))
+                    assert sum(r[0] for r in got) == B and len({r[1] for r in got}) == 1
+                    assert push < 0 or got[0][1] == push
+                    for r in got:
+                        assert all(need <= room for need, room in zip(r[2::2], r[3::2]))
