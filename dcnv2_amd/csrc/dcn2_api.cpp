@@ -199,8 +199,8 @@ BwdWorkspace bwd_workspace(const Geo &g0) {
     o += align256((size_t)gg.rows * g.Cgp * gg.row_esz);
     w.rsc = o;
     if (gg.row_scaled) o += align256((size_t)gg.rows * (g.Cgp / 32));
-    w.csum = o;  // fp32 corner sums [B][G*KK][N][4] of groups that workgroups share
-    if (csum_shape(g)) o += align256((size_t)g.B * g.G * g.KK * g.N * 16);
+    w.csum = o;  // fp32 corner sums of groups that workgroups share
+    o += align256((size_t)csum_planes(g) * g.B * g.G * g.KK * g.N * 16);
     w.rec = o;
     o += align256((size_t)gg.rows * 12);  // 12-byte sample records
     w.bcnt = o;
@@ -362,7 +362,7 @@ static int backward_impl(const Geo &g0, const void *input, const void *weight, c
         clr.p[2] = (float *)(base + ws.bcnt);
         clr.n[2] = gs.B > 0 ? (ws.bcur - ws.bcnt) / sizeof(int) + (size_t)gg.nbuckets : 0;
         clr.p[3] = (float *)(base + ws.csum);
-        clr.n[3] = ws.rec > ws.csum && gs.B > 0 ? (size_t)gs.B * g.G * g.KK * g.N * 4 : 0;
+        clr.n[3] = csum_planes(g) == 1 ? (size_t)gs.B * g.G * g.KK * g.N * 4 : 0;  // (added to)
         prof_begin(DCN2_STAGE_BWD_PACK, s);
         if ((rc = check_launch(launch_pack(gs, g.xt_direct ? nullptr : in_s, (void *)xt,
                                            first ? weight : nullptr, wt, tab, true, s, &clr,

@@ -33,7 +33,9 @@ struct BwdParams {
     // sample), so the storage is sized exactly and no bucket can overflow.
     void *cgm;          // [rows][Cgp] masked column gradient rows (RowOf)
     unsigned char *rsc; // [rows][Cgp/32] scale codes of bf16 rows (row_block_scale)
-    float *csum;        // [B][G*KK][N][4] corner sums of groups of several chunks (fused kernel)
+    float *csum;        // corner sums of groups that workgroups share (csum_planes)
+    int csum_n;         // its planes [B][G*KK][N][4]
+    size_t csum_ps;     // floats between them (0: one plane, added to with atomics)
     struct BucketRec *rec;  // [rows] sample records, in bucket order
     int *bcnt;          // [nbuckets] samples per bucket (count pass)
     int *bstart;        // [nbuckets + 1] first row of each bucket (exclusive scan of bcnt)

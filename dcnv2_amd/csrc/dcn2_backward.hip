@@ -1791,11 +1791,13 @@ void dcn2_bwd_fused_kernel(const BwdParams p) {
         const f32x4 S = sS[0][lane] + sS[1][lane];
         if (cpg > 1) {
             // a group of several chunks: this chunk's part of the corner sums
-            // goes to p.csum, summed over the group's chunks there, and
+            // goes to p.csum (its own plane, or added to the one plane), and
             // ring_final_kernel (corner_finish) turns the totals into grad_offset /
             // grad_mask
             float *cs4 = p.csum + (((size_t)b * p.G * KK + plane) * N + (nr < N ? nr : 0)) * 4;
-            if (nr < N) {
+            if (p.csum_ps) {
+                if (nr < N) *reinterpret_cast<f32x4 *>(cs4 + cbase / KC * p.csum_ps) = S;
+            } else if (nr < N) {
 #pragma unroll
                 for (int q = 0; q < 4; ++q) unsafeAtomicAdd(cs4 + q, S[q]);
             }
@@ -1991,12 +1993,11 @@ void dcn2_bwd_fused_kernel(const BwdParams p) {
 }
 
 // ---------------------------------------------------------------------------
-// grad_offset / grad_mask of the fused kernel for groups of several channel
-// chunks: the corner sums S_q of a sample, summed over the group's chunks in
-// csum by the fused kernel's workgroups, become the coordinate and mask
-// gradients (com.cu:431-501), with the sample position, corner validity and
-// mask value recomputed from the offsets exactly as the fused kernel's
-// sampler does.  One thread per sample (pixel n, plane g*KK + tap, image b),
+// grad_offset / grad_mask of groups whose channels several workgroups share: the
+// corner sums S_q of a sample, the sum of csum's planes in their order, become
+// the coordinate and mask gradients (com.cu:431-501), with the sample position,
+// corner validity and mask value recomputed from the offsets exactly as the
+// column-gradient kernel's sampler does.  One thread per sample (pixel n, plane g*KK + tap, image b),
 // run as a block range of ring_final_kernel.
 template <typename T>
 __device__ __forceinline__ void corner_finish(const BwdParams &p, int n, int plane, int b) {
@@ -2012,7 +2013,16 @@ __device__ __forceinline__ void corner_finish(const BwdParams &p, int n, int pla
         if (p.msk_logit) mv = mask_value(mv, 1);
     }
     const SamplePos sp = sample_pos(y, x, p.H, p.W);
-    const f32x4 S = *reinterpret_cast<const f32x4 *>(p.csum + (((size_t)b * p.G * KK + plane) * N + n) * 4);
+    const float *cs4 = p.csum + (((size_t)b * p.G * KK + plane) * N + n) * 4;
+    f32x4 S = *reinterpret_cast<const f32x4 *>(cs4);
+    for (int k = 1; k < p.csum_n; k += 8) {
+        f32x4 v[8];  // eight planes in flight: there are few samples to hide a plane's latency behind
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            v[u] = k + u < p.csum_n ? *reinterpret_cast<const f32x4 *>(cs4 + (k + u) * p.csum_ps) : f32x4(0.0f);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) S += v[u];
+    }
     const float S0 = sp.vy0 && sp.vx0 ? S[0] : 0.0f, S1 = sp.vy0 && sp.vx1 ? S[1] : 0.0f;
     const float S2 = sp.vy1 && sp.vx0 ? S[2] : 0.0f, S3 = sp.vy1 && sp.vx1 ? S[3] : 0.0f;
     const float fly = sp.ly, flx = sp.lx, hy = 1.0f - fly, hx = 1.0f - flx;
@@ -2877,8 +2887,8 @@ __global__ __launch_bounds__(256) void finalize_gw_kernel(const GwFinal<T> f) {
 //                 contiguous in NCHW);
 //   then          the other boundary pixels (all of them for channels-last),
 //                 one thread per pixel and 4 padded channels;
-//   then          grad_offset / grad_mask of the fused kernel's groups of
-//                 several chunks (corner_finish), one thread per sample;
+//   then          grad_offset / grad_mask of groups that workgroups share
+//                 (corner_finish), one thread per sample;
 //   then          grad_weight / grad_bias (their accumulators are complete
 //                 when this kernel runs).
 struct RingFinal {
@@ -2887,7 +2897,7 @@ struct RingFinal {
     long nb_rows;         // blocks of the NCHW row part
     long items;           // items of the per-thread part
     long nb_items;        // its blocks
-    long nb_corner;       // blocks of the fused kernel's corner-sum finish (0: none)
+    long nb_corner;       // blocks of the corner-sum finish (0: none)
 };
 __device__ __forceinline__ f32x4 ring_sum(const BwdParams &p, int b, int g, int ci, int Y, int X) {
     constexpr int TS = kCellTile;
@@ -2988,8 +2998,8 @@ __global__ __launch_bounds__(256) void ring_final_kernel(const BwdParams p, cons
     }
     const long cb = blk - r.nb_rows - r.nb_items;
     if (cb < r.nb_corner) {
-        // grad_offset / grad_mask of groups of several chunks (csum is complete:
-        // the fused kernel ran before the grad_input kernels)
+        // grad_offset / grad_mask from the corner sums (csum is complete: the
+        // column-gradient kernel ran before the grad_input kernels)
         const int N = p.Ho * p.Wo, planes = p.G * p.kh * p.kw;
         const long sidx = cb * 256 + threadIdx.x;
         if (sidx < (long)p.B * planes * N) {
@@ -3007,7 +3017,6 @@ __global__ __launch_bounds__(256) void ring_final_kernel(const BwdParams p, cons
 // The fused kernel (column gradient and grad_weight in one pass) serves
 // 2-byte types with Mp of 128 or 256 (one M chunk), and images of gO and xt
 // below 2 GiB each; the launch also needs gO rows that take 16-byte loads.
-// Groups of several K chunks (Cgp > KC) add their corner sums up in csum.
 // Option DCN2_OPT_BWD_FUSED = 0 selects the two-kernel path for every shape
 // (the tests compare both paths).
 bool fused_bwd_shape(const Geo &g) {
@@ -3016,8 +3025,10 @@ bool fused_bwd_shape(const Geo &g) {
            (long long)g.H * g.W * g.cs * g.esz <= kGoOutOfRange;
 }
 
-bool csum_shape(const Geo &g) {
-    return g.dtype == DCN2_F32 ? g.Cgp > f32_chan_tile(g) : fused_bwd_shape(g) && g.Cgp > g.KC;
+int csum_planes(const Geo &g) {
+    const int tiles = g.Cgp / (g.dtype == DCN2_F32 ? f32_chan_tile(g) : g.KC);
+    if (tiles == 1 || (g.esz == 2 && !fused_bwd_shape(g))) return 0;
+    return g.esz == 2 && !go_padded(g) ? 1 : tiles;
 }
 
 template <typename T>
@@ -3124,7 +3135,7 @@ static hipError_t backward_t(const Geo &g, const BwdParams &p0, void *grad_input
         }
         // grad_offset / grad_mask of groups whose chunks several workgroups
         // share are finished from the corner sums by ring_final_kernel
-        if ((fused || sizeof(T) == 4) && csum_shape(g))
+        if ((fused || sizeof(T) == 4) && csum_planes(g) > 0)
             corner_blocks = ((long)g.B * g.G * g.KK * g.N + 255) / 256;
         prof_end(DCN2_STAGE_BWD_COLGRAD, s);
         // 3. grad_weight / grad_bias of the two-kernel path
@@ -3332,6 +3343,8 @@ hipError_t launch_backward(const Geo &g, const void *xt, const void *wt, const v
     p.cgm = cgm;
     p.rsc = (unsigned char *)rsc;
     p.csum = csum;
+    p.csum_n = csum_planes(g);
+    p.csum_ps = p.csum_n > 1 ? (size_t)g.B * g.G * g.KK * g.N * 4 : 0;
     p.rec = (BucketRec *)rec;
     p.bcnt = bcnt;
     p.bstart = bstart;

@@ -60,7 +60,7 @@ __global__ __launch_bounds__(256) void dcn2_colgrad_f32_kernel(const CgF32Params
     struct Px {
         uint32_t off[4];
         float m, ly, lx;
-        int valid, row, cs, pad0, pad1;
+        int valid, row, pad[3];
     };
     constexpr size_t kG = sizeof(float) * 2 * kCgM * LDG, kC = sizeof(float) * NT * LDC;
     __shared__ __attribute__((aligned(16))) char smem[kG > kC ? kG : kC];
@@ -131,7 +131,7 @@ __global__ __launch_bounds__(256) void dcn2_colgrad_f32_kernel(const CgF32Params
 
     // thread's pixel of the consumers' descriptors
     float f_m = 0.0f, f_ly = 0.0f, f_lx = 0.0f;
-    int f_b = 0, f_nn = 0;
+    int f_b = 0, f_nn = 0, f_smp = 0;
     if (tid < NT) {
         const bool live = tid < live_px;
         const unsigned n = n0 + (live ? tid : 0), b = n / (unsigned)N;
@@ -143,7 +143,7 @@ __global__ __launch_bounds__(256) void dcn2_colgrad_f32_kernel(const CgF32Params
         const float x = (float)(ox * p.sw - p.pw + tap % p.kw * p.dw) + off[N];
         f_m = p.mask ? mask_value(((const float *)p.mask)[f_b * p.msk_bs + (size_t)plane * N + f_nn], p.msk_logit)
                      : 1.0f;
-        const int smp = (f_b * p.G * KK + plane) * N + f_nn;
+        f_smp = (f_b * p.G * KK + plane) * N + f_nn;
         const SamplePos sp = sample_pos(y, x, p.H, p.W);
         f_ly = sp.ly;
         f_lx = sp.lx;
@@ -155,10 +155,9 @@ __global__ __launch_bounds__(256) void dcn2_colgrad_f32_kernel(const CgF32Params
         d.off[2] = sp.vy1 && sp.vx0 ? base + row : c.x_bytes;
         d.off[3] = sp.vy1 && sp.vx1 ? base + row + cs : c.x_bytes;
         d.m = f_m;
-        d.row = live ? p.sidx[smp] : -1;
-        d.cs = live ? smp : -1;
+        d.row = live ? p.sidx[f_smp] : -1;
         d.ly = d.lx = 0.0f;
-        d.valid = d.pad0 = d.pad1 = 0;
+        d.valid = d.pad[0] = d.pad[1] = d.pad[2] = 0;
         sP[tid] = d;
     }
 
@@ -230,10 +229,11 @@ __global__ __launch_bounds__(256) void dcn2_colgrad_f32_kernel(const CgF32Params
     }
     __syncthreads();
     if (c.cpg > 1) {
-        // the group's channel tiles add their corner sums up
-        for (int i = tid; i < NT * 4; i += 256)
-            if (const int smp = sP[i >> 2].cs; smp >= 0)
-                unsafeAtomicAdd(p.csum + (size_t)smp * 4 + (i & 3), sS[i >> 2][i & 3]);
+        // each of the group's channel tiles stores its part in a plane of its own:
+        // added up with atomics, whose order varies, grad_offset and grad_mask of
+        // fp32 would differ in their last bits from run to run
+        if (tid < live_px)
+            *reinterpret_cast<f32x4 *>(p.csum + cc * p.csum_ps + (size_t)f_smp * 4) = sS[tid];
         return;
     }
     if (tid < live_px) {

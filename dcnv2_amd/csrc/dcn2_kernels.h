@@ -152,11 +152,14 @@ hipError_t launch_backward(const Geo &g, const void *xt, const void *wt, const v
                            float *gi_acc, float *gw_acc, float *gb_acc, void *cgm, void *rsc,
                            float *csum, void *rec, int *bcnt, int *bstart, int *bcur, int *sidx,
                            float *ring, const void *gop, bool last, hipStream_t s);
-// Whether the fused backward kernel may serve g (2-byte type, Cout <= 256),
-// and whether its column-gradient kernel (the fused one, or the fp32 one) needs
-// the corner-sum buffer (a group's channels shared by several workgroups).
+// Whether the fused backward kernel may serve g (2-byte type, Cout <= 256).
 bool fused_bwd_shape(const Geo &g);
-bool csum_shape(const Geo &g);
+// Planes [B][G*KK][N][4] of the corner-sum buffer: 0 where one workgroup sums all
+// channels of a group; else one per channel tile of a group, each stored by its own
+// workgroup, so that grad_offset and grad_mask are repeatable bit for bit.  The fused
+// kernel on a grad_output read in place adds its chunks up in one plane with atomics:
+// 16 bytes a sample however many they are, not repeatable.
+int csum_planes(const Geo &g);
 // Channels of one fp32 backward workgroup: two chunks of a group where they
 // pair up (and lie in one weight group), else one.
 inline int f32_chan_tile(const Geo &g) {

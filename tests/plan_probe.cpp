@@ -23,7 +23,7 @@ hipError_t launch_backward(const Geo &g, const void *, const void *, const void 
                            float *, const void *, bool, hipStream_t) {
     const GatherGeo gg = gather_geometry(g);
     auto room = [](const void *a, const void *b) { return (long)((const char *)b - (const char *)a); };
-    const long sums = csum_shape(g) ? (long)g.B * g.G * g.KK * g.N * 16 : 0;
+    const long sums = (long)csum_planes(g) * g.B * g.G * g.KK * g.N * 16;
     printf("%d %d  %ld %ld  %ld %ld  %ld %ld  %ld %ld\n", g.B, g.by_cells, gg.acc_bytes, room(gi_acc, gw_acc),
            gg.rows * g.Cgp * gg.row_esz, room(cgm, rsc), sums, room(csum, rec), gg.rows * 12, room(rec, bcnt));
     return hipSuccess;
