@@ -681,17 +681,34 @@ static bool ws_two_waves_per_simd() {
     return ok;
 }
 
-// The tile kernels serve this kernel's shapes when it would have few tiles (of 128
-// pixels of one image x 256 rows, or 128 up to 128 rows) per launch, or a register
-// count that would let three waves share a SIMD.
-// Measured (us, this kernel against those, fp16 3x3): 53.8 against 45.4 at 128 tiles
-// (Cout 256, C 256), 56.0 against 61.2 at 192; 27.2 against 20.5 at 128 (Cout 128, C
-// 128), 29.6 against 32.8 at 256; 19.9 against 14.0 at 128 (Cout 64, C 64), 33.2
-// against 38.6 at 512.
-constexpr int kWsMinTiles = 160;
-static bool ws_few_tiles(const Geo &g) {
-    const int rows = std::min(g.gsplit ? g.Cout / g.WG : g.Cout, kBiasRows);
-    if ((long long)g.B * ceil_div(g.N, 128) * ceil_div(rows, rows > 128 ? 256 : 128) < kWsMinTiles) return true;
+// Few tiles of this kernel (128 pixels of one image x 256 rows, or 128 up to 128 rows)
+// per launch: the tile kernels are faster.  The line, for this card's 256 CUs; ratios
+// are this kernel's time over theirs, 16 x (8 to 1264) maps, one image:
+//   128 tiles in general, up to which the tile kernels' half-sized tiles give each CU
+//     one: 1.09 / 0.86 at 128 / 132 tiles (fp16 3x3, C 128, Cout 256), 1.24 / 0.84 (7x7,
+//     Cout 128), 1.03 / 0.88 (3x3, C 64, Cout 512), 1.15 / 0.86 (bf16 5x5, C 128, Cout 512);
+//   159 where this kernel stores slowly and K is short: outputs whose rows 16-byte pieces
+//     cannot cover, up to 5x5 (1.2-1.7 at 132-158 tiles of 1x1, 1.05-1.3 at 3x3, 0.95-1.11
+//     at 5x5, 0.88-1.02 at 7x7), channels-last up to 3x3 (1.1-1.5 at 1x1, 0.98-1.14 at 3x3,
+//     0.88-1.09 at 5x5) and NCHW 1x1 up to 64 rows (1.10-1.20; 0.94-1.07 at 3x3);
+//   80 for NCHW 1x1 of one chunk and more than 128 rows (1.00 at 72, 0.95 at 96);
+//   64 up to 64 rows where each of more than 16 chunks has its own offsets and corners
+//     (7x7, C 64, Cout 64: 1.87 / 0.87 at 64 / 72 tiles; 5x5: 1.79 / 0.92; at 9 chunks
+//     still 1.03, and at C 128, two chunks to a set of corners, 1.04-1.10).
+bool forward_few_tiles(const Geo &g) {
+    const int rows = std::min(g.gsplit ? g.Cout / g.WG : g.Cout, kBiasRows), nch = g.KK * g.cpw;
+    const bool vec = g.out_nhwc ? g.Cout % 8 == 0 : g.N % 8 == 0;
+    int most = 128;
+    if (!vec ? g.KK <= 25 : g.out_nhwc ? g.KK <= 9 : rows <= 64 && g.KK == 1) most = 159;
+    else if (vec && rows <= 64 && g.Cgp == g.KC && nch > 16) most = 64;
+    else if (vec && rows > 128 && !g.out_nhwc && nch == 1) most = 80;
+    return (long long)g.B * ceil_div(g.N, 128) * ceil_div(rows, rows > 128 ? 256 : 128) <= most;
+}
+
+// The tile kernels serve this kernel's shapes when it would have few tiles, or a
+// register count that would let three waves share a SIMD.
+static bool ws_unfit(const Geo &g) {
+    if (forward_few_tiles(g)) return true;
     return g.dtype == DCN2_F16 ? !(ws_two_waves_per_simd<f16, 1>() && ws_two_waves_per_simd<f16, 2>())
                                : !(ws_two_waves_per_simd<bf16, 1>() && ws_two_waves_per_simd<bf16, 2>());
 }
@@ -742,7 +759,7 @@ hipError_t launch_forward(const Geo &g, const void *xt, const void *wp, const vo
                           const void *offset, const void *mask, const void *bias, void *out,
                           hipStream_t s) {
     if (g.B == 0) return hipSuccess;
-    if (g.dtype == DCN2_F32 || ws_few_tiles(g))
+    if (g.dtype == DCN2_F32 || ws_unfit(g))
         return launch_forward_tiles(g, xt, wp, tab, offset, mask, bias, out, s);
     FwdParams p;
     p.xt = xt;

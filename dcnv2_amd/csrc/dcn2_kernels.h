@@ -129,6 +129,9 @@ hipError_t launch_forward(const Geo &g, const void *xt, const void *wp, const vo
                           const void *offset, const void *mask, const void *bias, void *out,
                           hipStream_t s);
 
+// Whether a 2-byte forward has so few tiles that the small ones are faster.
+bool forward_few_tiles(const Geo &g);
+
 // dcn2_forward_tiles.hip: small tiles over the batch's pixels; every fp32 forward
 // and the 2-byte ones of few tiles (launch_forward calls it).
 hipError_t launch_forward_tiles(const Geo &g, const void *xt, const void *wp, const void *tab,

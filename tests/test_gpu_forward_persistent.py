@@ -29,6 +29,17 @@ SHAPES = [
     # just below either: the small tiles
     (47, 64, 8, 3, 136, 3, 1, 1, 1, False, True),
     (159, 16, 4, 4, 64, 3, 1, 1, 1, False, True),
+    # the role-specialised kernel from fewer tiles: 129; 65 up to 64 rows, 25 chunks of
+    # one plane; 81 at 1x1, one chunk, more than 128 rows; 160 where it stores slowly
+    (129, 40, 4, 4, 72, 3, 1, 1, 1, False, True),
+    (128, 40, 4, 4, 72, 3, 1, 1, 1, False, True),
+    (65, 64, 4, 4, 48, 5, 1, 1, 1, False, True),
+    (64, 64, 4, 4, 48, 5, 1, 1, 1, False, True),
+    (81, 33, 4, 6, 136, 1, 1, 1, 1, False, True),
+    (80, 33, 4, 6, 136, 1, 1, 1, 1, False, False),
+    (160, 24, 5, 3, 40, 3, 1, 1, 1, False, True),
+    (159, 24, 5, 3, 40, 3, 1, 1, 1, False, True),
+    (159, 24, 4, 4, 40, 3, 1, 1, 1, True, True),
 ]
 
 

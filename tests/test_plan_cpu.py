@@ -1,6 +1,7 @@
 """What the library's host code plans for a call, read on the CPU through
 ``plan_probe.cpp``: every slice of a backward call uses no more of the workspace than
-its layout holds, and all slices take the same grad_input kernel."""
+its layout holds, and all slices take the same grad_input kernel; the forward kernel on
+either side of the lines between them."""
 import glob
 import os
 import subprocess
@@ -11,7 +12,7 @@ from dcnv2_amd import build
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 DEFAULT_BUDGET = 192 << 20
-F32, F16 = 0, 1
+F32, F16, BF16 = 0, 1, 2
 
 
 @pytest.fixture(scope="module")
@@ -29,13 +30,14 @@ def probe(tmp_path_factory):
     def run(budget, push, desc):
         r = subprocess.run([exe], input=" ".join(str(v) for v in (budget, push, *desc)), text=True,
                            capture_output=True, check=True)
-        return [[int(v) for v in ln.split()] for ln in r.stdout.splitlines() if ln]
+        rows = [[int(v) for v in ln.split()] for ln in r.stdout.splitlines() if ln]
+        return rows[0], rows[1:]
 
     return run
 
 
-def _desc(dtype, B, C, H, W, Cout, k, dg=1):
-    return (B, C, H, W, Cout, k, k, 1, 1, k // 2, k // 2, 1, 1, dg, dtype, 1, 0, 0)
+def _desc(dtype, B, C, H, W, Cout, k, dg=1, wg=1, nhwc=0):
+    return (B, C, H, W, Cout, k, k, 1, 1, k // 2, k // 2, 1, 1, dg, dtype, wg, nhwc, nhwc)
 
 
 # The last slice is shorter than the others, so that it alone has fewer than 128
@@ -48,7 +50,7 @@ def _desc(dtype, B, C, H, W, Cout, k, dg=1):
     ((F16, 11, 64, 47, 47, 64, 7, 2), (4, 4, 3), 18), # 72: by pixels throughout
 ], ids=str)
 def test_short_last_slice_keeps_the_kernel(probe, case, slices, pairs):
-    got = probe(DEFAULT_BUDGET, -1, _desc(*case))
+    _, got = probe(DEFAULT_BUDGET, -1, _desc(*case))
     assert tuple(r[0] for r in got) == slices
     assert {r[1] for r in got} == {int(slices[0] * pairs >= 128)}
     for r in got:
@@ -63,8 +65,26 @@ def test_slices_fit_their_layout(probe):
         for B in range(1, 24, 2):
             for budget in (16 << 20, 100 << 20, DEFAULT_BUDGET):
                 for push in (-1, 0, 1):
-                    got = probe(budget, push, _desc(case[0], B, *case[1:]))
+                    _, got = probe(budget, push, _desc(case[0], B, *case[1:]))
                     assert sum(r[0] for r in got) == B and len({r[1] for r in got}) == 1
                     assert push < 0 or got[0][1] == push
                     for r in got:
                         assert all(need <= room for need, room in zip(r[2::2], r[3::2]))
+
+
+# The lines as measured (see forward_few_tiles): tiles of 128 pixels x 256 rows (128 up to
+# 128 rows), one image of 16 pixels a row (15 where rows are ragged) to a tile.
+@pytest.mark.parametrize("C,Cout,k,nhwc,ragged,wg,most", [
+    (128, 256, 3, 0, False, 1, 128), (128, 128, 7, 0, False, 1, 128), (64, 512, 3, 0, False, 1, 64),
+    (256, 256, 5, 1, False, 1, 128), (128, 100, 3, 1, False, 1, 159), (64, 256, 1, 1, False, 1, 159),
+    (64, 64, 1, 0, False, 1, 159), (64, 64, 3, 0, False, 1, 128), (64, 64, 5, 0, False, 1, 64),
+    (64, 40, 7, 1, False, 1, 64), (128, 64, 7, 0, False, 1, 128), (64, 256, 1, 0, False, 1, 80),
+    (65, 256, 1, 0, False, 1, 128), (64, 256, 5, 0, True, 1, 159), (64, 64, 7, 0, True, 1, 128),
+    (256, 256, 3, 0, False, 2, 128),
+])
+def test_few_tiles_of_the_16_bit_forward(probe, C, Cout, k, nhwc, ragged, wg, most):
+    for dtype in (F16, BF16):
+        for B in (most, most + 1):
+            rows, few = probe(DEFAULT_BUDGET, -1, _desc(dtype, B, C, 7, 15 if ragged else 16, Cout, k,
+                                                        wg=wg, nhwc=nhwc))[0]
+            assert few == (B == most)
