@@ -543,12 +543,14 @@ void dcn2_fwd_rw_kernel(const RwParams p) {
     for (int it = 0; it < 8; it += 2) flush_out(prv, it);
 }
 
-// Fewer than 48 tiles of 128 pixels leave most CUs without one, and each workgroup
-// first loads the whole weight: dcn2_forward_tiles.hip takes them (us, this kernel
-// against that, Cout 256, C 64: 13.6 / 10.9 at 8 tiles, 14.2 / 11.8 at 32, 14.9 / 15.3
-// at 64).
+// Few tiles of 128 pixels leave most CUs without one, and each workgroup first loads the
+// whole weight: dcn2_forward_tiles.hip takes them, up to 32 for NCHW (its 128 x 32 tiles
+// then give each CU one) and 47 for a channels-last output, which this kernel stores more
+// slowly.  us, pack and forward, this kernel / that, Cout 256, C 64: NCHW 14.9 / 11.6 at 4
+// tiles, 15.5 / 13.6 at 32, 15.2 / 15.7 at 34, 15.5 / 16.0 at 46; channels-last 15.1 / 12.5 at
+// 32, 15.3 / 14.9 at 46.
 bool rw_eligible(const Geo &g) {
-    if ((long long)g.B * ceil_div(g.N, 128) < 48) return false;
+    if ((long long)g.B * ceil_div(g.N, 128) <= (g.out_nhwc ? 47 : 32)) return false;
     return g.dtype == DCN2_F16 && g.G == 1 && g.Cgp == 64 && g.KK == kRwTaps && g.Mp == 256 &&
            g.WG == 1 && (g.out_nhwc ? g.Cout % 8 == 0 : g.N % 8 == 0) &&
            (long long)g.Cout * g.N * 2 < 0x7fffffffLL;

@@ -26,6 +26,10 @@ SHAPES = [
     (50, 64, 8, 3, 129, 3, 1, 1, 1, False, True),
     (49, 5, 4, 6, 256, 3, 1, 1, 1, True, False),
     (51, 33, 9, 8, 200, 3, 1, 1, 1, False, False),
+    (33, 64, 4, 4, 136, 3, 1, 1, 1, False, True),    # (from 33 tiles for NCHW)
+    (32, 64, 4, 4, 136, 3, 1, 1, 1, False, True),
+    (48, 64, 4, 5, 136, 3, 1, 1, 1, True, True),
+    (47, 64, 4, 5, 136, 3, 1, 1, 1, True, True),
     # just below either: the small tiles
     (47, 64, 8, 3, 136, 3, 1, 1, 1, False, True),
     (159, 16, 4, 4, 64, 3, 1, 1, 1, False, True),

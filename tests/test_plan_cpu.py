@@ -88,3 +88,10 @@ def test_few_tiles_of_the_16_bit_forward(probe, C, Cout, k, nhwc, ragged, wg, mo
             rows, few = probe(DEFAULT_BUDGET, -1, _desc(dtype, B, C, 7, 15 if ragged else 16, Cout, k,
                                                         wg=wg, nhwc=nhwc))[0]
             assert few == (B == most)
+
+
+def test_few_tiles_of_the_resident_weight_forward(probe):
+    for nhwc, most in ((0, 32), (1, 47)):
+        for B in (most, most + 1):
+            rw, few = probe(DEFAULT_BUDGET, -1, _desc(F16, B, 64, 8, 16, 256, 3, nhwc=nhwc))[0]
+            assert rw == (B > most) and few == 1
