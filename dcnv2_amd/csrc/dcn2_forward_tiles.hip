@@ -407,23 +407,25 @@ static hipError_t forward_tiles(const Geo &g, const void *xt, const void *wp, co
             p.cb = w * p.cpw;
             p.m_base = w * rows;
             p.m_end = p.m_base + rows;
-            // Tile rule, measured in us (rows, K, pixels; tile: rows x pixels, all with
+            // Tile rule for this card's 256 CUs, measured in us (rows, K, pixels; tile: rows x pixels, all with
             // 8 waves and one or two workgroups to a CU unless noted):
             //   64x32, K over 4 groups of waves, while one workgroup to a CU does: fp16
             //     13.5 against 16.2 (128x32) at 128, 1152, 4096; 32 against 39 at 512,
             //     4608, 1024; fp32 9.6 against 11.6 at 32, 288, 1024.  Past that 38
             //     against 24 at 256, 2304, 2100.
-            //   128x32, K over 2, while two and a half do: fp16 33 against 43 (256x64)
-            //     at 256, 2304, 8192, but 60 against 45 at 16384; fp32 50.7 against 79.9
-            //     at 256, 1024, 6272.
+            //   128x32, K over 2, while two and a half do: fp32 50.7 against 79.9 (256x64)
+            //     at 256, 1024, 6272; 16 bits, more than 128 rows and 8 chunks: two, fp16
+            //     38.2 at 256, 2304, 8192 but past that 52.3 against 48.9 at 8704, 77.8 /
+            //     72.5 at 512, 3136, 4352 and 115.7 / 97.8 at 1000, 4800, 2176.
             //   256x64 (a pixel is sampled once for 256 rows): fp32 64.7 against 71.1
             //     for 128x64 at 256, 64, 100352; 48.7 against 51.7 at 2048, 512, 1568.
             //   128x64 and 64x64 (4 waves): the rest, whose rows 256x64 would pad.
             auto tiles = [&](int bm, int bn) { return (long long)ceil_div(rows, bm) * ceil_div(p.total, bn); };
+            const int most = sizeof(T) == 2 && rows > 128 && p.nch > 8 ? 512 : 640;
             hipError_t e;
             if (tiles(64, 32) <= 256)
                 e = launch_tile<T, 1, 1, 2, 1, 4>(p, rows, g.out_nhwc, s);
-            else if (rows > 64 && tiles(128, 32) <= 640)
+            else if (rows > 64 && tiles(128, 32) <= most)
                 e = launch_tile<T, 1, 1, 4, 1, 2>(p, rows, g.out_nhwc, s);
             else if (rows > 128)
                 e = launch_tile<T, 1, 2, 8, 1, 1>(p, rows, g.out_nhwc, s);
