@@ -57,3 +57,34 @@ def test_backward_f32_tiles(shape):
         # 2^-24 per rounding over at most 50000 additions in any order: a random
         # walk of 224 * 2^-24 = 1.4e-5 of a result, against the largest one
         check(name, a, r, 2e-5)
+
+
+def test_channels_last_costs_no_more_than_nchw():
+    """grad_bias of a channels-last grad_output: with an atomic per load in place of one
+    per row and workgroup this layer took 2.2 times the time of its NCHW form (now 1.0;
+    the bound leaves room for a busy machine)."""
+    g = torch.Generator().manual_seed(1)
+    B, C, H, W, Cout = 5, 28, 42, 86, 91
+    x, go = torch.randn(B, C, H, W, generator=g).cuda(), torch.randn(B, Cout, H, W, generator=g).cuda()
+    w, b = torch.randn(Cout, C, 1, 1, generator=g).cuda(), torch.randn(Cout, generator=g).cuda()
+    off, mask = torch.randn(B, 4, H, W, generator=g).cuda(), torch.rand(B, 2, H, W, generator=g).cuda()
+
+    def run(fmt):
+        xs, gs = x.contiguous(memory_format=fmt), go.contiguous(memory_format=fmt)
+        times = []
+        for _ in range(8):
+            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            e0.record()
+            for _ in range(20):
+                grads = _C.dcn_v2_backward(xs, w, mask, off, b, gs, 1, 1, 0, 0, 1, 1, 2)
+            e1.record()
+            e1.synchronize()
+            times.append(e0.elapsed_time(e1))
+        return min(times), grads[4]
+
+    t0, gb0 = run(torch.contiguous_format)
+    t1, gb1 = run(torch.channels_last)
+    ref = go.double().sum((0, 2, 3)).cpu()
+    check("grad_bias", gb0, ref, TOL[torch.float32])
+    check("grad_bias (channels_last)", gb1, ref, TOL[torch.float32])
+    assert t1 < 1.6 * t0
