@@ -8,7 +8,7 @@ import torch
 from dcnv2_amd import _C
 from oracle import oracle
 
-from util import GRADS, check
+from util import GRADS, TOL, check
 
 pytestmark = pytest.mark.gpu
 
