@@ -38,6 +38,24 @@ int fail(int code, const char *fmt, ...) {
 
 static size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
+// grad_output whose rows 16-byte loads cannot read whatever its address (NCHW with
+// N % 8, or channels-last with Cout % 8): the backward reads a padded NCHW copy,
+// so that the kernels with 16-byte loads (the fused one among them) serve it too.
+// Measured at bf16 3x3, C 256 -> 256, 2 x 25 x 42 (N = 1050): 32 us in the fused
+// kernel against 118 + 47 in the two that read such rows by elements; the copy
+// adds 2 us to the pack launch.  Above 256 rows, which the fused kernel does not
+// hold, whole backwards went 1661.8 -> 855.3 (C 256 -> 300, 3x3, 8 x 55 x 55) and
+// 358.1 -> 231.2 (256 -> 513, 1x1); only a single chunk of K over few NCHW pixels does
+// not earn the copy of more than 512 rows back: 89.8 against 109.6 at 1x1, 64 ->
+// 1001, 7 x 85 x 13 (63 tiles of 128 pixels), 125.1 / 148.6 at 64 -> 2047, 55 x 55 (24),
+// but 117.6 / 116.9 at 64 -> 1001, 111 x 111 (97) and 246.3 / 214.8 at 8 x 55 x 55 (192).
+// (Of the whole call, so that all slices agree on it and on the workspace.)
+static bool pads_grad_output(const Geo &g) {
+    if (g.esz != 2 || (g.out_nhwc ? g.Cout : g.N) % 8 == 0) return false;
+    if ((long long)g.Cout * go_pitch(g) * g.esz > kGoMaxBytes) return false;
+    return g.out_nhwc || g.Cout <= 512 || g.Kp > g.KC || (long long)g.B * ceil_div(g.N, 128) >= 96;
+}
+
 // Validates `d` and derives the packing geometry.  Returns DCN2_OK or an error.
 int make_geo(const dcn2_desc *d, Geo &g) {
     if (!d) return fail(DCN2_EINVAL, "dcn2: null descriptor");
@@ -111,6 +129,7 @@ int make_geo(const dcn2_desc *d, Geo &g) {
         (long long)g.B * g.G * g.KK * g.Ho * g.Wo >= lim || g.H > 32767 || g.W > 32767)
         return fail(DCN2_ERANGE, "dcn2: problem exceeds the 32-bit per-image index range");
     g.Kp = (int)Kp;
+    g.go_pad = pads_grad_output(g) ? 1 : 0;
     // weight-group walk (see Geo::gsplit): every chunk (deformable group dg,
     // channel chunk cc) must lie inside the group q / cpw of its index q in
     // the tap
@@ -222,7 +241,7 @@ BwdWorkspace bwd_workspace(const Geo &g0) {
         o += ring_bytes;
     }
     w.gop = o;
-    if (go_padded(g)) o += align256((size_t)g.B * g.Cout * go_pitch(g) * g.esz);
+    if (g.go_pad) o += align256((size_t)g.B * g.Cout * go_pitch(g) * g.esz);
     w.total = o;
     return w;
 }
@@ -366,7 +385,7 @@ static int backward_impl(const Geo &g0, const void *input, const void *weight, c
         prof_begin(DCN2_STAGE_BWD_PACK, s);
         if ((rc = check_launch(launch_pack(gs, g.xt_direct ? nullptr : in_s, (void *)xt,
                                            first ? weight : nullptr, wt, tab, true, s, &clr,
-                                           gs.B > 0 && go_padded(gs) ? at(grad_output, go_img) : nullptr,
+                                           gs.B > 0 && gs.go_pad ? at(grad_output, go_img) : nullptr,
                                            base + ws.gop),
                                "pack")))
             return rc;

@@ -3028,7 +3028,7 @@ bool fused_bwd_shape(const Geo &g) {
 int csum_planes(const Geo &g) {
     const int tiles = g.Cgp / (g.dtype == DCN2_F32 ? f32_chan_tile(g) : g.KC);
     if (tiles == 1 || (g.esz == 2 && !fused_bwd_shape(g))) return 0;
-    return g.esz == 2 && !go_padded(g) ? 1 : tiles;
+    return g.esz == 2 && !g.go_pad ? 1 : tiles;
 }
 
 template <typename T>
@@ -3105,7 +3105,7 @@ static hipError_t backward_t(const Geo &g, const BwdParams &p0, void *grad_input
     do {                                                                                    \
         constexpr bool F16 = std::is_same<T, f16>::value;                                   \
         if (p.go_nhwc) dcn2_bwd_fused_kernel<T, true, MPV, F16><<<grid, 512, 0, s>>>(pf);  \
-        else if (go_padded(g)) dcn2_bwd_fused_kernel<T, false, MPV, false><<<grid, 512, 0, s>>>(pf); \
+        else if (g.go_pad) dcn2_bwd_fused_kernel<T, false, MPV, false><<<grid, 512, 0, s>>>(pf); \
         else dcn2_bwd_fused_kernel<T, false, MPV, F16><<<grid, 512, 0, s>>>(pf);           \
     } while (0)
                     if (g.Mp == 256) DCN2_FUSED(256);
@@ -3305,7 +3305,7 @@ hipError_t launch_backward(const Geo &g, const void *xt, const void *wt, const v
     p.tab = tab;
     p.offset = offset;
     p.mask = mask;
-    const bool padded = go_padded(g);  // (copied by the pack launch)
+    const bool padded = g.go_pad;  // (copied by the pack launch)
     p.gout = padded ? gop : grad_out;
     p.goff = grad_offset;
     p.gmask = grad_mask;

@@ -50,6 +50,8 @@ struct Geo {
     // whether grad_input goes by cells: one decision for all slices of a call,
     // which also lays out their common workspace (plan_backward).
     int Bs, by_cells;
+    // The backward reads a padded NCHW copy of grad_output (pads_grad_output).
+    int go_pad;
 };
 
 // dcn2_api.cpp: the descriptor check shared by every entry point, the forward
@@ -106,23 +108,15 @@ struct ClearList {
     size_t n[kClearBufs];
 };
 // With `go`, it also copies the 2-byte grad_output of g.B images to `gop`, NCHW with
-// rows of go_pitch(g) elements, zeros past the N pixels (see go_padded).
+// rows of go_pitch(g) elements, zeros past the N pixels (see Geo::go_pad).
 hipError_t launch_pack(const Geo &g, const void *input, void *xt, const void *weight, void *wp,
                        void *tab, bool transpose, hipStream_t s, const ClearList *clear = nullptr,
                        const void *go = nullptr, void *gop = nullptr);
 
-// grad_output whose rows 16-byte loads cannot read whatever its address (NCHW with
-// N % 8, or channels-last with Cout % 8): the backward reads a padded NCHW copy,
-// so that the kernels with 16-byte loads (the fused one among them) serve it too.
-// Measured at bf16 3x3, C 256 -> 256, 2 x 25 x 42 (N = 1050): 32 us in the fused
-// kernel against 118 + 47 in the two that read such rows by elements; the copy
-// adds 2 us to the pack launch.
-constexpr long long kGoMaxBytes = 0x7ffffff0;  // one image of grad_output those kernels address
+// Elements of a row of the padded copy of grad_output (Geo::go_pad), and the bytes of
+// one image of grad_output that the kernels with 16-byte loads address.
+constexpr long long kGoMaxBytes = 0x7ffffff0;
 inline int go_pitch(const Geo &g) { return (g.N + 7) / 8 * 8; }
-inline bool go_padded(const Geo &g) {
-    return g.esz == 2 && (g.out_nhwc ? g.Cout : g.N) % 8 != 0 &&
-           (long long)g.Cout * go_pitch(g) * g.esz <= kGoMaxBytes;
-}
 
 // dcn2_forward.hip
 hipError_t launch_forward(const Geo &g, const void *xt, const void *wp, const void *tab,

@@ -13,7 +13,7 @@
 // Blocks [0, nw) pack 256 16-byte pieces of the weight each; blocks
 // [nw, nw + nin) transpose 64 pixels x CT channels of the input each (CT*esz
 // = 128 bytes, one channel chunk of a pixel); the rest clear accumulators and copy
-// grad_output rows that need padding (go_padded).
+// grad_output rows that need padding (Geo::go_pad).
 // The halves are independent, so the (small, latency bound) weight packing,
 // dispatched first, overlaps the (bandwidth bound) input transpose.
 #include "dcn2_common.h"
@@ -38,7 +38,7 @@ struct PackParams {
     float4 *clr[kClearBufs];       // buffers to zero, 16-byte pieces each
     long clr_n4[kClearBufs];
     int clr_blk[kClearBufs + 1];   // first clearing block of each buffer (prefix sums)
-    const void *go;                // grad_output to copy in padded rows (go_padded), and its copy
+    const void *go;                // grad_output to copy in padded rows (Geo::go_pad), and its copy
     void *gop;
     int N, go_nhwc;
     long ngo;                      // its 16-byte pieces, 256 to a block

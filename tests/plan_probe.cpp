@@ -2,8 +2,8 @@
 // library's objects, the launchers defined here take the place of its own.
 //
 // Each input line: slice budget, option gi_push, the 18 fields of a dcn2_desc.
-// First one line: whether the forward keeps the weight in registers, and whether it is
-// one of few tiles.  Then per backward slice one line: images, whether grad_input goes by cells, and for
+// First one line: whether the forward keeps the weight in registers, whether it is one of
+// few tiles, and whether the backward reads a padded copy of grad_output.  Then per backward slice one line: images, whether grad_input goes by cells, and for
 // gi_acc, the hand-off rows, the corner sums and the records the bytes that the slice
 // uses and those that the workspace holds for it.
 #include <cstdio>
@@ -43,7 +43,7 @@ int main() {
         dcn2_set_option(DCN2_OPT_GI_PUSH, push);
         dcn2::Geo g;
         if (dcn2::make_geo(&d, g)) return 3;
-        printf("%d %d\n", g.rw, (int)dcn2::forward_few_tiles(g));
+        printf("%d %d %d\n", g.rw, (int)dcn2::forward_few_tiles(g), g.go_pad);
         char *const p = (char *)0x10000;  // (never read: nothing is launched)
         const int rc = dcn2_backward(&d, p, p, p, p, p, p, p, p, p, p, p, dcn2_backward_workspace_bytes(&d), nullptr);
         if (rc) return fprintf(stderr, "%s\n", dcn2_last_error()), 3;

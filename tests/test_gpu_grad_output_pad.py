@@ -21,6 +21,10 @@ SHAPES = [(2, 64, 1, n, 40, 1, 1, False, False) for n in range(1, 8)] + \
         (2, 64, 7, 9, 301, 1, 1, True, False),
         (5, 64, 15, 17, 72, 3, 1, False, True),
         (5, 64, 15, 17, 70, 3, 1, True, True),
+        # more than 512 rows and one chunk: read in place below 96 tiles of 128 pixels,
+        # in slices too
+        (3, 40, 5, 7, 514, 1, 1, False, False),
+        (96, 8, 3, 3, 514, 1, 1, False, True),
     ]
 
 

@@ -85,7 +85,7 @@ def test_slices_fit_their_layout(probe):
 def test_few_tiles_of_the_16_bit_forward(probe, C, Cout, k, nhwc, ragged, wg, most):
     for dtype in (F16, BF16):
         for B in (most, most + 1):
-            rows, few = probe(DEFAULT_BUDGET, -1, _desc(dtype, B, C, 7, 15 if ragged else 16, Cout, k,
+            _, few, _ = probe(DEFAULT_BUDGET, -1, _desc(dtype, B, C, 7, 15 if ragged else 16, Cout, k,
                                                         wg=wg, nhwc=nhwc))[0]
             assert few == (B == most)
 
@@ -93,5 +93,16 @@ def test_few_tiles_of_the_16_bit_forward(probe, C, Cout, k, nhwc, ragged, wg, mo
 def test_few_tiles_of_the_resident_weight_forward(probe):
     for nhwc, most in ((0, 32), (1, 47)):
         for B in (most, most + 1):
-            rw, few = probe(DEFAULT_BUDGET, -1, _desc(F16, B, 64, 8, 16, 256, 3, nhwc=nhwc))[0]
+            rw, few, _ = probe(DEFAULT_BUDGET, -1, _desc(F16, B, 64, 8, 16, 256, 3, nhwc=nhwc))[0]
             assert rw == (B > most) and few == 1
+
+
+def test_padded_grad_output(probe):
+    def pad(*a, **kw):
+        return probe(DEFAULT_BUDGET, -1, _desc(*a, **kw))[0][2]
+
+    assert not pad(F32, 2, 64, 9, 9, 64, 1) and not pad(F16, 2, 64, 8, 9, 60, 1)  # fp32; N % 8 == 0
+    assert pad(F16, 1, 64, 9, 9, 512, 1) and not pad(F16, 1, 64, 9, 9, 513, 1)   # one chunk of K
+    assert pad(F16, 1, 65, 9, 9, 513, 1) and pad(F16, 1, 64, 9, 9, 513, 3)       # more
+    assert not pad(BF16, 95, 64, 9, 9, 513, 1) and pad(BF16, 96, 64, 9, 9, 513, 1)  # tiles of 128 pixels
+    assert pad(F16, 1, 64, 9, 9, 513, 1, nhwc=1) and not pad(F16, 1, 64, 9, 9, 520, 1, nhwc=1)
