@@ -687,21 +687,25 @@ static bool ws_two_waves_per_simd() {
 //   128 tiles in general, up to which the tile kernels' half-sized tiles give each CU
 //     one: 1.09 / 0.86 at 128 / 132 tiles (fp16 3x3, C 128, Cout 256), 1.24 / 0.84 (7x7,
 //     Cout 128), 1.03 / 0.88 (3x3, C 64, Cout 512), 1.15 / 0.86 (bf16 5x5, C 128, Cout 512);
-//   159 where this kernel stores slowly and K is short: outputs whose rows 16-byte pieces
-//     cannot cover, up to 5x5 (1.2-1.7 at 132-158 tiles of 1x1, 1.05-1.3 at 3x3, 0.95-1.11
-//     at 5x5, 0.88-1.02 at 7x7), channels-last up to 3x3 (1.1-1.5 at 1x1, 0.98-1.14 at 3x3,
-//     0.88-1.09 at 5x5) and NCHW 1x1 up to 64 rows (1.10-1.20; 0.94-1.07 at 3x3);
+//   159 where this kernel stores slowly and there are few sets of offsets and corners
+//     (planes: taps x deformable groups): outputs whose rows 16-byte pieces cannot cover, up
+//     to 25 (1.2-1.7 at 132-158 tiles of 1x1, 1.05-1.3 at 3x3, 0.95-1.11 at 5x5, but 0.88-1.02
+//     at 7x7 and 0.89 at 5x5 with four groups), channels-last up to 9 (1.1-1.5 at 1x1,
+//     0.98-1.14 at 3x3, 0.88-1.09 at 5x5) and NCHW 1x1 up to 64 rows (1.10-1.20; 0.94-1.07 at
+//     3x3);
 //   80 for NCHW 1x1 of one chunk and more than 128 rows (1.00 at 72, 0.95 at 96);
-//   64 up to 64 rows where each of more than 16 chunks has its own offsets and corners
-//     (7x7, C 64, Cout 64: 1.87 / 0.87 at 64 / 72 tiles; 5x5: 1.79 / 0.92; at 9 chunks
-//     still 1.03, and at C 128, two chunks to a set of corners, 1.04-1.10).
+//   64 up to 64 rows where each chunk is of another plane and there are more than 16 (49
+//     where this kernel stores slowly): 1.87 / 0.87 at 64 / 72 tiles (7x7, C 64, Cout 64), 1.79
+//     / 0.92 (5x5), 0.91 at 84 (7x7, four groups of 9 channels, Cout 5, channels-last); at 9
+//     planes still 1.03, and at C 128, two chunks to a plane, 1.04-1.10.
 bool forward_few_tiles(const Geo &g) {
-    const int rows = std::min(g.gsplit ? g.Cout / g.WG : g.Cout, kBiasRows), nch = g.KK * g.cpw;
+    const int rows = std::min(g.gsplit ? g.Cout / g.WG : g.Cout, kBiasRows);
+    const int cpg = g.Cgp / g.KC, planes = g.KK * ceil_div(g.cpw, cpg);
     const bool vec = g.out_nhwc ? g.Cout % 8 == 0 : g.N % 8 == 0;
     int most = 128;
-    if (!vec ? g.KK <= 25 : g.out_nhwc ? g.KK <= 9 : rows <= 64 && g.KK == 1) most = 159;
-    else if (vec && rows <= 64 && g.Cgp == g.KC && nch > 16) most = 64;
-    else if (vec && rows > 128 && !g.out_nhwc && nch == 1) most = 80;
+    if (planes <= (!vec ? 25 : g.out_nhwc ? 9 : rows <= 64 ? 1 : 0)) most = 159;
+    else if (rows <= 64 && cpg == 1 && planes > (vec ? 16 : 49)) most = 64;
+    else if (vec && rows > 128 && !g.out_nhwc && g.KK * g.cpw == 1) most = 80;
     return (long long)g.B * ceil_div(g.N, 128) * ceil_div(rows, rows > 128 ? 256 : 128) <= most;
 }
 

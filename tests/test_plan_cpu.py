@@ -74,19 +74,20 @@ def test_slices_fit_their_layout(probe):
 
 # The lines as measured (see forward_few_tiles): tiles of 128 pixels x 256 rows (128 up to
 # 128 rows), one image of 16 pixels a row (15 where rows are ragged) to a tile.
-@pytest.mark.parametrize("C,Cout,k,nhwc,ragged,wg,most", [
-    (128, 256, 3, 0, False, 1, 128), (128, 128, 7, 0, False, 1, 128), (64, 512, 3, 0, False, 1, 64),
-    (256, 256, 5, 1, False, 1, 128), (128, 100, 3, 1, False, 1, 159), (64, 256, 1, 1, False, 1, 159),
-    (64, 64, 1, 0, False, 1, 159), (64, 64, 3, 0, False, 1, 128), (64, 64, 5, 0, False, 1, 64),
-    (64, 40, 7, 1, False, 1, 64), (128, 64, 7, 0, False, 1, 128), (64, 256, 1, 0, False, 1, 80),
-    (65, 256, 1, 0, False, 1, 128), (64, 256, 5, 0, True, 1, 159), (64, 64, 7, 0, True, 1, 128),
-    (256, 256, 3, 0, False, 2, 128),
+@pytest.mark.parametrize("C,Cout,k,nhwc,ragged,dg,wg,most", [
+    (128, 256, 3, 0, False, 1, 1, 128), (128, 128, 7, 0, False, 1, 1, 128), (64, 512, 3, 0, False, 1, 1, 64),
+    (256, 256, 5, 1, False, 1, 1, 128), (128, 100, 3, 1, False, 1, 1, 159), (64, 256, 1, 1, False, 1, 1, 159),
+    (64, 64, 1, 0, False, 1, 1, 159), (64, 64, 3, 0, False, 1, 1, 128), (64, 64, 5, 0, False, 1, 1, 64),
+    (64, 40, 7, 1, False, 1, 1, 64), (128, 64, 7, 0, False, 1, 1, 128), (64, 256, 1, 0, False, 1, 1, 80),
+    (65, 256, 1, 0, False, 1, 1, 128), (64, 256, 5, 0, True, 1, 1, 159), (64, 64, 7, 0, True, 1, 1, 128),
+    (256, 256, 3, 0, False, 1, 2, 128), (36, 446, 5, 0, True, 4, 1, 64),
+    (36, 5, 7, 1, False, 4, 1, 64), (36, 40, 3, 0, False, 4, 1, 64), (36, 72, 3, 1, False, 2, 1, 128),
 ])
-def test_few_tiles_of_the_16_bit_forward(probe, C, Cout, k, nhwc, ragged, wg, most):
+def test_few_tiles_of_the_16_bit_forward(probe, C, Cout, k, nhwc, ragged, dg, wg, most):
     for dtype in (F16, BF16):
         for B in (most, most + 1):
             _, few, _ = probe(DEFAULT_BUDGET, -1, _desc(dtype, B, C, 7, 15 if ragged else 16, Cout, k,
-                                                        wg=wg, nhwc=nhwc))[0]
+                                                        dg=dg, wg=wg, nhwc=nhwc))[0]
             assert few == (B == most)
 
 
