@@ -474,29 +474,31 @@ __global__ __launch_bounds__(64 * WM * CB) void dcn2_gradw_f32_kernel(const GwF3
             if (m < p.Cout) unsafeAtomicAdd(p.gw_acc + (size_t)m * p.Kp + k, acc[i][r]);
         }
     if (do_bias) {
-        // One atomic per row and workgroup: channels-last threads, whose loads are all of
-        // one row, sum theirs through LDS (an atomic per load was 118 against 24 us at
-        // 1x1, C 28 -> 91, 5 x 42 x 86, where every workgroup has the bias to add).
+        // One atomic per row and workgroup, 64 rows to an instruction: the atomics of all
+        // workgroups meet on a few cache lines.  From the threads that hold the sums (two
+        // rows to an instruction, or one per load where a thread's loads are of one row)
+        // they took longer than the rest: grad_weight 34 against 15 us at 1x1, C 11 -> 20, 2
+        // x 151 x 105, and 118 against 13 at C 28 -> 91, 5 x 42 x 86, channels-last.
+        float *const red = &sG[0][0][0];  // (the stages are free after the last barrier)
+        constexpr int RN = GM == 2 ? NT / BM : 1;  // parts of a row's sum
         if constexpr (GM == 2) {
-            float *const red = &sG[0][0][0];  // (the stages are free after the last barrier)
             float v = 0.0f;
 #pragma unroll
             for (int i = 0; i < NG; ++i) v += bsum[i];
             red[gpx * BM + grow] = v;
-            __syncthreads();
-            if (tid < BM && m0 + tid < p.Cout) {
-                v = 0.0f;
-#pragma unroll
-                for (int k = 0; k < NT / BM; ++k) v += red[k * BM + tid];
-                unsafeAtomicAdd(p.gb_acc + m0 + tid, v);
-            }
         } else {
 #pragma unroll
             for (int i = 0; i < NG; ++i) {
-                const int m = m0 + grow + i * GRS;
                 const float v = lane_sum<PS / GE>(bsum[i]);
-                if (gpx == 0 && m < p.Cout) unsafeAtomicAdd(p.gb_acc + m, v);
+                if (gpx == 0) red[grow + i * GRS] = v;
             }
+        }
+        __syncthreads();
+        if (tid < BM && m0 + tid < p.Cout) {
+            float v = 0.0f;
+#pragma unroll
+            for (int k = 0; k < RN; ++k) v += red[k * BM + tid];
+            unsafeAtomicAdd(p.gb_acc + m0 + tid, v);
         }
     }
 }
