@@ -19,11 +19,10 @@
 namespace dcn2 {
 
 struct FwdParams {
-    const void *xt, *wp, *tab, *offset, *mask;
-    const void *bias;           // of this launch's first row
+    const void *xt, *wp, *tab, *offset, *mask, *bias;
     void *out;
     int H, W, Cout, kh, kw, sh, sw, ph, pw, dh, dw, G, Cgp, Ho, Wo, Kp;
-    int Mp, brows;              // padded rows of this launch; those of them with a bias
+    int Mp, brows;              // padded output rows; those of them with a bias
     int ntiles, mtiles, tiles;  // pixel tiles per image, M tiles, B*ntiles*mtiles
     // Chunks and M tiles walked by this launch.  A launch covers the M tiles
     // [mt_base, mt_base + mtiles) and, per tile, the nch_eff = KK*cpw chunks
@@ -105,7 +104,7 @@ template <typename T> struct Blend8 {
 };
 
 // Rows of the LDS bias table of the warp-specialised forward (32 KB: one workgroup
-// to a CU either way), and so of a launch.
+// to a CU either way); more take the tile kernels.
 constexpr int kBiasRows = 8192;
 
 // MASK: 0 no mask (all ones), 1 mask values, 2 mask logits (sigmoid on load);
@@ -299,13 +298,14 @@ __global__ __launch_bounds__(512) void dcn2_fwd_ws_kernel(const FwdParams p) {
         f32x16 acc[IB][JB];
         const T *bias = (const T *)p.bias;
         const T *wbase = (const T *)p.wp + (size_t)lane * KPL;
-        // Bias of this wave's rows of every M tile of the launch in LDS (fp32, 0
-        // past Cout; the host keeps a launch within kBiasRows rows), so starting a tile never waits
-        // on a global load queued behind the A loads in flight.  Each wave
-        // writes and reads only its own rows: no barrier needed.
-        // (Bounds and pointer of the launch come from the host: worked out here from
-        // mt_base they cost the channels-last f16 kernel 16 more spilled registers,
-        // 35.2 against 32.6 us at 3x3, C 128 -> 256, 25,600 pixels.)
+        // Bias of this wave's rows of every M tile in LDS (fp32, 0 past Cout), so starting
+        // a tile never waits on a global load queued behind the A loads in flight.  Each
+        // wave writes and reads only its own rows: no barrier needed.
+        // (Filled up to bounds from the host and indexed by the row itself.  With bounds
+        // worked out here from mt_base, for launches of a part of the rows, the
+        // channels-last f16 kernel spilled 16 more registers: 35.2 against 32.6 us at 3x3, C
+        // 128 -> 256, 25,600 pixels.  With the launch's first row taken off the index, outputs
+        // of ragged rows took 358 against 345 us at 1x1, C 324 -> 545, 28 x 150 x 30.)
         for (int r = lane; r < p.Mp; r += 64)
             if ((r / ROWS) % 4 == rw) sBias[r] = r < p.brows ? to_f32(bias[r]) : 0.0f;
         // The MFMAs compute the transposed tile D^T[n][m] (the weight
@@ -325,7 +325,7 @@ __global__ __launch_bounds__(512) void dcn2_fwd_ws_kernel(const FwdParams p) {
 #pragma unroll
                     for (int rq = 0; rq < 4; ++rq) {
                         const f32x4 b4 = *reinterpret_cast<const f32x4 *>(
-                            &sBias[m0 - p.mt_base * 4 * ROWS + rw * ROWS + i * 32 + 8 * rq + 4 * (lane >> 5)]);
+                            &sBias[m0 + rw * ROWS + i * 32 + 8 * rq + 4 * (lane >> 5)]);
 #pragma unroll
                         for (int j = 0; j < JB; ++j)
 #pragma unroll
@@ -335,7 +335,7 @@ __global__ __launch_bounds__(512) void dcn2_fwd_ws_kernel(const FwdParams p) {
                 typedef unsigned long long u64x8 __attribute__((ext_vector_type(8)));
 #pragma unroll
                 for (int i = 0; i < IB; ++i) {
-                    const uint32_t bb = __float_as_uint(sBias[m0 - p.mt_base * 4 * ROWS + rw * ROWS + i * 32 + (lane & 31)]);
+                    const uint32_t bb = __float_as_uint(sBias[m0 + rw * ROWS + i * 32 + (lane & 31)]);
                     const unsigned long long b2 = ((unsigned long long)bb << 32) | bb;
 #pragma unroll
                     for (int j = 0; j < JB; ++j) acc[i][j] = __builtin_bit_cast(f32x16, u64x8(b2));
@@ -699,7 +699,7 @@ static bool ws_two_waves_per_simd() {
 //     / 0.92 (5x5), 0.91 at 84 (7x7, four groups of 9 channels, Cout 5, channels-last); at 9
 //     planes still 1.03, and at C 128, two chunks to a plane, 1.04-1.10.
 bool forward_few_tiles(const Geo &g) {
-    const int rows = std::min(g.gsplit ? g.Cout / g.WG : g.Cout, kBiasRows);
+    const int rows = g.gsplit ? g.Cout / g.WG : g.Cout;
     const int cpg = g.Cgp / g.KC, planes = g.KK * ceil_div(g.cpw, cpg);
     const bool vec = g.out_nhwc ? g.Cout % 8 == 0 : g.N % 8 == 0;
     int most = 128;
@@ -709,30 +709,22 @@ bool forward_few_tiles(const Geo &g) {
     return (long long)g.B * ceil_div(g.N, 128) * ceil_div(rows, rows > 128 ? 256 : 128) <= most;
 }
 
-// The tile kernels serve this kernel's shapes when it would have few tiles, or a
-// register count that would let three waves share a SIMD.
+// The tile kernels serve this kernel's shapes when it would have few tiles, more rows
+// than the bias table, or a register count that would let three waves share a SIMD.
 static bool ws_unfit(const Geo &g) {
-    if (forward_few_tiles(g)) return true;
+    if (forward_few_tiles(g) || g.Mp > kBiasRows) return true;
     return g.dtype == DCN2_F16 ? !(ws_two_waves_per_simd<f16, 1>() && ws_two_waves_per_simd<f16, 2>())
                                : !(ws_two_waves_per_simd<bf16, 1>() && ws_two_waves_per_simd<bf16, 2>());
 }
 
 // The output rows [row0, row0 + rows) with M tile bm (256 or 128 rows; rows and
-// row0 are multiples of it), at most kBiasRows to a launch.
+// row0 are multiples of it).
 template <typename T>
 static hipError_t launch_fwd_dt(const Geo &g, FwdParams p, int bm, int row0, int rows,
                                 hipStream_t s) {
-    const void *const bias = p.bias;
-    for (int r = 0; r < rows; r += kBiasRows) {
-        p.mt_base = (row0 + r) / bm;
-        p.Mp = std::min(kBiasRows, rows - r);
-        p.mtiles = p.Mp / bm;
-        p.bias = bias ? (const T *)bias + row0 + r : nullptr;
-        p.brows = bias ? std::min(p.Mp, std::max(0, g.Cout - row0 - r)) : 0;
-        const hipError_t e = bm == 256 ? launch_fwd_ws<T, 2>(g, p, s) : launch_fwd_ws<T, 1>(g, p, s);
-        if (e != hipSuccess) return e;
-    }
-    return hipSuccess;
+    p.mt_base = row0 / bm;
+    p.mtiles = rows / bm;
+    return bm == 256 ? launch_fwd_ws<T, 2>(g, p, s) : launch_fwd_ws<T, 1>(g, p, s);
 }
 
 // Ungrouped (or not splittable): one launch over every row and chunk.  With
@@ -775,6 +767,8 @@ hipError_t launch_forward(const Geo &g, const void *xt, const void *wp, const vo
     p.msk_bs = g.msk_bs;
     p.msk_logit = mask ? g.msk_logit : 0;
     p.bias = bias;
+    p.Mp = g.Mp;
+    p.brows = bias ? g.Cout : 0;
     p.out = out;
     p.out_nhwc = g.out_nhwc;
     p.H = g.H;

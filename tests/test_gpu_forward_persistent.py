@@ -21,7 +21,8 @@ SHAPES = [
     (170, 128, 3, 4, 256, 3, 2, 1, 2, False, True),
     (85, 40, 11, 13, 257, 1, 1, 1, 1, False, True),
     (60, 33, 5, 4, 1100, 1, 1, 1, 1, False, True),
-    (45, 64, 2, 3, 8500, 1, 1, 1, 1, True, False),   # two launches of rows
+    (45, 64, 2, 3, 8500, 1, 1, 1, 1, True, False),   # more rows than it holds: the small tiles
+    (45, 64, 2, 4, 8192, 1, 1, 1, 1, True, False),   # as many as it holds
     # resident-weight kernel (fp16): 48 tiles or more
     (50, 64, 8, 3, 129, 3, 1, 1, 1, False, True),
     (49, 5, 4, 6, 256, 3, 1, 1, 1, True, False),
