@@ -45,6 +45,9 @@ SHAPES = [
     (160, 24, 5, 3, 40, 3, 1, 1, 1, False, True),
     (159, 24, 5, 3, 40, 3, 1, 1, 1, False, True),
     (159, 24, 4, 4, 40, 3, 1, 1, 1, True, True),
+    # more than 1024 rows that 16-byte pieces cannot cover: the small tiles at any number
+    (130, 24, 3, 5, 1025, 1, 1, 1, 1, False, True),
+    (130, 24, 3, 5, 1024, 1, 1, 1, 1, False, True),
     # 512 and 516 tiles of 128 rows x 32 pixels: those, and 256 x 64 past them
     (1, 72, 64, 128, 200, 3, 1, 1, 1, False, True),
     (1, 72, 64, 129, 200, 3, 1, 1, 1, True, True),

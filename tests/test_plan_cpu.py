@@ -91,6 +91,11 @@ def test_few_tiles_of_the_16_bit_forward(probe, C, Cout, k, nhwc, ragged, dg, wg
             assert few == (B == most)
 
 
+def test_wide_ragged_layers_take_the_small_tiles(probe):
+    for Cout, ragged, nhwc, few in ((1024, 1, 0, 0), (1028, 1, 0, 1), (1032, 0, 0, 0), (1028, 0, 1, 1), (1032, 1, 1, 0)):
+        assert probe(DEFAULT_BUDGET, -1, _desc(F16, 200, 64, 7, 15 if ragged else 16, Cout, 1, nhwc=nhwc))[0][1] == few
+
+
 def test_few_tiles_of_the_resident_weight_forward(probe):
     for nhwc, most in ((0, 32), (1, 47)):
         for B in (most, most + 1):
