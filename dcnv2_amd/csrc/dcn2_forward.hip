@@ -698,14 +698,14 @@ static bool ws_two_waves_per_simd() {
 //     where this kernel stores slowly): 1.87 / 0.87 at 64 / 72 tiles (7x7, C 64, Cout 64), 1.79
 //     / 0.92 (5x5), 0.91 at 84 (7x7, four groups of 9 channels, Cout 5, channels-last); at 9
 //     planes still 1.03, and at C 128, two chunks to a plane, 1.04-1.10;
-//   any number above 1024 rows where 16-byte pieces cannot cover the output's: 1.0-1.9 at
-//     1100 to 4096 rows, 4 x 41 x 41 to 16 x 81 x 81 (255 us against 166 at 1x1, 64 -> 1100, 16
-//     x 81 x 81), channels-last 1.2-3.1.
+//   any number above 1024 rows where 16-byte pieces cannot cover the output's, up to 25
+//     planes: 1.0-1.9 at 1100 to 4096 rows, 4 x 41 x 41 to 16 x 81 x 81 (255 us against 166 at
+//     1x1, 64 -> 1100, 16 x 81 x 81), channels-last 1.2-3.1; 0.86-0.94 at 36 and 196 planes.
 bool forward_few_tiles(const Geo &g) {
     const int rows = g.gsplit ? g.Cout / g.WG : g.Cout;
     const int cpg = g.Cgp / g.KC, planes = g.KK * ceil_div(g.cpw, cpg);
     const bool vec = g.out_nhwc ? g.Cout % 8 == 0 : g.N % 8 == 0;
-    if (!vec && rows > 1024) return true;
+    if (!vec && rows > 1024 && planes <= 25) return true;
     int most = 128;
     if (planes <= (!vec ? 25 : g.out_nhwc ? 9 : rows <= 64 ? 1 : 0)) most = 159;
     else if (rows <= 64 && cpg == 1 && planes > (vec ? 16 : 49)) most = 64;
