@@ -15,8 +15,8 @@ pytestmark = pytest.mark.gpu
 # (B, C, H, W, Cout, k, stride, dg, wg, nhwc, logits)
 SHAPES = [
     (40, 64, 7, 7, 33, 1, 1, 1, 1, False, False),    # 49-pixel images, one channel tile
-    (3, 64, 131, 127, 257, 1, 1, 1, 1, False, True),  # 128-pixel tiles, one row past a step
-    (9, 200, 14, 14, 65, 1, 1, 1, 1, False, True),   # 256 padded channels: four tiles share the corner sums
+    (3, 64, 131, 127, 257, 1, 1, 1, 1, False, True),  # many 64-pixel tiles, one row past a step
+    (9, 200, 14, 14, 65, 1, 1, 1, 1, False, True),   # 224 padded channels: seven 32-channel tiles share the corner sums
     (2, 256, 13, 9, 31, 3, 1, 2, 1, True, False),    # two tiles per group, channels_last
     (3, 96, 11, 10, 130, 3, 2, 1, 1, False, False),  # 96 padded channels: three 32-channel tiles
     (1, 3, 3, 4, 1, 1, 1, 1, 1, False, True),        # the smallest

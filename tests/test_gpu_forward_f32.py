@@ -1,4 +1,4 @@
-"""The fp32 forward's tiles (dcn2_forward_f32.hip) at their edges, against the
+"""The fp32 forward's tiles (dcn2_forward_tiles.hip) at their edges, against the
 oracle: every tile of the launch rule, tiles that span images, rows and pixels
 that end inside a tile, K walks that do not fill a split step, a group of several
 channel chunks, a channels_last output and weight groups."""
@@ -14,17 +14,22 @@ pytestmark = pytest.mark.gpu
 
 # (B, C, H, W, Cout, k, stride, dg, wg, nhwc): tile
 SHAPES = [
-    (3, 40, 65, 67, 257, 1, 1, 1, 1, False),    # 256x64, one row past a tile
-    (70, 33, 7, 7, 2048, 1, 1, 1, 1, False),    # 256x64, 49-pixel images
-    (2, 64, 129, 131, 65, 1, 1, 1, 1, False),   # 128x64, many tiles
-    (3, 160, 61, 60, 100, 1, 1, 1, 1, True),    # 128x64, 5 chunks
-    (3, 96, 61, 60, 128, 3, 1, 1, 1, False),    # 128x64, K split
-    (5, 32, 31, 29, 127, 3, 1, 1, 1, True),     # 128x32, K split, 9 chunks
-    (9, 16, 45, 43, 33, 3, 1, 2, 1, False),     # 64x64
-    (3, 70, 9, 5, 34, 3, 2, 1, 1, True),        # 64x32, K split
-    (1, 3, 4, 3, 1, 1, 1, 1, 1, False),         # 64x32, K split, one chunk
-    (2, 16, 13, 11, 32, 5, 1, 4, 1, True),      # 64x32, 100 chunks
-    (2, 64, 33, 35, 256, 3, 1, 1, 2, False),    # weight groups, one launch each
+    (3, 40, 65, 67, 257, 1, 1, 1, 1, False),     # 256x64, one row past a tile, 2 chunks
+    (70, 33, 7, 7, 2048, 1, 1, 1, 1, False),     # 256x64, 49-pixel images, 2 chunks
+    (2, 64, 129, 131, 65, 1, 1, 1, 1, False),    # 128x64, 2 chunks
+    (3, 160, 61, 60, 100, 1, 1, 1, 1, True),     # 128x32, K split, 5 chunks
+    (3, 96, 61, 60, 128, 3, 1, 1, 1, False),     # 128x32, K split, 27 chunks
+    (5, 32, 31, 29, 127, 3, 1, 1, 1, True),      # 128x32, K split, 9 chunks
+    (9, 16, 45, 43, 33, 3, 1, 2, 1, False),      # 64x64, 18 chunks
+    (3, 70, 9, 5, 34, 3, 2, 1, 1, True),         # 64x32, K split, 27 chunks
+    (1, 3, 4, 3, 1, 1, 1, 1, 1, False),          # 64x32, K split, 1 chunk
+    (2, 16, 13, 11, 32, 5, 1, 4, 1, True),       # 64x32, K split, 100 chunks
+    (2, 64, 33, 35, 256, 3, 1, 1, 2, False),     # 64x32, K split, 9 chunks, weight groups
+    (3, 40, 65, 67, 257, 1, 1, 1, 1, True),      # 256x64, 2 chunks, channels_last
+    (2, 64, 129, 131, 65, 1, 1, 1, 1, True),     # 128x64, 2 chunks, channels_last
+    (9, 16, 45, 43, 33, 3, 1, 2, 1, True),       # 64x64, 18 chunks, channels_last
+    (2, 64, 103, 101, 256, 3, 1, 1, 2, False),   # 128x64, 9 chunks, weight groups
+    (2, 64, 73, 71, 512, 1, 1, 1, 2, True),      # 256x64, 1 chunk, weight groups, channels_last
 ]
 
 
