@@ -1,10 +1,10 @@
 #!/usr/bin/env python
 """Headline benchmark of dcnv2_amd on one MI355X.
 
-Metric (BASELINE.json): DCNv2 forward TFLOPS by the reference README formula
+Metric: DCNv2 forward TFLOPS by the reference README formula
 (README.md:17-19: B*Hout*Wout*Cout*(10*kh*kw*C + 2*kh*kw)) at the README shape
-B8 C64 128x128 Cout256 3x3 fp16, plus forward+backward
-milliseconds at the same shape (config 2).
+B8 C64 128x128 Cout256 3x3 fp16, plus forward+backward milliseconds at the same
+shape.
 
 A step is one forward over one batch of synthetic inputs already resident in
 HBM.  The warm-up runs W untimed steps and keeps going until at least
@@ -46,7 +46,7 @@ PEAK_FP32_TFLOPS = 157.3
 PEAK_HBM_GBS = 8000.0
 REF_README_TFLOPS = 90.2    # reference README.md:14 (RTX 3090, com_2buffer_cpasyc.cu)
 METRIC = "DCNv2 fwd TFLOPS (README formula) @B8 C64 128² Co256 3×3 fp16; fwd+bwd ms"
-# Forward floors of BASELINE.md section 2 (us): c3 MFMA-bound, c4 HBM/gather-bound.
+# Forward floors (us): c3 MFMA-bound, c4 HBM/gather-bound.
 FWD_FLOOR_US = {"c1_readme_fwd": 15.4, "c3_neck_bf16_dg4": 30.7, "c4_stress_s2_d2": 5.5}
 MFMA_STAGES = ("fwd_main", "bwd_colgrad", "bwd_gradw")
 
@@ -407,7 +407,7 @@ def main():
                          "TFLOPS (com_2buffer_cpasyc.cu, RTX 3090, README.md:14) is other "
                          "hardware",
         "dtype": "fp16",
-        "data": "synthetic (seeded, BASELINE.json config distributions; inputs resident in HBM)",
+        "data": "synthetic (seeded, distributions of dcnv2_amd/workloads.py; inputs resident in HBM)",
         "config": {"workload": "c1_readme_fwd: B8 C64 H128 W128 Cout256 3x3 s1 p1 d1 dg1 fp16, "
                                "forward", "global_batch": c1.B, "parallelism": "single GPU"},
         "fwd_real_tflops": round(c1.gemm_flops() / (ms * 1e-3) / 1e12, 2),

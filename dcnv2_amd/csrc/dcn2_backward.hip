@@ -2347,12 +2347,12 @@ __global__ __launch_bounds__(512) void dcn2_gi_gather_kernel(const BwdParams p) 
                         if (live && (first || last || tot > 0)) {
                             f32x4 *d4 =
                                 reinterpret_cast<f32x4 *>(gi + ((py - 1) * (TS - 1) + px - 1) * p.Cgp + cc * KC + co * EPL);
-    #pragma unroll
+#pragma unroll
                             for (int i = 0; i < EPL / 4; ++i) {
                                 f32x4 v = f32x4{sum[4 * i], sum[4 * i + 1], sum[4 * i + 2], sum[4 * i + 3]};
                                 if (!first) v += d4[i];
                                 if (!last) d4[i] = v;
-    #pragma unroll
+#pragma unroll
                                 for (int k = 0; k < 4; ++k) sum[4 * i + k] = v[k];
                             }
                         }
@@ -2362,12 +2362,12 @@ __global__ __launch_bounds__(512) void dcn2_gi_gather_kernel(const BwdParams p) 
                         // to it; this lane wrote the same entry in every earlier batch.
                         f32x4 *r4 = reinterpret_cast<f32x4 *>(
                             p.ring + ((size_t)bucket * kRing + ring_index(py, px)) * p.Cgp + cc * KC + co * EPL);
-    #pragma unroll
+#pragma unroll
                         for (int i = 0; i < EPL / 4; ++i) {
                             f32x4 v = f32x4{sum[4 * i], sum[4 * i + 1], sum[4 * i + 2], sum[4 * i + 3]};
                             if (!first) v += r4[i];
                             r4[i] = v;
-    #pragma unroll
+#pragma unroll
                             for (int k = 0; k < 4; ++k) sum[4 * i + k] = v[k];
                         }
                     }
@@ -2386,7 +2386,7 @@ __global__ __launch_bounds__(512) void dcn2_gi_gather_kernel(const BwdParams p) 
                                 if (p.gi_vec && c0 + EPL <= p.Cg) {
                                     *reinterpret_cast<uint4 *>(dst) = pack16<T>(sum);
                                 } else {
-    #pragma unroll
+#pragma unroll
                                     for (int e = 0; e < EPL; ++e)
                                         if (c0 + e < p.Cg) dst[e] = from_f32<T>(sum[e]);
                                 }
@@ -2398,7 +2398,7 @@ __global__ __launch_bounds__(512) void dcn2_gi_gather_kernel(const BwdParams p) 
                             constexpr int PPL = KC / 8;  // pixels per lane: 16 bytes
                             const int cl = lane % KC, lpx = (lane / KC) * PPL;
                             T v[PPL];
-    #pragma unroll
+#pragma unroll
                             for (int e = 0; e < PPL; ++e) v[e] = stage[wave][(lpx + e) * KC + cl];
                             const int X0 = ox + 1 + 8 * (qp & 1) + lpx, cgi = cc * KC + cl;
                             if (Y < p.H && X0 < p.W && cgi < p.Cg) {
@@ -2406,7 +2406,7 @@ __global__ __launch_bounds__(512) void dcn2_gi_gather_kernel(const BwdParams p) 
                                 if (p.gi_vec && X0 + PPL <= p.W) {
                                     *reinterpret_cast<uint4 *>(dst) = __builtin_bit_cast(uint4, v);
                                 } else {
-    #pragma unroll
+#pragma unroll
                                     for (int e = 0; e < PPL; ++e)
                                         if (X0 + e < p.W) dst[e] = v[e];
                                 }

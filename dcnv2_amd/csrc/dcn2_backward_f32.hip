@@ -265,7 +265,10 @@ __global__ __launch_bounds__(256) void dcn2_colgrad_f32_kernel(const CgF32Params
 // Against the 8-wave kernel this replaces, whose rows came by one 4-byte load per
 // MFMA in the MFMA loop (us): 125 -> 66, 122 -> 57, 195 -> 58, 170 -> 58 at the
 // column gradient's four shapes.
-struct FastDiv {  // n / d for n < 2^31: (umulhi(n, mul) + n) >> shift
+// n / d for n < 2^31 as (umulhi(n, mul) + n) >> shift: division by an invariant
+// integer after Granlund and Montgomery ("Division by Invariant Integers using
+// Multiplication", PLDI 1994), whose 33-bit multiplier 2^32 + mul is applied in two parts.
+struct FastDiv {
     uint32_t mul, d;
     int shift;
 };

@@ -419,7 +419,8 @@ static hipError_t forward_tiles(const Geo &g, const void *xt, const void *wp, co
             //     72.5 at 512, 3136, 4352 and 115.7 / 97.8 at 1000, 4800, 2176.
             //   256x64 (a pixel is sampled once for 256 rows): fp32 64.7 against 71.1
             //     for 128x64 at 256, 64, 100352; 48.7 against 51.7 at 2048, 512, 1568.
-            //   128x64 and 64x64 (4 waves): the rest, whose rows 256x64 would pad.
+            //   128x64 (fp32: 16-bit layers of 65 to 128 rows that come here stay below the
+            //     line above) and 64x64 (4 waves): the rest, whose rows 256x64 would pad.
             auto tiles = [&](int bm, int bn) { return (long long)ceil_div(rows, bm) * ceil_div(p.total, bn); };
             const int most = sizeof(T) == 2 && rows > 128 && p.nch > 8 ? 512 : 640;
             hipError_t e;
@@ -429,8 +430,9 @@ static hipError_t forward_tiles(const Geo &g, const void *xt, const void *wp, co
                 e = launch_tile<T, 1, 1, 4, 1, 2>(p, rows, g.out_nhwc, s);
             else if (rows > 128)
                 e = launch_tile<T, 1, 2, 8, 1, 1>(p, rows, g.out_nhwc, s);
-            else if (rows > 64)
-                e = launch_tile<T, 1, 2, 4, 1, 1>(p, rows, g.out_nhwc, s);
+            else if constexpr (sizeof(T) == 4)
+                e = rows > 64 ? launch_tile<T, 1, 2, 4, 1, 1>(p, rows, g.out_nhwc, s)
+                              : launch_tile<T, 1, 1, 2, 2, 1>(p, rows, g.out_nhwc, s);
             else
                 e = launch_tile<T, 1, 1, 2, 2, 1>(p, rows, g.out_nhwc, s);
             if (e != hipSuccess) return e;

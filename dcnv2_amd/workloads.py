@@ -1,5 +1,4 @@
-"""The benchmark workloads of this path: the five configurations of
-BASELINE.json, with seeded synthetic inputs.
+"""The five benchmark workloads of this path, with seeded synthetic inputs.
 
 Inputs are drawn on the CPU from ``torch.Generator(seed)`` in float32, in the
 fixed order input, offset, mask, weight, bias, grad_output, and only then cast
@@ -62,7 +61,6 @@ class Workload:
                     deformable_groups=self.groups)
 
 
-# BASELINE.json "configs", in order.
 CONFIGS = [
     Workload("c0_cpu_plumbing", 1, 16, 32, 32, 32, 3, 1, 1, 1, 1, torch.float32,
              "normal:1", "sigmoid_normal", "normal:0.1", False, 0),

@@ -4,7 +4,7 @@
 The operator reads the offset-and-mask predictor's raw output ``om``: offsets
 are its first ``2*G*kh*kw`` channels and the mask is ``sigmoid`` of the rest,
 the split the reference's ``DCN.forward`` makes (``dcn_v2_mm.py:133-137``).
-Checks, to the tolerances of ``north_star`` (``tests/util.py::TOL``):
+Checks, to the tolerances of ``tests/util.py::TOL``:
 
 * against the CPU oracle in fp64 with ``offset = om[:, :2GK]`` and
   ``mask = sigmoid(om[:, 2GK:])``; the expected ``grad_om`` is

@@ -1,11 +1,11 @@
 """GPU parity of the HIP path (called through the C ABI via dcnv2_amd._C).
 
-Checks: max|y - y_ref| / max|y_ref| <= 1e-2 for
+Checks max|y - y_ref| / max|y_ref| <= 1e-2 for
 fp16/bf16 and <= 1e-4 for fp32, for the output and all five gradients.
 
 * golden fixtures (tests/golden, made by the independent grid_sample
   formulation): every dtype, forward and backward;
-* the five BASELINE configurations at full size: forward of the first and last
+* the five workloads of dcnv2_amd/workloads.py at full size: forward of the first and last
   image against the CPU oracle, forward+backward of one image against the
   oracle in the config dtype and in an fp32 rerun, and the whole batch against
   the independent grid_sample formulation evaluated in fp32 on the GPU;

@@ -6,7 +6,7 @@ import os
 import numpy as np
 import torch
 
-# Tolerance on max|y - y_ref| / max|y_ref| per compute dtype (BASELINE north_star).
+# Tolerance on max|y - y_ref| / max|y_ref| per compute dtype.
 TOL = {torch.float32: 1e-4, torch.float16: 1e-2, torch.bfloat16: 1e-2}
 GRADS = ("grad_input", "grad_offset", "grad_mask", "grad_weight", "grad_bias")
 
