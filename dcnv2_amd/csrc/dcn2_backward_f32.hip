@@ -59,8 +59,8 @@ __global__ __launch_bounds__(256) void dcn2_colgrad_f32_kernel(const CgF32Params
     constexpr int NG = NT * kCgM / 256;
     struct Px {
         uint32_t off[4];
-        float m, ly, lx;
-        int valid, row, pad[3];
+        float m;
+        int row, pad[2];
     };
     constexpr size_t kG = sizeof(float) * 2 * kCgM * LDG, kC = sizeof(float) * NT * LDC;
     __shared__ __attribute__((aligned(16))) char smem[kG > kC ? kG : kC];
@@ -156,8 +156,7 @@ __global__ __launch_bounds__(256) void dcn2_colgrad_f32_kernel(const CgF32Params
         d.off[3] = sp.vy1 && sp.vx1 ? base + row + cs : c.x_bytes;
         d.m = f_m;
         d.row = live ? p.sidx[f_smp] : -1;
-        d.ly = d.lx = 0.0f;
-        d.valid = d.pad[0] = d.pad[1] = d.pad[2] = 0;
+        d.pad[0] = d.pad[1] = 0;
         sP[tid] = d;
     }
 
