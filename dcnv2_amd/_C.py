@@ -104,17 +104,25 @@ def _ptr(t):
     return None if t is None else t.data_ptr()
 
 
+def _current_stream(index):
+    return torch.cuda.current_stream(index).cuda_stream
+
+
+# The handle without a Stream object (3 us of a call of 18) where torch has it: the
+# function is not part of torch's public interface.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", _current_stream)
+
+
 def _launch(name, entry, device, *args):
     """entry(*args, current stream of `device`) with `device` current; raises on a
     status other than 0.  Small layers are bound by the host, so the device guard
-    is entered only when another GPU is current, and the stream handle is read
-    without building a Stream object (3 us of a call of 18)."""
+    is entered only when another GPU is current."""
     index = device.index
     if torch.cuda.current_device() == index:
-        rc = entry(*args, torch._C._cuda_getCurrentRawStream(index))
+        rc = entry(*args, _raw_stream(index))
     else:
         with torch.cuda.device(index):
-            rc = entry(*args, torch._C._cuda_getCurrentRawStream(index))
+            rc = entry(*args, _raw_stream(index))
     if rc != 0:
         raise _err(name)
 

@@ -70,3 +70,9 @@ def test_two_threads_two_streams():
             assert torch.equal(y, y0), f"forward of thread {i}"
             for name, a, b in zip(GRADS, g, g0):
                 check(f"{name} (thread {i})", a, b, TOL[w.dtype])
+
+
+def test_both_stream_handles_agree():
+    for s in (torch.cuda.current_stream(), torch.cuda.Stream()):
+        with torch.cuda.stream(s):
+            assert _C._raw_stream(0) == _C._current_stream(0) == s.cuda_stream

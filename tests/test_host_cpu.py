@@ -479,3 +479,13 @@ def test_torchvision_signature(oracle_C):
         dcnv2_amd.deform_conv2d(x, off[:, :5], w)
     with pytest.raises(RuntimeError):
         dcnv2_amd.deform_conv2d(x, off, w, mask=m[:, :4])
+
+
+def test_stream_handle_without_the_private_function(monkeypatch):
+    """A torch that lacks the function reads the handle off the public Stream."""
+    import importlib.util
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream", raising=False)
+    spec = importlib.util.spec_from_file_location("dcnv2_amd._C_probe", _C.__file__)
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    assert mod._raw_stream is mod._current_stream
