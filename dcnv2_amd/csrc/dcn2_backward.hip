@@ -3205,10 +3205,11 @@ static hipError_t backward_t(const Geo &g, const BwdParams &p0, void *grad_input
         // Few buckets: their channel chunks (and, per pixel, their window passes)
         // are shared out over workgroups until every CU has one; each part sorts
         // the bucket's records itself.  Kernel us, one workgroup per bucket against
-        // this rule: 337 -> 49 (32 buckets of 32 chunks, fp32 1x1 at 32 x 14 x 14),
-        // 85 -> 15 (32 of 16, 32 x 7 x 7), by cells 65 -> 23 (64 of 4, fp32 3x3 at 4 x
-        // 56 x 56), 115 -> 35 (12 of 4, bf16 3x3 at 2 x 25 x 42).  Two or four to a CU
-        // measured 50-55, 17-22, 23, 35: the sorts repeat.
+        // this rule: 337 -> 34 (32 buckets of 32 chunks, fp32 1x1 at 32 x 14 x 14),
+        // 85 -> 12 (32 of 16, 32 x 7 x 7), by cells 65 -> 22 (64 of 4, fp32 3x3 at 4 x
+        // 56 x 56), per pixel instead of by cells 115 -> 15 (12 of 4, bf16 3x3 at 2 x 25 x
+        // 42).  Two or four workgroups to a CU were slower (the sorts repeat): 50-55 against
+        // 49, 17-22 / 15, 23 / 23, 35 / 35 when passes did not yet take chunks in turn.
         const int gcpg = g.Cgp / g.KC;
         if (g.by_cells) {
             p.gi_cs = std::min(gcpg, ceil_div(ncu, nbk));

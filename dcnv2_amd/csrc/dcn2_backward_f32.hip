@@ -14,8 +14,8 @@
 // per chunk there.  Here every (pixel tile, channel tile) is its own 4-wave
 // workgroup, several to a CU, and pixels are numbered through the batch.  Measured
 // (us, old -> new; 3.3-3.7 GFLOP each, 21-24 us at the 154 TFLOP/s of a large
-// product): 203 -> 54 at Cout 256, K 64, 32 x 56 x 56; 392 -> 50 at 256, 1024, 32 x
-// 14 x 14; 1558 -> 60 at 2048, 512, 32 x 7 x 7; 142 -> 58 at 128, 1152, 4 x 56 x 56.
+// product): 203 -> 53 at Cout 256, K 64, 32 x 56 x 56; 392 -> 52 at 256, 1024, 32 x
+// 14 x 14; 1558 -> 60 at 2048, 512, 32 x 7 x 7; 142 -> 57 at 128, 1152, 4 x 56 x 56.
 #include <algorithm>
 #include <cstddef>
 #include <type_traits>
@@ -262,7 +262,7 @@ __global__ __launch_bounds__(256) void dcn2_colgrad_f32_kernel(const CgF32Params
 // blocks (one set per workgroup).  128 x 64 blocks on 4 waves: 256 x 64 on 8 waves
 // measured the same at 256 rows and more (57.6-61.8 us) and 85-97 against 58 at 128.
 // Against the 8-wave kernel this replaces, whose rows came by one 4-byte load per
-// MFMA in the MFMA loop (us): 125 -> 66, 122 -> 57, 195 -> 58, 170 -> 58 at the
+// MFMA in the MFMA loop (us): 125 -> 62, 122 -> 56, 195 -> 56, 170 -> 57 at the
 // column gradient's four shapes.
 // n / d for n < 2^31 as (umulhi(n, mul) + n) >> shift: division by an invariant
 // integer after Granlund and Montgomery ("Division by Invariant Integers using

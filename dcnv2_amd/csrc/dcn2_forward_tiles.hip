@@ -15,13 +15,13 @@
 //     is pixel i % N of image i / N), and a tile may span images;
 //   * the tile is chosen by how many workgroups it gives (forward_tiles), and where
 //     they are few K is split over the waves of a workgroup (WK).
-// Measured against the kernels this replaces (us): fp32 79.0 -> 64.7 at Cout 256,
-// K 64, 32 x 56 x 56; 174.9 -> 50.7 at 256, 1024, 32 x 14 x 14; 100.2 -> 48.7 at
-// 2048, 512, 32 x 7 x 7; 111.2 -> 59.4 at 128, 1152, 4 x 56 x 56 (3x3); 31.3 -> 9.6
+// Measured against the kernels this replaces (us): fp32 79.0 -> 64.9 at Cout 256,
+// K 64, 32 x 56 x 56; 174.9 -> 51.9 at 256, 1024, 32 x 14 x 14; 100.2 -> 48.1 at
+// 2048, 512, 32 x 7 x 7; 111.2 -> 58.2 at 128, 1152, 4 x 56 x 56 (3x3); 31.3 -> 9.6
 // at 32, 144, 32 x 32 (3x3).  The 3.29 GFLOP of the first three take 21 us at the
-// 154 TFLOP/s a large fp32 matrix product reaches here.  16 bits, 3x3: 50.5 -> 32.8
-// at 256, 2304, 50 x 84; 65.3 -> 24.3 at 256, 2304, 2 x 25 x 42; 92.3 -> 32.0 at
-// 512, 4608, 32 x 32; 25.7 -> 13.5 at 128, 1152, 64 x 64.
+// 154 TFLOP/s a large fp32 matrix product reaches here.  16 bits, 3x3: 50.5 -> 31.0
+// at 256, 2304, 50 x 84 (channels-last 51.1 -> 28.9); 65.3 -> 21.4 at 256, 2304, 2 x 25 x
+// 42; 92.3 -> 31.8 at 512, 4608, 32 x 32; 25.7 -> 13.0 at 128, 1152, 64 x 64.
 //
 // A workgroup owns 32*IB*WM output rows x 32*JB*WN pixels and walks K in steps
 // of WK chunks (128 bytes of channels of one tap and group each).  Step s:
